@@ -69,6 +69,7 @@ SWIT_OPT_EXACT_FUSED = 64
 SWIT_OPT_BWD_TILE_X = 128
 SWIT_OPT_STREAMS = 256
 SWIT_OPT_BWD_BALANCE = 512
+SWIT_OPT_RESIDENT = 1024
 
 
 class SwitPrecond(ctypes.Structure):

@@ -189,7 +189,9 @@ __device__ __forceinline__ float wave_max(float v) {
 // kEncThreads threads) from the FP32 ring ring[ns][nring][S] (row r in slot r % nring):
 // the row's max |v| goes to smax (float bits) and each value to 16 bits at that scale.
 constexpr int kEncThreads = 256;
-constexpr int kStripRing = 32;     // rows of the FP32 ring; encoded in batches of up to this many
+// rows of the FP32 ring, encoded in batches of up to this many; the resident forward puts its
+// state out and in once per ring
+constexpr int kStripRing = 128;
 template <int SM>
 __global__ __launch_bounds__(kEncThreads) void k_strip_encode(Dims d, int first_row, int nring, int s0,
                                                               const float *__restrict__ ring,

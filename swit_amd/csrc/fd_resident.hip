@@ -1,0 +1,763 @@
+// Resident time loops: the wavefields of a shot stay in registers for the whole loop.
+//
+// The step kernels of fd_batched.hip read and write every field once per time step, so a
+// step cannot be faster than HBM (219.8 MB a forward step at 481x141 with 49 shots, 37 us
+// at the 5.9 TB/s that plain streaming reaches; the kernel took 38.8 us).  The state itself
+// is small: 73 MB there, against 128 MB of vector registers on the chip.  Here one launch
+// runs many time steps.  A shot is cut into P windows of columns, one workgroup each, which
+// hold p, u, w of their columns in registers; only the columns next to a window's edge are
+// exchanged, through memory, and only receivers and boundary strips are written.
+//
+// Layout.  A lane holds R consecutive rows (rows z0 + lane R + r, so one wave spans the
+// whole height: 64 R rows) of C consecutive columns; wave w of a workgroup holds columns
+// w C .. w C + C - 1 of the window.  Stencils along z stay inside the lane except at its
+// first and last rows, which the neighbouring lanes hand over by wave shifts; stencils
+// along x stay inside the thread except at the wave's first and last columns, which go
+// through LDS (2 columns of p one way and 1 the other, the same for u).  A step is then
+// two phases (p, then u and w) with one barrier each.
+//
+// Windows overlap: one reaches 3 columns past its own columns on each inner side.  A step
+// spoils them (p needs u at x-2..x+1, u needs p at x-1..x+2), so after every step the
+// windows send each other fresh values of the 3 own columns next to them.  Those columns
+// always are the first and last six of a window, so they sit in known registers of its first
+// and last wave.  These run the velocity phase at raised priority, send, and wait for the
+// neighbour while the other waves still compute.  A message word is 8 bytes, {value, number
+// of the message}, stored and polled with relaxed agent-scope atomics: the word that carries
+// a value also says that it has arrived, so no flag, fence or cache flush is needed (measured
+// between workgroups on different XCDs, 64 words: 0.93 us per exchange with tagged words,
+// 2.7 us and more with data, fence and flag).  Two slots alternate: a neighbour sends message
+// n+2 only after it has received n+1, which is sent after n was read.
+//
+// Progress.  Workgroups take their place by a ticket counter when they start to run, and P
+// consecutive tickets form the group of one shot.  So at any time at most one group of a
+// launch is incomplete, and it waits only for workgroups that are dispatched next; complete
+// groups run to their end.  Several such launches at once hold at most P - 1 waiting
+// workgroups each, far fewer than the chip's slots, so one of them always completes.  Every
+// wait is bounded by the clock all the same: past kWaitTicks a wave stops waiting for good,
+// sets *err, and the job's outputs are overwritten with NaN.
+//
+// Per-cell arithmetic and its order are those of the step kernels: results are the same
+// bits.  Cells outside an update region have K (or B) = 0 and hold zeros, so they need no
+// test: fac * 0 - 0 * d = 0.
+#include "fd_common.h"
+#include "fd_kernels.h"
+
+namespace swit {
+namespace rk {
+
+typedef unsigned long long u64;
+
+
+constexpr u64 kWaitTicks = 3000000000ull;       // 30 s of the 100 MHz clock
+
+// lane l gets lane l+1's (up) or l-1's (dn) value, 0 past the ends; every lane active
+__device__ __forceinline__ float up1(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float dn1(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+
+// Barrier for LDS alone: __syncthreads also waits for every global store in flight, and
+// with it for the acknowledgement of message words, receiver samples and strips.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// One window configuration.
+struct Cfg {
+    int R, C, W, P;      // rows per lane, columns per wave, waves, windows per shot
+    int G;               // groups (shots in flight)
+    int z0;              // padded row of lane 0's first row
+};
+constexpr int kH = 3;    // halo columns
+// Columns: window j covers W C columns from 1 + j (W C - 2 kH).
+__host__ __device__ inline int window_x(int W, int C, int j) { return 1 + j * (W * C - 2 * kH); }
+__host__ __device__ inline int window_os(int W, int C, int j) { return window_x(W, C, j) + (j > 0 ? kH : 0); }
+__host__ __device__ inline int window_oe(int W, int C, int j, int P, int nxp) {
+    return j + 1 < P ? window_x(W, C, j) + W * C - 1 - kH : nxp;
+}
+
+struct Ctl {
+    unsigned ticket;
+    int err;
+};
+
+// Columns of a message.  From the left: u of the three halo columns, p and w of the last (the
+// others' cannot be updated by the next step); from the right: u of the three, p and w of
+// the first two.  R rows of 64 lanes each.
+constexpr int kFromLeft = 5, kFromRight = 7;
+
+struct FwdArgs {
+    Dims d;
+    Cfg c;
+    int s0, ns;                 // shots s0 .. s0 + ns - 1
+    int it0, it1;               // steps it0 .. it1
+    const float *co;            // [1 + ncol][5][64 R] coefficients of columns 0 .. ncol (k_res_setup)
+    int ncol;
+    const float *fpx;           // [1 + ncol] 1 - kappa_p of a column's own layer
+    const ShotGeom *geo;
+    const float *src;           // [ns][nt]
+    // Receivers.  Staged (most surveys: few distinct rows): a window's receivers leave through
+    // the p stage; rtab [ns][P][2][W * 64]: stage offset of a receiver, -1 none, rbase [ns][P]:
+    // first slot.  Direct (rtab null): rec [ns][P][W * 64] {cells of the thread with a
+    // receiver (64 bits), first slot, 0}.
+    const int *rtab, *rbase;
+    const uint4 *rec;
+    unsigned long long pmask;   // lanes whose p rows are staged (strip rows, receiver rows)
+    float *seis_t;              // [ns][nt][ngmax], receivers in slot order
+    float *strips;              // null, or [ns][s_rows][S]: row (it - 1) % s_rows
+    int s_rows;
+    DSave hist;
+    const float *in;            // null (zero state) or [ns][3][nxp][ld]
+    float *out;                 // null or [ns][3][nxp][ld]
+    float *end;                 // null or [ns][3][nx][nz]
+    u64 *msg;                   // [G P][2 slots][2 sides][7 R][64]
+    Ctl *ctl;
+};
+
+// A value the compiler must take as changed: what is computed or loaded from it inside a
+// time step stays there instead of being carried (spilled) across the whole time loop.
+__device__ __forceinline__ void opaque_s(int &v) {
+    v = __builtin_amdgcn_readfirstlane(v);
+    asm volatile("" : "+s"(v));
+}
+__device__ __forceinline__ void opaque_v(unsigned &v) { asm volatile("" : "+v"(v)); }
+// The value is computed by here: the compiler may not move its arithmetic further down.
+__device__ __forceinline__ void pin(float &v) { asm volatile("" : "+v"(v)); }
+
+// One column's rows into a message (row r at o + 64 r words).
+template <int R> __device__ __forceinline__ void send_col(u64 *o, unsigned tag, const float (&v)[R]) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        // through a register of its own: a word formed from the state's register would turn
+        // that register into a pair for the whole time loop
+        unsigned b;
+        asm volatile("v_mov_b32 %0, %1" : "=v"(b) : "v"(v[r]));
+        __hip_atomic_store(o + r * 64, ((u64)tag << 32) | b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+// N columns' rows out of a message, polled until every word carries the tag (all loads of a
+// round in flight together).  A wave that has waited too long once waits no more.
+template <int R, int N>
+__device__ __forceinline__ void recv_cols(const u64 *in, unsigned tag, Ctl *ctl, bool &dead, float (&v)[N][R]) {
+    u64 t0 = 0, q[N][R];
+    for (;;) {
+        unsigned bad = 0;
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                q[n][r] = __hip_atomic_load(in + (n * R + r) * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                bad |= (unsigned)(q[n][r] >> 32) ^ tag;
+            }
+        if (__all(bad == 0) || dead) break;
+        const u64 t = wall_clock64();
+        if (t0 == 0) t0 = t;
+        if (t - t0 > kWaitTicks) {
+            dead = true;
+            if ((threadIdx.x & 63) == 0) __hip_atomic_store(&ctl->err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int r = 0; r < R; ++r)      // as in send_col
+            asm volatile("v_mov_b32 %0, %1" : "=v"(v[n][r]) : "v"((unsigned)q[n][r]));
+}
+
+// LDS of a workgroup: the waves' edge columns, the p stage (NS lanes), the u, w stage.
+__host__ __device__ inline int lds_edge_floats(int W, int R) { return W * 6 * R * 64; }
+__host__ __device__ inline int lds_stage_floats(int W, int C, int R, int NS) { return W * C * (NS + 8) * R; }
+
+// The kernel's arguments as they lie in memory.  Taken anew (opaque) where a step needs one
+// that is not used all the time, so that it is loaded there instead of being held, or
+// spilled to vector lanes, over the whole loop.
+template <class A> using ArgPtr = const __attribute__((address_space(4))) A *;
+template <class A> __device__ __forceinline__ ArgPtr<A> fresh_args() {
+    ArgPtr<A> k = (ArgPtr<A>)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));
+    return k;
+}
+// R consecutive floats from a buffer: byte offset voff of this lane plus the wave-uniform soff
+typedef unsigned vec2 __attribute__((ext_vector_type(2)));
+typedef unsigned vec3 __attribute__((ext_vector_type(3)));
+typedef unsigned vec4 __attribute__((ext_vector_type(4)));
+template <int R>
+__device__ __forceinline__ void buffer_rows(__amdgpu_buffer_rsrc_t rs, unsigned voff, int soff, float (&v)[R]) {
+    constexpr int N = R >= 4 ? 4 : R;
+    if constexpr (N == 4) {
+        const vec4 q = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 0);
+        for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(q[i]);
+    } else if constexpr (N == 3) {
+        const vec3 q = __builtin_amdgcn_raw_buffer_load_b96(rs, voff, soff, 0);
+        for (int i = 0; i < 3; ++i) v[i] = __uint_as_float(q[i]);
+    } else if constexpr (N == 2) {
+        const vec2 q = __builtin_amdgcn_raw_buffer_load_b64(rs, voff, soff, 0);
+        for (int i = 0; i < 2; ++i) v[i] = __uint_as_float(q[i]);
+    }
+    if constexpr (R > 4) {
+        constexpr int M = R - 4;
+        if constexpr (M == 1) {
+            v[4] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, voff + 16, soff, 0));
+        } else if constexpr (M == 2) {
+            const vec2 q = __builtin_amdgcn_raw_buffer_load_b64(rs, voff + 16, soff, 0);
+            for (int i = 0; i < 2; ++i) v[4 + i] = __uint_as_float(q[i]);
+        } else if constexpr (M == 3) {
+            const vec3 q = __builtin_amdgcn_raw_buffer_load_b96(rs, voff + 16, soff, 0);
+            for (int i = 0; i < 3; ++i) v[4 + i] = __uint_as_float(q[i]);
+        } else {
+            const vec4 q = __builtin_amdgcn_raw_buffer_load_b128(rs, voff + 16, soff, 0);
+            for (int i = 0; i < 4; ++i) v[4 + i] = __uint_as_float(q[i]);
+        }
+    }
+}
+
+// Forward steps it0 .. it1 (fdcore.f90:75-160) of every shot, the state in registers.
+// Bound by vector issue: 28 operations per cell and step without contraction (the
+// reference's rounding), about 40 with shifts, receivers and exchange.  R C <= 20 (80 registers
+// of state and K) runs at four waves per SIMD, above (up to 200) at two.
+// HIST: also store the divergence history (the exact adjoint's forward).
+template <int R, int C, bool HIST>
+__global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs a) {
+    extern __shared__ float lds[];
+    __shared__ int sh_ticket;
+    constexpr int PF = R * C > 20 ? 2 : 1;               // columns whose coefficients are in flight
+    constexpr int kCol = 64 * R * 4;                     // bytes of a column of one array
+    const int W = a.c.W, P = a.c.P;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (threadIdx.x == 0) sh_ticket = (int)atomicAdd(&a.ctl->ticket, 1u);
+    __syncthreads();
+    const int t = __builtin_amdgcn_readfirstlane(sh_ticket);
+    const int grp = __builtin_amdgcn_readfirstlane(t / P), j = __builtin_amdgcn_readfirstlane(t % P);
+    float *eU = lds;                                     // [W][3][R][64]: first, last but one, last column of u
+    float *eP = eU + W * 3 * R * 64;                     // [W][3][R][64]: first, second, last column of p
+    const int NS = __popcll(a.pmask);
+    float *sp = eP + W * 3 * R * 64;                     // p stage [NS][W C][R]
+    float *sv = sp + W * C * NS * R;                     // u, w stage [2][4][W C][R]
+
+    // this wave's first column; the first and the last wave exchange with the neighbours
+    const int x0w = window_x(W, C, j) + wave * C;
+    const bool edge_l = j > 0 && wave == 0, edge_r = j + 1 < P && wave == W - 1;
+    const unsigned voff0 = lane * R * 4;                 // byte offset of this lane's rows in a column
+    const bool mirror = a.d.free_surface == 1 && lane == 0;
+    // any column in the side layers: their damping factors differ along x; the other waves
+    // take one column's factors for all of theirs (column 0 of the coefficient array)
+    const bool wave_pml = x0w <= a.d.npml || x0w + C - 1 >= a.d.npml + a.d.nx;
+    const __amdgpu_buffer_rsrc_t co = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(a.co), 0, (int)((unsigned)(a.ncol + 1) * 5u * kCol), 0x00027000);
+    unsigned tag = 0;
+    bool dead = false;
+    // The pressure phase loads nothing: K stays in registers, and 1 - kappa_p is the smaller
+    // of the column's and the row's (the damping is the larger of the two layers' profiles,
+    // and 1 - damp dt rounds monotonically).  So the stores at a step's end (loads wait for
+    // every earlier store: the counter is in order) complete behind it.
+    float K[C][R], fpz[R];
+#pragma unroll
+    for (int c = 0; c < C; ++c) buffer_rows<R>(co, voff0, (x0w + c) * (5 * kCol), K[c]);
+    buffer_rows<R>(co, voff0, 2 * kCol, fpz);
+
+    const bool p_lane = (a.pmask >> lane) & 1;
+    const int p_slot = __popcll(a.pmask & ((1ull << lane) - 1));
+    // strip values this thread copies from the stages: NP of p (5 per column), NV of u, w (4)
+    constexpr int NP = (5 * C + 63) / 64, NV = (4 * C + 63) / 64;
+    int sp_lds[NP], sp_slot[NP], sv_lds[NV], sv_slot[NV];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) sp_lds[i] = -1;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) sv_lds[i] = -1;
+    bool v_lane = false;
+    int v_slot = 0;
+    if (a.strips) {
+        const int npml = a.d.npml, nx = a.d.nx, nz = a.d.nz, xw = window_x(W, C, j);
+        const int os = window_os(W, C, j), oe = window_oe(W, C, j, P, a.d.nxp);
+        const int lb = (nz - 1 + npml - a.c.z0) / R;     // lane of interior row nz - 1
+        v_lane = lane < 2 || lane == lb || lane == lb + 1;
+        v_slot = lane < 2 ? lane : 2 + lane - lb;
+        const int top0 = 3 * nx + 6 * nz;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const int n = threadIdx.x + i * W * 64, col = n / 5, v = n % 5, x = xw + col, jx = x - npml;
+            if (col < W * C && x >= os && x <= oe && jx >= 1 && jx <= nx) {
+                const int jz = v < 3 ? v + 1 : v == 3 ? nz : nz - 1;
+                const int q = jz + npml - a.c.z0, L = q / R;
+                sp_lds[i] = (__popcll(a.pmask & ((1ull << L) - 1)) * W * C + col) * R + q % R;
+                sp_slot[i] = v < 3 ? top0 + 6 * (jx - 1) + v : 3 * (jx - 1) + v - 3;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int n = threadIdx.x + i * W * 64, col = n / 4, v = n % 4, x = xw + col, jx = x - npml;
+            if (col < W * C && x >= os && x <= oe && jx >= 1 && jx <= nx) {
+                // u of rows 1 and 2, w of row 1, w of row nz - 1
+                const int jz = v < 2 ? v + 1 : v == 2 ? 1 : nz - 1;
+                const int q = jz + npml - a.c.z0, L = q / R;
+                sv_lds[i] = (((v < 2 ? 0 : 4) + (L < 2 ? L : 2 + L - lb)) * W * C + col) * R + q % R;
+                sv_slot[i] = v < 3 ? top0 + 6 * (jx - 1) + 3 + v : 3 * (jx - 1) + 2;
+            }
+        }
+    }
+    // one side column of the strips (interior columns 1, 2, nx - 1, nx): its rows of field
+    // column `v` to row[3 nx + 6 (jz - 1) + q]
+    auto side_column = [&](ArgPtr<FwdArgs> k, float *row, int x, unsigned voff, int q, const float (&v)[R]) {
+        if (q < 0 || x < window_os(k->c.W, C, j) || x > window_oe(k->c.W, C, j, k->c.P, k->d.nxp)) return;
+        const int jz0 = k->c.z0 + (int)(voff >> 2) - k->d.npml, nz = k->d.nz;
+        float *o = row + 3 * k->d.nx + q;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (jz0 + r >= 1 && jz0 + r <= nz) o[6 * (jz0 + r - 1)] = v[r];
+    };
+    auto copy_velocities = [&](ArgPtr<FwdArgs> k, int s, int row) {
+        float *q = k->strips + ((size_t)s * k->s_rows + row % k->s_rows) * k->d.S;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            if (sv_lds[i] >= 0) q[sv_slot[i]] = sv[sv_lds[i]];
+    };
+
+    for (int s = a.s0 + grp; s < a.s0 + a.ns; s += a.c.G) {
+        const int isx = a.geo[s].isx, isz = a.geo[s].isz;
+        const float *src = a.src + (size_t)s * a.d.nt;
+        float p[C][R], u[C][R], w[C][R];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int r = 0; r < R; ++r) p[c][r] = u[c][r] = w[c][r] = 0.0f;
+        if (a.in) {
+            const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+            int x0 = x0w;
+            unsigned voff = voff0;
+            opaque_s(x0);
+            opaque_v(voff);
+            const int zr = k->c.z0 + (int)(voff >> 2), ld = k->d.ld, np = k->d.nxp * ld;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                if (x0 + c > k->d.nxp) continue;
+                const float *f = k->in + (size_t)s * 3 * np + (size_t)(x0 + c - 1) * ld;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    if (zr + r > k->d.nzp) continue;
+                    const unsigned o = zr + r - 1;
+                    p[c][r] = f[o];
+                    u[c][r] = f[np + o];
+                    w[c][r] = f[2 * np + o];
+                }
+            }
+        }
+        // receivers: stage offsets of this thread's two, or (direct) its cells' bits
+        int ro0 = -1, ro1 = -1, rbase = 0;
+        uint4 rec0 = make_uint4(0, 0, 0, 0);
+        unsigned wm0 = 0, wm1 = 0;                           // cells with a receiver in any lane
+        if (a.rtab) {
+            const int *q = a.rtab + ((size_t)s * P + j) * 2 * (W * 64) + threadIdx.x;
+            ro0 = q[0];
+            ro1 = q[W * 64];
+            rbase = a.rbase[s * P + j];
+        } else {
+            rec0 = a.rec[((size_t)s * P + j) * (W * 64) + threadIdx.x];
+            wm0 = rec0.x;
+            wm1 = rec0.y;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                wm0 |= __shfl_xor(wm0, o);
+                wm1 |= __shfl_xor(wm1, o);
+            }
+            wm0 = __builtin_amdgcn_readfirstlane(wm0);
+            wm1 = __builtin_amdgcn_readfirstlane(wm1);
+        }
+
+        // u of the edge columns for the next step
+        auto put_u = [&]() {
+            float *e = eU + (size_t)wave * 3 * R * 64 + lane;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                e[r * 64] = u[0][r];
+                e[(R + r) * 64] = u[C - 2][r];
+                e[(2 * R + r) * 64] = u[C - 1][r];
+            }
+        };
+        // velocity coefficients of column c, in flight PF columns ahead
+        float cB[PF + 1][R], cfu[PF + 1][R], cfw[PF + 1][R];
+        auto fetch_v = [&](int x, unsigned voff, int c) {
+            const int f = wave_pml ? (x + c) * (5 * kCol) : 0;
+            buffer_rows<R>(co, voff, (x + c) * (5 * kCol) + kCol, cB[c % (PF + 1)]);
+            buffer_rows<R>(co, voff, f + 3 * kCol, cfu[c % (PF + 1)]);
+            buffer_rows<R>(co, voff, f + 4 * kCol, cfw[c % (PF + 1)]);
+        };
+        put_u();
+        lds_barrier();
+        float srcv = a.d.dt * src[a.it0 - 1];
+        const int it1 = a.it1;
+        for (int it = a.it0; it <= it1; ++it) {
+            const float src_next = it < it1 ? src[it] : 0.0f;
+            int x0 = x0w;
+            unsigned voff = voff0;
+            opaque_s(x0);
+            opaque_v(voff);
+            // ---- p: u of the neighbouring waves' columns x0-2, x0-1 and x0+C ----
+            {
+                const ArgPtr<float> fpx = (ArgPtr<float>)fresh_args<FwdArgs>()->fpx + x0;
+                float ul2[R], ul1[R], ur1[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float *e = eU + lane;
+                    ul2[r] = wave > 0 ? e[(((wave - 1) * 3 + 1) * R + r) * 64] : 0.0f;
+                    ul1[r] = wave > 0 ? e[(((wave - 1) * 3 + 2) * R + r) * 64] : 0.0f;
+                    ur1[r] = wave + 1 < W ? e[((wave + 1) * 3 * R + r) * 64] : 0.0f;
+                }
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    const float fx = fpx[c];
+                    const float wd1 = dn1(w[c][R - 1]), wd2 = dn1(w[c][R - 2]), wu = up1(w[c][0]);
+                    float dv[R];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float um1 = c >= 1 ? u[c - (c >= 1)][r] : ul1[r];
+                        const float um2 = c >= 2 ? u[c - (c >= 2 ? 2 : 0)][r] : c == 1 ? ul1[r] : ul2[r];
+                        const float up = c + 1 < C ? u[c + (c + 1 < C)][r] : ur1[r];
+                        const float wm1 = r >= 1 ? w[c][r - (r >= 1)] : wd1;
+                        const float wm2 = r >= 2 ? w[c][r - (r >= 2 ? 2 : 0)] : r == 1 ? wd1 : wd2;
+                        const float wp1 = r + 1 < R ? w[c][r + (r + 1 < R)] : wu;
+                        dv[r] = div_term(u[c][r], um1, up, um2, w[c][r], wm1, wp1, wm2);
+                        p[c][r] = fminf(fx, fpz[r]) * p[c][r] - K[c][r] * dv[r];
+                    }
+#pragma unroll
+                    for (int r = 0; r < R; ++r) pin(p[c][r]);
+                    if (HIST) {
+                        const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+                        const int x = x0 + c, zr = k->c.z0 + (int)(voff >> 2), nzp = k->d.nzp;
+                        if (x >= window_os(k->c.W, C, j) && x <= window_oe(k->c.W, C, j, k->c.P, k->d.nxp)) {
+                            float *h = k->hist.p + ((size_t)s * k->hist.slots + (it - 1 - k->hist.base)) *
+                                                       (k->d.nxp * k->d.ld) + (size_t)(x - 1) * k->d.ld;
+                            const unsigned o = zr - 1;
+                            if (zr + R - 1 <= nzp) {
+                                __builtin_memcpy(h + o, dv, sizeof(float) * R);
+                            } else {
+#pragma unroll
+                                for (int r = 0; r < R; ++r)
+                                    if (zr + r <= nzp) h[o + r] = dv[r];
+                            }
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < PF; ++c) fetch_v(x0, voff, c);
+            // source (fdcore.f90:88-89)
+            if ((unsigned)(isx - x0) < (unsigned)C) {
+                const int zr = fresh_args<FwdArgs>()->c.z0 + (int)(voff >> 2);
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+                    if (x0 + c == isx) {
+#pragma unroll
+                        for (int r = 0; r < R; ++r)
+                            if (zr + r == isz) p[c][r] = p[c][r] + srcv;
+                    }
+            }
+            // p mirror: lane 0 holds rows fs-1, fs, fs+1 (fs+1 in lane 1 when R = 2)
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const float pm = R > 2 ? p[c][R > 2 ? 2 : 0] : up1(p[c][0]);
+                if (mirror) p[c][0] = -pm;
+            }
+            {
+                float *e = eP + (size_t)wave * 3 * R * 64 + lane;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    e[r * 64] = p[0][r];
+                    e[(R + r) * 64] = p[1][r];
+                    e[(2 * R + r) * 64] = p[C - 1][r];
+                }
+            }
+            // p of the staged rows (receivers, strips); the last step's u, w leave their stage
+            if (p_lane) {
+                float *q = sp + (p_slot * W + wave) * (C * R);
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) q[c * R + r] = p[c][r];
+            }
+            if (a.strips && it > a.it0) copy_velocities(fresh_args<FwdArgs>(), s, it - 2);
+            lds_barrier();
+            // ---- u, w: p of the neighbouring waves' columns x0-1, x0+C, x0+C+1 ----
+            if (edge_l || edge_r) __builtin_amdgcn_s_setprio(3);
+            {
+                float pl1[R], pr1[R], pr2[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float *e = eP + lane;
+                    pl1[r] = wave > 0 ? e[(((wave - 1) * 3 + 2) * R + r) * 64] : 0.0f;
+                    pr1[r] = wave + 1 < W ? e[((wave + 1) * 3 * R + r) * 64] : 0.0f;
+                    pr2[r] = wave + 1 < W ? e[(((wave + 1) * 3 + 1) * R + r) * 64] : 0.0f;
+                }
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    if (c + PF < C) fetch_v(x0, voff, c + PF);
+                    const float pd = dn1(p[c][R - 1]), pu0 = up1(p[c][0]), pu1 = up1(p[c][1]);
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float xm = c >= 1 ? p[c - (c >= 1)][r] : pl1[r];
+                        const float xp = c + 1 < C ? p[c + (c + 1 < C)][r] : pr1[r];
+                        const float xq = c + 2 < C ? p[c + (c + 2 < C ? 2 : 0)][r] : c + 2 == C ? pr1[r] : pr2[r];
+                        const float zm = r >= 1 ? p[c][r - (r >= 1)] : pd;
+                        const float zp = r + 1 < R ? p[c][r + (r + 1 < R)] : pu0;
+                        const float zq = r + 2 < R ? p[c][r + (r + 2 < R ? 2 : 0)] : r + 2 == R ? pu0 : pu1;
+                        const float b = cB[c % (PF + 1)][r];
+                        u[c][r] = v_update_f(u[c][r], b, cfu[c % (PF + 1)][r], p[c][r], xp, xq, xm);
+                        w[c][r] = v_update_f(w[c][r], b, cfw[c % (PF + 1)][r], p[c][r], zp, zq, zm);
+                    }
+                    if (mirror) w[c][0] = w[c][1];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        pin(u[c][r]);
+                        pin(w[c][r]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // ---- exchange, out: inboxes [group][window][slot][side], side 0 from the left ----
+            const bool exch = it < it1;
+            ++tag;
+            u64 *box = nullptr;
+            if ((edge_l || edge_r) && exch) {
+                const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+                constexpr int kMsg = kFromRight * R * 64;
+                box = k->msg + ((size_t)(grp * k->c.P + j) * 2 + (tag & 1)) * (2 * kMsg) + voff / (4 * R);
+                if (edge_l) {                            // own first three columns: the left window's right halo
+                    u64 *o = box - 3 * kMsg;
+                    send_col<R>(o, tag, u[3]);
+                    send_col<R>(o + R * 64, tag, u[4]);
+                    send_col<R>(o + 2 * R * 64, tag, u[5]);
+                    send_col<R>(o + 3 * R * 64, tag, p[3]);
+                    send_col<R>(o + 4 * R * 64, tag, p[4]);
+                    send_col<R>(o + 5 * R * 64, tag, w[3]);
+                    send_col<R>(o + 6 * R * 64, tag, w[4]);
+                }
+                if (edge_r) {                            // own last three: the right window's left halo
+                    u64 *o = box + 4 * kMsg;
+                    send_col<R>(o, tag, u[C - 6]);
+                    send_col<R>(o + R * 64, tag, u[C - 5]);
+                    send_col<R>(o + 2 * R * 64, tag, u[C - 4]);
+                    send_col<R>(o + 3 * R * 64, tag, p[C - 4]);
+                    send_col<R>(o + 4 * R * 64, tag, w[C - 4]);
+                }
+            }
+            // ---- receivers (fdcore.f90:123-128) and strips (:130-159): all stores of the step
+            // come here, p stands since the pressure phase ----
+            {
+                const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+                float *q = k->seis_t + ((size_t)s * k->d.nt + (it - 1)) * k->d.ngmax + rbase;
+                const int T = k->c.W * 64;
+                if (ro0 >= 0) q[threadIdx.x] = sp[ro0];
+                if (ro1 >= 0) q[threadIdx.x + T] = sp[ro1];
+            }
+            if (wm0 | wm1) {
+                const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+                int m0 = __builtin_amdgcn_readfirstlane(wm0), m1 = __builtin_amdgcn_readfirstlane(wm1);
+                unsigned r0 = rec0.x, r1 = rec0.y, slot0 = rec0.z;
+                opaque_s(m0);
+                opaque_s(m1);
+                opaque_v(r0);
+                opaque_v(r1);
+                opaque_v(slot0);
+                float *q = k->seis_t + ((size_t)s * k->d.nt + (it - 1)) * k->d.ngmax;
+                const unsigned slot1 = slot0 + __popc(r0);
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const int b = c * R + r;
+                        const unsigned bit = 1u << (b % 32);
+                        const unsigned rm = b < 32 ? r0 : r1;
+                        if (((b < 32 ? m0 : m1) & (int)bit) && (rm & bit))
+                            q[(b < 32 ? slot0 : slot1) + __popc(rm & (bit - 1))] = p[c][r];
+                    }
+            }
+            if (a.strips) {
+                const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+                if (v_lane) {
+                    float *q = sv + (v_slot * W + wave) * (C * R), *qw = q + 4 * W * C * R;
+#pragma unroll
+                    for (int c = 0; c < C; ++c)
+#pragma unroll
+                        for (int r = 0; r < R; ++r) {
+                            q[c * R + r] = u[c][r];
+                            qw[c * R + r] = w[c][r];
+                        }
+                }
+                float *row = k->strips + ((size_t)s * k->s_rows + (it - 1) % k->s_rows) * k->d.S;
+#pragma unroll
+                for (int i = 0; i < NP; ++i)
+                    if (sp_lds[i] >= 0) row[sp_slot[i]] = sp[sp_lds[i]];
+                const int c1 = k->d.npml + 1 - x0, cn = k->d.npml + k->d.nx - x0;   // columns of jx = 1, nx
+                if ((c1 >= -1 && c1 < C) || (cn >= 0 && cn <= C)) {
+#pragma unroll
+                    for (int c = 0; c < C; ++c) {
+                        side_column(k, row, x0 + c, voff,
+                                    c == c1 ? 0 : c == c1 + 1 ? 1 : c == cn ? 3 : c == cn - 1 ? 4 : -1, p[c]);
+                        side_column(k, row, x0 + c, voff, c == c1 ? 2 : c == cn - 1 ? 5 : -1, u[c]);
+                    }
+                }
+            }
+            // ---- exchange, in: fresh halo columns ----
+            if (edge_l && exch) {
+                const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+                float v[3][R], q[2][R];
+                recv_cols<R, 3>(box, tag, k->ctl, dead, v);
+                recv_cols<R, 2>(box + 3 * R * 64, tag, k->ctl, dead, q);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    u[0][r] = v[0][r];
+                    u[1][r] = v[1][r];
+                    u[2][r] = v[2][r];
+                    p[2][r] = q[0][r];
+                    w[2][r] = q[1][r];
+                }
+            }
+            if (edge_r && exch) {
+                const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+                const u64 *in = box + kFromRight * R * 64;
+                float v[3][R], q[2][R];
+                recv_cols<R, 3>(in, tag, k->ctl, dead, v);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    u[C - 3][r] = v[0][r];
+                    u[C - 2][r] = v[1][r];
+                    u[C - 1][r] = v[2][r];
+                }
+                recv_cols<R, 2>(in + 3 * R * 64, tag, k->ctl, dead, q);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    p[C - 3][r] = q[0][r];
+                    p[C - 2][r] = q[1][r];
+                }
+                recv_cols<R, 2>(in + 5 * R * 64, tag, k->ctl, dead, q);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    w[C - 3][r] = q[0][r];
+                    w[C - 2][r] = q[1][r];
+                }
+            }
+            if (edge_l || edge_r) __builtin_amdgcn_s_setprio(0);
+            put_u();
+            srcv = fresh_args<FwdArgs>()->d.dt * src_next;
+            lds_barrier();
+        }
+        if (a.strips) copy_velocities(fresh_args<FwdArgs>(), s, it1 - 1);
+        // state out: own columns
+        if (a.out || a.end) {
+            const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+            int x0 = x0w;
+            unsigned voff = voff0;
+            opaque_s(x0);
+            opaque_v(voff);
+            const int npml = k->d.npml, nx = k->d.nx, nz = k->d.nz, nzp = k->d.nzp, ld = k->d.ld;
+            const int np = k->d.nxp * ld, ni = nx * nz;
+            const int zr = k->c.z0 + (int)(voff >> 2), jz0 = zr - npml;
+            const int os_ = window_os(k->c.W, C, j), oe_ = window_oe(k->c.W, C, j, k->c.P, k->d.nxp);
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const int x = x0 + c, jx = x - npml;
+                if (x < os_ || x > oe_) continue;
+                if (k->out) {
+                    float *f = k->out + (size_t)s * 3 * np + (size_t)(x - 1) * ld;
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (zr + r <= nzp) {
+                            const unsigned o = zr + r - 1;
+                            f[o] = p[c][r];
+                            f[np + o] = u[c][r];
+                            f[2 * np + o] = w[c][r];
+                        }
+                }
+                if (k->end && jx >= 1 && jx <= nx) {
+                    float *f = k->end + (size_t)s * 3 * ni + (size_t)(jx - 1) * nz;
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (jz0 + r >= 1 && jz0 + r <= nz) {
+                            const unsigned o = jz0 + r - 1;
+                            f[o] = p[c][r];
+                            f[ni + o] = u[c][r];
+                            f[2 * ni + o] = w[c][r];
+                        }
+                }
+            }
+        }
+        lds_barrier();               // the edges and the stage are rewritten by the next shot
+    }
+}
+
+// Coefficients of a configuration, column by column (1 .. ncol, past nxp zero):
+// {pressure update's, velocity updates', 1-kappa_p, 1-kappa_u, 1-kappa_w}[64 R rows from z0].
+// The forward's pressure coefficient is K and its velocity coefficient B, the adjoint's the
+// other way round.  They are zero outside the update regions: pressure rows zp0 .. nzp-2 and
+// columns 3 .. nxp-2, velocity rows zv0 .. nzp-2 and columns 2 .. nxp-2 (the reference's
+// regions hold one more row of u and one more column of w, whose stencils read only zeros:
+// they stay zero).  Column 0 holds the factors of a column away from the side layers;
+// fpx[x] is column x's 1-kappa_p on the interior rows.
+__global__ void k_res_setup(Dims d, int R, int z0, int ncol, int zp0, int zv0, int adjoint,
+                            const float2 *__restrict__ KB, const float2 *__restrict__ CP,
+                            const float4 *__restrict__ CV, float *__restrict__ co, float *__restrict__ fpx) {
+    const int row = blockIdx.x * blockDim.x + threadIdx.x, col = blockIdx.y;
+    if (row >= 64 * R || col > ncol) return;
+    const int z = z0 + row, x = col ? col : d.npml + 1;
+    const bool in = z >= 1 && z <= d.nzp && x <= d.nxp;
+    float K = 0.0f, B = 0.0f, fp = 1.0f, fu = 1.0f, fw = 1.0f;
+    if (in) {
+        const size_t k = pidx(d, z, x);
+        const float2 kb = KB[k];
+        const float4 cv = CV[k];
+        K = kb.x;
+        B = kb.y;
+        fp = CP[k].y;
+        fu = cv.y;
+        fw = cv.z;
+    }
+    const bool rp = in && z >= zp0 && z <= d.nzp - 2 && x >= 3 && x <= d.nxp - 2;
+    const bool rv = in && z >= zv0 && z <= d.nzp - 2 && x >= 2 && x <= d.nxp - 2;
+    const size_t n = (size_t)64 * R;
+    float *o = co + (size_t)col * 5 * n + row;
+    o[0] = rp ? (adjoint ? B : K) : 0.0f;
+    o[n] = rv ? (adjoint ? K : B) : 0.0f;
+    o[2 * n] = fp;
+    o[3 * n] = fu;
+    o[4 * n] = fw;
+    // the column's own damping: that of an interior row
+    if (row == 0) fpx[col] = x <= d.nxp ? CP[pidx(d, d.npml + 1, x)].y : 1.0f;
+}
+
+// Start of a launch: the message words (tags) and the ticket counter.
+__global__ void k_res_begin(u64 *__restrict__ msg, size_t n, Ctl *ctl, int clear_err) {
+    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) {
+        ctl->ticket = 0;
+        if (clear_err) ctl->err = 0;
+    }
+    for (; i < n; i += (size_t)gridDim.x * blockDim.x) msg[i] = 0;
+}
+
+// Receiver slots to traces: out[s][r][t] = in[s][t][map[s][r]], zero for a receiver past the
+// shot's own count (map -1) and at t = 0; NaN everywhere if a wait of the job ran out.
+// Tiles of 32 samples x 32 receivers through LDS; block (32, 8).
+__global__ void k_res_traces(int nt, int ngmax, const int *__restrict__ map, const float *__restrict__ in,
+                             float *__restrict__ out, const Ctl *ctl) {
+    __shared__ float tile[32][33];
+    const int s = blockIdx.z, r0 = blockIdx.x * 32, t0 = blockIdx.y * 32;
+    const bool bad = ctl->err != 0;
+    const int r = r0 + threadIdx.x;
+    const int m = r < ngmax ? map[(size_t)s * ngmax + r] : -1;
+    for (int k = threadIdx.y; k < 32; k += 8) {
+        const int t = t0 + k;
+        float v = 0.0f;
+        if (m >= 0 && t < nt) v = in[((size_t)s * nt + t) * ngmax + m];
+        tile[k][threadIdx.x] = bad ? __int_as_float(0x7fc00000) : v;
+    }
+    __syncthreads();
+    for (int k = threadIdx.y; k < 32; k += 8) {
+        const int rr = r0 + k, t = t0 + threadIdx.x;
+        if (rr < ngmax && t < nt) out[((size_t)s * ngmax + rr) * nt + t] = tile[threadIdx.x][k];
+    }
+}
+
+}  // namespace rk
+}  // namespace swit

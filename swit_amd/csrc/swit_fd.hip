@@ -18,6 +18,7 @@
 #include "fd_kernels.h"
 #include "fd_plain.hip"
 #include "fd_batched.hip"
+#include "fd_resident.hip"
 #include "fd_misfit.hip"
 #include "fd_exact.hip"
 #include "fd_precond.hip"
@@ -50,6 +51,27 @@ int set_err(int code, const char *fmt, ...) {
 int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 }  // namespace
+
+// Resident time loops of a plan (fd_resident.hip): the forward's window configuration, the
+// arrays laid out for it and its launch state.  use_*: SWIT_OPT_RESIDENT, and 0 for a direction
+// whose step kernels were configured by an option of theirs.
+struct ResidentState {
+    int use_fwd = 1, use_bwd = 1, use_exact = 1;
+    bool fwd = false;            // the forward's configuration exists
+    rk::Cfg fc{};
+    size_t f_lds = 0;
+    float *f_co = nullptr;       // coefficients [1 + f_ncol][5][64 R]
+    float *f_fpx = nullptr;      // [1 + f_ncol]
+    unsigned long long f_pmask = 0;
+    int *f_rtab = nullptr;       // [ns][P][2][64 W] (staged receivers) ...
+    uint4 *f_rec = nullptr;      // ... or [ns][P][64 W] (direct)
+    int *f_rbase = nullptr;      // [ns][P]
+    int *f_map = nullptr;        // [ns][ngmax] receiver -> slot of seis_t
+    int f_ncol = 0;
+    rk::u64 *msg = nullptr;      // exchange words (shared by the plan's resident launches)
+    size_t f_msg = 0;
+    rk::Ctl *ctl = nullptr;
+};
 
 struct swit_plan {
     Dims d{};
@@ -85,6 +107,7 @@ struct swit_plan {
     bool model_set = false;
     bool strips_valid = false;
     BatchedState bat;
+    ResidentState res;
 
     template <typename T>
     int alloc(T **p, size_t count) {
@@ -444,6 +467,9 @@ static int plain_adjoint(swit_plan *pl, const float *src, hipStream_t st) {
     return SWIT_OK;
 }
 
+static int resident_now(bool built, int use, hipStream_t st, bool *yes);
+static int resident_forward(swit_plan *pl, const float *src, float *seis, int save, hipStream_t st);
+
 // ---- public jobs -------------------------------------------------------------------
 
 extern "C" int swit_forward(swit_plan *pl, const float *src, float *seis, int save_strips,
@@ -457,6 +483,13 @@ extern "C" int swit_forward(swit_plan *pl, const float *src, float *seis, int sa
         return set_err(SWIT_EINVAL, "the plan was created without strips (SWIT_PLAN_NO_STRIPS)");
     const int save = save_strips == 1;
     if (save_strips != 2) pl->strips_valid = false;
+    bool resident = false;
+    TRY(resident_now(pl->res.fwd, pl->res.use_fwd, stream, &resident));
+    if (resident) {
+        TRY(resident_forward(pl, src, seis, save, stream));
+        if (save_strips != 2) pl->strips_valid = save_strips == 1;
+        return SWIT_OK;
+    }
     if (pl->flags & SWIT_PATH_BATCHED)
         TRY(batched_forward(pl, src, save, stream));
     else
@@ -634,6 +667,10 @@ static int copyk(const float *a, float *b, size_t n, hipStream_t st) {
     return SWIT_OK;
 }
 
+static int resident_init(swit_plan *pl);
+static int resident_set_model(swit_plan *pl, hipStream_t st);
+static int resident_autotune(swit_plan *pl, double *us, hipStream_t st);
+
 static int batched_init(swit_plan *pl) {
     BatchedState &bs = pl->bat;
     const Dims &d = pl->d;
@@ -784,6 +821,7 @@ static int batched_init(swit_plan *pl) {
     const char *eg = getenv("SWIT_NO_GRAPH");
     bs.use_graph = !(eg && atoi(eg) > 0);
     HIP_TRY(hipStreamCreateWithFlags(&bs.cap, hipStreamNonBlocking));
+    TRY(resident_init(pl));
     bs.ready = 1;
     return SWIT_OK;
 }
@@ -820,7 +858,7 @@ static int batched_set_model(swit_plan *pl, hipStream_t st) {
     hipLaunchKernelGGL(k_setup_cvec, grd, blk, 0, st, d, pl->K, pl->B, pl->prof, pl->bat.CP, pl->bat.CV,
                        pl->bat.KB);
     LAUNCH_CHECK();
-    return SWIT_OK;
+    return resident_set_model(pl, st);
 }
 
 static int pool_event(BatchedState &bs, hipEvent_t *e) {
@@ -1182,6 +1220,341 @@ static int batched_adjoint(swit_plan *pl, const float *src, double *grad, double
     return SWIT_OK;
 }
 
+// ---- resident time loops (host side) ---------------------------------------------------
+
+namespace {
+
+struct FwdKernel {
+    int R, C;
+    void (*fn[2])(rk::FwdArgs);     // without / with the divergence history
+};
+// 4 R C registers of state and K per thread: R C <= 20 at four waves per SIMD (128 registers),
+// above at two (256 registers, workgroups of at most 8 waves)
+#define SWIT_FWD(R, C) {R, C, {rk::k_fwd_resident<R, C, false>, rk::k_fwd_resident<R, C, true>}}
+const FwdKernel kFwdKernels[] = {
+    SWIT_FWD(2, 6), SWIT_FWD(2, 9), SWIT_FWD(2, 14), SWIT_FWD(2, 20), SWIT_FWD(2, 24),
+    SWIT_FWD(3, 6), SWIT_FWD(3, 9), SWIT_FWD(3, 12), SWIT_FWD(3, 14), SWIT_FWD(3, 16),
+    SWIT_FWD(4, 6), SWIT_FWD(4, 8), SWIT_FWD(4, 10), SWIT_FWD(4, 12),
+    SWIT_FWD(5, 6), SWIT_FWD(5, 8), SWIT_FWD(5, 10),
+    SWIT_FWD(6, 6), SWIT_FWD(6, 8), SWIT_FWD(7, 7), SWIT_FWD(8, 6),
+};
+#undef SWIT_FWD
+constexpr int kCuLds = 160 * 1024;
+int fwd_cu_waves(const FwdKernel &k) { return k.R * k.C <= 20 ? 16 : 8; }
+
+size_t fwd_lds_bytes(const rk::Cfg &c, int NS) {
+    return sizeof(float) * (rk::lds_edge_floats(c.W, c.R) + rk::lds_stage_floats(c.W, c.C, c.R, NS));
+}
+
+// Estimated time of one resident step (us): the vector issue of the waves that share a
+// compute unit, with what their latency adds, and the exchange and the barriers.  Fitted to
+// the forward on grids of 201x81 to 481x141 (2.4 GHz): with one wave per SIMD 1.34 times the
+// issue time, with two or more 0.93 (36 operations are counted per cell, some waves have
+// fewer), plus 2.0 us with an exchange (one shot, R = 2, C = 6, W = 3: 2.97 measured, 2.96
+// estimated; 49 shots, R = 3, C = 16, W = 8: 7.37 and 7.36).
+double resident_step_us(int waves_on_cu, double cell_ops, bool exchange) {
+    const double issue = cdiv(waves_on_cu, 4) * cell_ops * 4 / 2400.0;
+    return (waves_on_cu > 4 ? 0.93 : 1.34) * issue + (exchange ? 2.0 : 0.9);
+}
+
+// Windows of the forward for ns shots on ncu compute units: of every (columns per wave,
+// waves) the one with the least estimated time, rounds of shots x time of a step.
+bool choose_fwd(const Dims &d, int ns, int ncu, int NS, rk::Cfg *best) {
+    const int rows = d.nzp - (d.fs - 1) + 1;
+    const int R = std::max(2, cdiv(rows, 64));
+    double best_t = 1e30;
+    for (const FwdKernel &kn : kFwdKernels) {
+        if (kn.R != R) continue;
+        const int cu_waves = fwd_cu_waves(kn);
+        for (int W = 1; W <= cu_waves; ++W) {
+            rk::Cfg c{};
+            c.R = R;
+            c.C = kn.C;
+            c.W = W;
+            c.z0 = d.fs - 1;
+            const int cols = W * c.C;
+            c.P = d.nxp <= cols ? 1 : cols > 2 * rk::kH ? cdiv(d.nxp - 2 * rk::kH, cols - 2 * rk::kH) : 0;
+            // a window's first and last six columns in one wave each, three own columns at least
+            if (c.P < 1 || (c.P > 1 && (c.C < 2 * rk::kH || cols < 3 * rk::kH))) continue;
+            const size_t lds = fwd_lds_bytes(c, NS);
+            if (lds + 1024 > kCuLds) continue;
+            const int per_cu = std::min(cu_waves / W, (int)(kCuLds / (lds + 1024)));
+            if (c.P > per_cu * ncu) continue;
+            const int rounds = cdiv(ns, std::min(ns, per_cu * ncu / c.P));
+            c.G = cdiv(ns, rounds);
+            const double t = rounds * resident_step_us(W * cdiv(c.G * c.P, ncu), 36.0 * c.C * R, c.P > 1);
+            if (t < best_t) {
+                best_t = t;
+                *best = c;
+            }
+        }
+    }
+    return best_t < 1e30;
+}
+
+const FwdKernel *find_fwd(int R, int C) {
+    for (const FwdKernel &k : kFwdKernels)
+        if (k.R == R && k.C == C) return &k;
+    return nullptr;
+}
+
+}  // namespace
+
+// Lanes whose p rows the forward stages in LDS: those of the strips' rows and of every
+// receiver's; all lanes if that is more than 8 (the receivers are then written directly).
+static unsigned long long resident_stage_lanes(const swit_plan *pl, int R, int z0, bool *direct) {
+    const Dims &d = pl->d;
+    unsigned long long m = 0;
+    auto row = [&](int z) { m |= 1ull << ((z - z0) / R); };
+    for (int k = 0; k < 3; ++k) row(d.fs + k);
+    row(d.npml + d.nz);
+    row(d.npml + d.nz - 1);
+    const unsigned long long strips = m;
+    for (int s = 0; s < pl->ns; ++s)
+        for (int r = 0; r < pl->geo_h[s].ng; ++r) row(pl->rec_cells_fwd[(size_t)s * d.ngmax + r] % d.ld + 1);
+    *direct = __builtin_popcountll(m) > 8;
+    return *direct ? strips : m;
+}
+
+// Receivers by window and thread cell: slots are numbered in that order, a receiver's slot in
+// map.  Staged: rtab, rbase (every window's count fits two per thread); direct: rec.
+static void resident_receivers(const swit_plan *pl, const rk::Cfg &c, unsigned long long pmask, bool *direct,
+                               std::vector<int> &rtab, std::vector<int> &rbase, std::vector<uint4> &rec,
+                               std::vector<int> &map) {
+    const Dims &d = pl->d;
+    const int T = c.W * 64;
+    map.assign((size_t)pl->ns * d.ngmax, -1);
+    rbase.assign((size_t)pl->ns * c.P, 0);
+    rtab.assign((size_t)pl->ns * c.P * 2 * T, -1);
+    rec.assign((size_t)pl->ns * c.P * T, make_uint4(0, 0, 0, 0));
+    struct Cell {
+        int j, col, row, r;
+        bool operator<(const Cell &o) const {
+            return j != o.j ? j < o.j : col != o.col ? col < o.col : row != o.row ? row < o.row : r < o.r;
+        }
+    };
+    std::vector<Cell> cell;
+    for (int s = 0; s < pl->ns; ++s) {
+        cell.clear();
+        for (int r = 0; r < pl->geo_h[s].ng; ++r) {
+            const int o = pl->rec_cells_fwd[(size_t)s * d.ngmax + r];
+            const int z = o % d.ld + 1, x = o / d.ld + 1;
+            int j = 0;
+            while (x > rk::window_oe(c.W, c.C, j, c.P, d.nxp)) ++j;
+            cell.push_back(Cell{j, x - rk::window_x(c.W, c.C, j), z - c.z0, r});
+        }
+        // by window, thread (wave, lane) and bit, as the direct writes number them
+        auto key = [&](const Cell &q) {
+            return (((long long)q.j * T + (q.col / c.C) * 64 + q.row / c.R) * 64) + (q.col % c.C) * c.R + q.row % c.R;
+        };
+        std::stable_sort(cell.begin(), cell.end(), [&](const Cell &x, const Cell &y) { return key(x) < key(y); });
+        int slot = -1, first = 0, lastj = -1;
+        long long last = -1;
+        for (const Cell &q : cell) {
+            if (key(q) != last) {
+                ++slot;
+                if (q.j != lastj) {
+                    first = slot;
+                    rbase[(size_t)s * c.P + q.j] = slot;
+                    lastj = q.j;
+                }
+                last = key(q);
+                uint4 &t = rec[((size_t)s * c.P + q.j) * T + (q.col / c.C) * 64 + q.row / c.R];
+                const int bit = (q.col % c.C) * c.R + q.row % c.R, n = slot - first;
+                if (!t.x && !t.y) t.z = slot;
+                (bit < 32 ? t.x : t.y) |= 1u << (bit % 32);
+                if (n >= 2 * T) *direct = true;
+                else if (!*direct)
+                    rtab[((size_t)s * c.P + q.j) * 2 * T + n] =
+                        (__builtin_popcountll(pmask & ((1ull << (q.row / c.R)) - 1)) * c.W * c.C + q.col) * c.R + q.row % c.R;
+            }
+            map[(size_t)s * d.ngmax + q.r] = slot;
+        }
+    }
+}
+
+static int resident_init(swit_plan *pl) {
+    ResidentState &rs = pl->res;
+    const Dims &d = pl->d;
+    int dev = 0, ncu = 0;
+    HIP_TRY(hipGetDevice(&dev));
+    HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    rs.fwd = choose_fwd(d, pl->ns, ncu, 8, &rs.fc);
+    if (!rs.fwd) return SWIT_OK;
+    const rk::Cfg &c = rs.fc;
+    bool direct = false;
+    rs.f_pmask = resident_stage_lanes(pl, c.R, c.z0, &direct);
+    rs.f_lds = fwd_lds_bytes(c, __builtin_popcountll(rs.f_pmask));
+    for (auto *fn : find_fwd(c.R, c.C)->fn)
+        HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rs.f_lds));
+    rs.f_ncol = d.nxp + c.W * c.C;
+    const size_t col = (size_t)64 * c.R;
+    TRY(pl->alloc(&rs.f_co, (rs.f_ncol + 1) * 5 * col));
+    TRY(pl->alloc(&rs.f_fpx, rs.f_ncol + 1));
+    std::vector<int> rtab, rbase, map;
+    std::vector<uint4> rec;
+    resident_receivers(pl, c, rs.f_pmask, &direct, rtab, rbase, rec, map);
+    if (direct) {
+        TRY(pl->alloc(&rs.f_rec, rec.size()));
+        HIP_TRY(hipMemcpy(rs.f_rec, rec.data(), sizeof(uint4) * rec.size(), hipMemcpyHostToDevice));
+    } else {
+        TRY(pl->alloc(&rs.f_rtab, rtab.size()));
+        HIP_TRY(hipMemcpy(rs.f_rtab, rtab.data(), sizeof(int) * rtab.size(), hipMemcpyHostToDevice));
+    }
+    TRY(pl->alloc(&rs.f_rbase, rbase.size()));
+    TRY(pl->alloc(&rs.f_map, map.size()));
+    HIP_TRY(hipMemcpy(rs.f_rbase, rbase.data(), sizeof(int) * rbase.size(), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(rs.f_map, map.data(), sizeof(int) * map.size(), hipMemcpyHostToDevice));
+    rs.f_msg = c.P > 1 ? (size_t)c.G * c.P * 4 * rk::kFromRight * c.R * 64 : 0;
+    TRY(pl->alloc(&rs.msg, rs.f_msg));
+    TRY(pl->alloc(&rs.ctl, 1));
+    return SWIT_OK;
+}
+
+static int resident_set_model(swit_plan *pl, hipStream_t st) {
+    ResidentState &rs = pl->res;
+    const BatchedState &bs = pl->bat;
+    const Dims &d = pl->d;
+    if (rs.fwd) {
+        hipLaunchKernelGGL(rk::k_res_setup, dim3(rs.fc.R, rs.f_ncol + 1), dim3(64), 0, st, d, rs.fc.R, rs.fc.z0,
+                           rs.f_ncol, d.fs + 1, d.fs, 0, bs.KB, bs.CP, bs.CV, rs.f_co, rs.f_fpx);
+        LAUNCH_CHECK();
+    }
+    return SWIT_OK;
+}
+
+// Whether a job on stream st takes the resident loops: not inside a capture (a replay would
+// find the words of the launch before it).
+static int resident_now(bool built, int use, hipStream_t st, bool *yes) {
+    *yes = false;
+    if (!built || !use) return SWIT_OK;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(st, &cs));
+    *yes = cs == hipStreamCaptureStatusNone;
+    return SWIT_OK;
+}
+
+static int resident_begin(swit_plan *pl, size_t words, bool first, hipStream_t st) {
+    ResidentState &rs = pl->res;
+    const int blocks = (int)std::min<size_t>(words / 256 + 1, 2048);
+    hipLaunchKernelGGL(rk::k_res_begin, dim3(blocks), dim3(256), 0, st, rs.msg, words, rs.ctl, first ? 1 : 0);
+    LAUNCH_CHECK();
+    return SWIT_OK;
+}
+
+// Forward steps it0 .. it1 of every shot in one launch.
+static int resident_forward_steps(swit_plan *pl, int it0, int it1, const float *src, int save, DSave hist,
+                                  const float *in, float *out, float *end, bool first, hipStream_t st) {
+    ResidentState &rs = pl->res;
+    BatchedState &bs = pl->bat;
+    TRY(resident_begin(pl, rs.f_msg, first, st));
+    rk::FwdArgs a{};
+    a.d = pl->d;
+    a.c = rs.fc;
+    a.s0 = 0;
+    a.ns = pl->ns;
+    a.it0 = it0;
+    a.it1 = it1;
+    a.co = rs.f_co;
+    a.ncol = rs.f_ncol;
+    a.fpx = rs.f_fpx;
+    a.geo = pl->geo;
+    a.src = src;
+    a.rtab = rs.f_rtab;
+    a.rbase = rs.f_rbase;
+    a.rec = rs.f_rec;
+    a.pmask = rs.f_pmask;
+    a.seis_t = pl->seis_t;
+    a.strips = !save ? nullptr : bs.strip_mode == 0 ? pl->strips : bs.ring;
+    a.s_rows = bs.strip_mode == 0 ? pl->d.nt : kStripRing;
+    a.hist = hist;
+    a.in = in;
+    a.out = out;
+    a.end = end;
+    a.msg = rs.msg;
+    a.ctl = rs.ctl;
+    hipLaunchKernelGGL(find_fwd(rs.fc.R, rs.fc.C)->fn[hist.p ? 1 : 0], dim3(rs.fc.G * rs.fc.P), dim3(64 * rs.fc.W), rs.f_lds, st, a);
+    LAUNCH_CHECK();
+    return SWIT_OK;
+}
+
+static int resident_traces(swit_plan *pl, float *seis, hipStream_t st) {
+    const Dims &d = pl->d;
+    hipLaunchKernelGGL(rk::k_res_traces, dim3(cdiv(d.ngmax, 32), cdiv(d.nt, 32), pl->ns), dim3(32, 8), 0, st, d.nt,
+                       d.ngmax, pl->res.f_map, pl->seis_t, seis, pl->res.ctl);
+    LAUNCH_CHECK();
+    return SWIT_OK;
+}
+
+// The whole forward job: strips as batched_forward saves them.  16-bit plans stop at every
+// full ring (the state goes through F) and encode it.
+static int resident_forward(swit_plan *pl, const float *src, float *seis, int save, hipStream_t st) {
+    BatchedState &bs = pl->bat;
+    const Dims &d = pl->d;
+    BatchedState::Timed t{0, (long long)d.nt - 1, nullptr, nullptr};
+    hipLaunchKernelGGL(k_zero_rows, dim3(pl->ns), dim3(256), 0, st, pl->seis_t, (size_t)d.nt * d.ngmax, d.ngmax);
+    if (save && bs.strip_mode == 0)
+        hipLaunchKernelGGL(k_zero_rows, dim3(pl->ns), dim3(256), 0, st, pl->strips, (size_t)d.nt * d.S, d.S);
+    else if (save) {
+        hipLaunchKernelGGL(k_zero_rows16, dim3(pl->ns), dim3(256), 0, st, bs.strips16, (size_t)d.nt * d.S, d.S);
+        TRY(fill(reinterpret_cast<float *>(bs.smax), (size_t)pl->ns * d.nt, st));
+    }
+    LAUNCH_CHECK();
+    if (bs.profile) {
+        TRY(pool_event(bs, &t.e0));
+        TRY(pool_event(bs, &t.e1));
+        bs.pending.push_back(t);
+        HIP_TRY(hipEventRecord(t.e0, st));
+    }
+    const DSave none{nullptr, 0, 0};
+    if (!save || bs.strip_mode == 0) {
+        TRY(resident_forward_steps(pl, 2, d.nt, src, save, none, nullptr, nullptr, save ? bs.end : nullptr, true, st));
+    } else {
+        int k = 0;
+        for (int a = 2; a <= d.nt; ++k) {
+            // rows a - 1 .. b - 1, the last one in the ring's last slot
+            const int b = std::min(d.nt, a + kStripRing - 1 - (a - 1) % kStripRing);
+            TRY(resident_forward_steps(pl, a, b, src, save, none, a == 2 ? nullptr : bs.F[(k + 1) & 1],
+                                       b == d.nt ? nullptr : bs.F[k & 1], b == d.nt ? bs.end : nullptr, a == 2, st));
+            launch_encode(pl, a - 1, b - 1, st);
+            LAUNCH_CHECK();
+            a = b + 1;
+        }
+    }
+    if (bs.profile) HIP_TRY(hipEventRecord(t.e1, st));
+    return resident_traces(pl, seis, st);
+}
+
+// The resident loops against the step kernels' best times us[0] (forward), us[1] (backward)
+// per time step: each is used where it is faster, and us gets its time.  A job of up to 200
+// steps is timed (best of three).
+static int resident_autotune(swit_plan *pl, double *us, hipStream_t st) {
+    ResidentState &rs = pl->res;
+    BatchedState &bs = pl->bat;
+    const Dims &d = pl->d;
+    if (!rs.fwd) return SWIT_OK;
+    hipEvent_t e0, e1;
+    TRY(pool_event(bs, &e0));
+    TRY(pool_event(bs, &e1));
+    const int it1 = std::min(d.nt, 201);
+    const int save = (pl->flags & SWIT_PLAN_NO_STRIPS) ? 0 : 1;
+    double best = 1e30;
+    for (int k = 0; k < 4; ++k) {
+        HIP_TRY(hipEventRecord(e0, st));
+        TRY(resident_forward_steps(pl, 2, it1, bs.src, save, DSave{nullptr, 0, 0}, nullptr, nullptr, nullptr, true, st));
+        HIP_TRY(hipEventRecord(e1, st));
+        HIP_TRY(hipEventSynchronize(e1));
+        float ms = 0.0f;
+        HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
+        if (k) best = std::min(best, 1000.0 * ms / (it1 - 1));
+    }
+    rs.use_fwd = best < us[0];
+    if (rs.use_fwd) us[0] = best;
+    bs.ev_pool.push_back(e0);
+    bs.ev_pool.push_back(e1);
+    return SWIT_OK;
+}
+
 // ---- options and measurement -----------------------------------------------------------
 
 // Captured graphs hold the launch arguments: drop them when those change.
@@ -1328,7 +1701,7 @@ extern "C" int swit_plan_autotune(swit_plan *pl, int steps, int *choice, double 
     choice[5] = bbal;
     us[0] = best_f;
     us[1] = sp_max ? best_b : 0.0;
-    return SWIT_OK;
+    return resident_autotune(pl, us, stream);
 }
 
 extern "C" int swit_plan_set_option(swit_plan *pl, int option, int value) {
@@ -1351,6 +1724,7 @@ extern "C" int swit_plan_set_option(swit_plan *pl, int option, int value) {
         if (value < 1 || value > pl->ns) return set_err(SWIT_EINVAL, "group size %d outside [1, ns]", value);
         bs.Gf = value;
         bs.ngroups_f = cdiv(pl->ns, value);
+        pl->res.use_fwd = 0;
         drop_graphs(bs);
         return SWIT_OK;
     case SWIT_OPT_FWD_COLGROUP:
@@ -1359,6 +1733,7 @@ extern "C" int swit_plan_set_option(swit_plan *pl, int option, int value) {
         if (value < 1 || value > tm.nxt) return set_err(SWIT_EINVAL, "column group %d outside [1, %d]", value, tm.nxt);
         tm.cg = value;
         if (option == SWIT_OPT_BWD_COLGROUP) bs.bwd2.cg = value;
+        (option == SWIT_OPT_BWD_COLGROUP ? pl->res.use_bwd : pl->res.use_fwd) = 0;
         drop_graphs(bs);
         return SWIT_OK;
     }
@@ -1369,11 +1744,13 @@ extern "C" int swit_plan_set_option(swit_plan *pl, int option, int value) {
         if (wi < 0) return set_err(SWIT_EINVAL, "backward tile width %d is not one of %d, %d", value, bk::kBTXs[0],
                                    bk::kBTXs[1]);
         select_bwd_width(bs, wi);
+        pl->res.use_bwd = 0;
         drop_graphs(bs);
         return SWIT_OK;
     }
     case SWIT_OPT_EXACT_FUSED:
         bs.exact_fused = value != 0;
+        pl->res.use_exact = 0;
         if (bs.gex_b) { (void)hipGraphExecDestroy(bs.gex_b); bs.gex_b = nullptr; }
         for (auto &row : bs.gex_h)
             for (auto &g : row)
@@ -1382,15 +1759,21 @@ extern "C" int swit_plan_set_option(swit_plan *pl, int option, int value) {
     case SWIT_OPT_BWD_STEPS:
         if (value != 1 && value != 2) return set_err(SWIT_EINVAL, "backward steps per launch must be 1 or 2");
         bs.bwd_steps = value;
+        pl->res.use_bwd = 0;
         drop_graphs(bs);
         return SWIT_OK;
     case SWIT_OPT_STREAMS:
         if (value != 1 && value != 2) return set_err(SWIT_EINVAL, "streams must be 1 or 2");
         bs.streams = value;
         return SWIT_OK;
+    case SWIT_OPT_RESIDENT:
+        if (value != 0 && value != 1) return set_err(SWIT_EINVAL, "resident must be 0 or 1");
+        pl->res.use_fwd = pl->res.use_bwd = pl->res.use_exact = value;
+        return SWIT_OK;
     case SWIT_OPT_BWD_BALANCE:
         if (value != 0 && value != 1) return set_err(SWIT_EINVAL, "backward balance must be 0 or 1");
         bs.bwd_balance = value;
+        pl->res.use_bwd = 0;
         drop_graphs(bs);
         return SWIT_OK;
     default:
