@@ -16,12 +16,13 @@
 // through LDS (2 columns of p one way and 1 the other, the same for u).  A step is then
 // two phases (p, then u and w) with one barrier each.
 //
-// Windows overlap: one reaches 3 columns past its own columns on each inner side.  A step
-// spoils them (p needs u at x-2..x+1, u needs p at x-1..x+2), so after every step the
-// windows send each other fresh values of the 3 own columns next to them.  Those columns
-// always are the first and last six of a window, so they sit in known registers of its first
-// and last wave.  These run the velocity phase at raised priority, send, and wait for the
-// neighbour while the other waves still compute.  A message word is 8 bytes, {value, number
+// Windows overlap: one reaches 3 columns past its own columns on each inner side.  p needs u
+// at x-2..x+1 and u needs p at x-1..x+2, so with fresh u in the 3 columns after every forward
+// step (fresh p after every reverse step) the rest of the halo that is needed keeps itself
+// right.  The columns that are sent and received always are the first and last six of a
+// window, so they sit in known registers of its first and last waves.  These run the step's
+// second phase at raised priority, send, and wait for the neighbour while the other waves
+// still compute.  A message word is 8 bytes, {value, number
 // of the message}, stored and polled with relaxed agent-scope atomics: the word that carries
 // a value also says that it has arrived, so no flag, fence or cache flush is needed (measured
 // between workgroups on different XCDs, 64 words: 0.93 us per exchange with tagged words,
@@ -81,11 +82,6 @@ struct Ctl {
     int err;
 };
 
-// Columns of a message.  From the left: u of the three halo columns, p and w of the last (the
-// others' cannot be updated by the next step); from the right: u of the three, p and w of
-// the first two.  R rows of 64 lanes each.
-constexpr int kFromLeft = 5, kFromRight = 7;
-
 struct FwdArgs {
     Dims d;
     Cfg c;
@@ -110,7 +106,7 @@ struct FwdArgs {
     const float *in;            // null (zero state) or [ns][3][nxp][ld]
     float *out;                 // null or [ns][3][nxp][ld]
     float *end;                 // null or [ns][3][nx][nz]
-    u64 *msg;                   // [G P][2 slots][2 sides][7 R][64]
+    u64 *msg;                   // [G P][2 slots][2 sides][3 R][64]
     Ctl *ctl;
 };
 
@@ -165,6 +161,41 @@ __device__ __forceinline__ void recv_cols(const u64 *in, unsigned tag, Ctl *ctl,
             asm volatile("v_mov_b32 %0, %1" : "=v"(v[n][r]) : "v"((unsigned)q[n][r]));
 }
 
+// A window's first and last six columns: position q from the left (right) end lies in wave
+// q / C (W - 1 - q / C) at column q % C (C - 1 - q % C).  Sends the three own columns next to
+// each neighbour (positions 3, 4, 5) into its inbox; halo column h of the left window's right
+// side is this window's position 3 + h, of the right window's left side position 5 - h.
+template <int R, int C>
+__device__ __forceinline__ void send_edges(bool has_l, bool has_r, int wave, int W, u64 *to_l, u64 *to_r, unsigned tag,
+                                           const float (&f)[C][R]) {
+#pragma unroll
+    for (int h = 0; h < kH; ++h) {
+        const int ql = kH + h, qr = 2 * kH - 1 - h;
+        if (has_l && wave == ql / C) send_col<R>(to_l + h * R * 64, tag, f[ql % C]);
+        if (has_r && wave == W - 1 - qr / C) send_col<R>(to_r + h * R * 64, tag, f[C - 1 - qr % C]);
+    }
+}
+// Fresh halo columns from the inboxes: positions 0, 1, 2 from each end (C >= 3: one wave).
+template <int R, int C>
+__device__ __forceinline__ void recv_edges(bool has_l, bool has_r, int wave, int W, const u64 *from_l,
+                                           const u64 *from_r, unsigned tag, Ctl *ctl, bool &dead, float (&f)[C][R]) {
+    float v[kH][R];
+    if (has_l && wave == 0) {
+        recv_cols<R, kH>(from_l, tag, ctl, dead, v);
+#pragma unroll
+        for (int h = 0; h < kH; ++h)
+#pragma unroll
+            for (int r = 0; r < R; ++r) f[h][r] = v[h][r];
+    }
+    if (has_r && wave == W - 1) {
+        recv_cols<R, kH>(from_r, tag, ctl, dead, v);
+#pragma unroll
+        for (int h = 0; h < kH; ++h)
+#pragma unroll
+            for (int r = 0; r < R; ++r) f[C - kH + h][r] = v[h][r];
+    }
+}
+
 // LDS of a workgroup: the waves' edge columns, the p stage (NS lanes), the u, w stage.
 __host__ __device__ inline int lds_edge_floats(int W, int R) { return W * 6 * R * 64; }
 __host__ __device__ inline int lds_stage_floats(int W, int C, int R, int NS) { return W * C * (NS + 8) * R; }
@@ -211,6 +242,27 @@ __device__ __forceinline__ void buffer_rows(__amdgpu_buffer_rsrc_t rs, unsigned 
         }
     }
 }
+template <int R>
+__device__ __forceinline__ void buffer_store_rows(__amdgpu_buffer_rsrc_t rs, unsigned voff, int soff,
+                                                  const float (&v)[R]) {
+    auto bits = [&](int i) { return __float_as_uint(v[i]); };
+    if constexpr (R == 2) {
+        __builtin_amdgcn_raw_buffer_store_b64(vec2{bits(0), bits(1)}, rs, voff, soff, 0);
+    } else if constexpr (R == 3) {
+        __builtin_amdgcn_raw_buffer_store_b96(vec3{bits(0), bits(1), bits(2)}, rs, voff, soff, 0);
+    } else {
+        __builtin_amdgcn_raw_buffer_store_b128(vec4{bits(0), bits(1), bits(2), bits(3)}, rs, voff, soff, 0);
+        if constexpr (R == 5) __builtin_amdgcn_raw_buffer_store_b32(bits(R > 4 ? 4 : 0), rs, voff + 16, soff, 0);
+        else if constexpr (R == 6)
+            __builtin_amdgcn_raw_buffer_store_b64(vec2{bits(R > 4 ? 4 : 0), bits(R > 5 ? 5 : 0)}, rs, voff + 16, soff, 0);
+        else if constexpr (R == 7)
+            __builtin_amdgcn_raw_buffer_store_b96(vec3{bits(R > 4 ? 4 : 0), bits(R > 5 ? 5 : 0), bits(R > 6 ? 6 : 0)}, rs,
+                                                  voff + 16, soff, 0);
+        else if constexpr (R == 8)
+            __builtin_amdgcn_raw_buffer_store_b128(vec4{bits(R > 4 ? 4 : 0), bits(R > 5 ? 5 : 0), bits(R > 6 ? 6 : 0),
+                                                        bits(R > 7 ? 7 : 0)}, rs, voff + 16, soff, 0);
+    }
+}
 
 // Forward steps it0 .. it1 (fdcore.f90:75-160) of every shot, the state in registers.
 // Bound by vector issue: 28 operations per cell and step without contraction (the
@@ -236,9 +288,10 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
     float *sp = eP + W * 3 * R * 64;                     // p stage [NS][W C][R]
     float *sv = sp + W * C * NS * R;                     // u, w stage [2][4][W C][R]
 
-    // this wave's first column; the first and the last wave exchange with the neighbours
+    // this wave's first column; the first and the last waves exchange with the neighbours
     const int x0w = window_x(W, C, j) + wave * C;
-    const bool edge_l = j > 0 && wave == 0, edge_r = j + 1 < P && wave == W - 1;
+    const bool has_l = j > 0, has_r = j + 1 < P;
+    const bool edge = (has_l && wave <= (2 * kH - 1) / C) || (has_r && wave >= W - 1 - (2 * kH - 1) / C);
     const unsigned voff0 = lane * R * 4;                 // byte offset of this lane's rows in a column
     const bool mirror = a.d.free_surface == 1 && lane == 0;
     // any column in the side layers: their damping factors differ along x; the other waves
@@ -480,7 +533,7 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
             if (a.strips && it > a.it0) copy_velocities(fresh_args<FwdArgs>(), s, it - 2);
             lds_barrier();
             // ---- u, w: p of the neighbouring waves' columns x0-1, x0+C, x0+C+1 ----
-            if (edge_l || edge_r) __builtin_amdgcn_s_setprio(3);
+            if (edge) __builtin_amdgcn_s_setprio(3);
             {
                 float pl1[R], pr1[R], pr2[R];
 #pragma unroll
@@ -517,30 +570,13 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
             }
             // ---- exchange, out: inboxes [group][window][slot][side], side 0 from the left ----
             const bool exch = it < it1;
-            ++tag;
+            if (exch) ++tag;
             u64 *box = nullptr;
-            if ((edge_l || edge_r) && exch) {
+            constexpr int kMsg = kH * R * 64;
+            if (edge && exch) {
                 const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
-                constexpr int kMsg = kFromRight * R * 64;
                 box = k->msg + ((size_t)(grp * k->c.P + j) * 2 + (tag & 1)) * (2 * kMsg) + voff / (4 * R);
-                if (edge_l) {                            // own first three columns: the left window's right halo
-                    u64 *o = box - 3 * kMsg;
-                    send_col<R>(o, tag, u[3]);
-                    send_col<R>(o + R * 64, tag, u[4]);
-                    send_col<R>(o + 2 * R * 64, tag, u[5]);
-                    send_col<R>(o + 3 * R * 64, tag, p[3]);
-                    send_col<R>(o + 4 * R * 64, tag, p[4]);
-                    send_col<R>(o + 5 * R * 64, tag, w[3]);
-                    send_col<R>(o + 6 * R * 64, tag, w[4]);
-                }
-                if (edge_r) {                            // own last three: the right window's left halo
-                    u64 *o = box + 4 * kMsg;
-                    send_col<R>(o, tag, u[C - 6]);
-                    send_col<R>(o + R * 64, tag, u[C - 5]);
-                    send_col<R>(o + 2 * R * 64, tag, u[C - 4]);
-                    send_col<R>(o + 3 * R * 64, tag, p[C - 4]);
-                    send_col<R>(o + 4 * R * 64, tag, w[C - 4]);
-                }
+                send_edges<R, C>(has_l, has_r, wave, W, box - 3 * kMsg, box + 4 * kMsg, tag, u);
             }
             // ---- receivers (fdcore.f90:123-128) and strips (:130-159): all stores of the step
             // come here, p stands since the pressure phase ----
@@ -600,45 +636,9 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
                 }
             }
             // ---- exchange, in: fresh halo columns ----
-            if (edge_l && exch) {
-                const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
-                float v[3][R], q[2][R];
-                recv_cols<R, 3>(box, tag, k->ctl, dead, v);
-                recv_cols<R, 2>(box + 3 * R * 64, tag, k->ctl, dead, q);
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    u[0][r] = v[0][r];
-                    u[1][r] = v[1][r];
-                    u[2][r] = v[2][r];
-                    p[2][r] = q[0][r];
-                    w[2][r] = q[1][r];
-                }
-            }
-            if (edge_r && exch) {
-                const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
-                const u64 *in = box + kFromRight * R * 64;
-                float v[3][R], q[2][R];
-                recv_cols<R, 3>(in, tag, k->ctl, dead, v);
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    u[C - 3][r] = v[0][r];
-                    u[C - 2][r] = v[1][r];
-                    u[C - 1][r] = v[2][r];
-                }
-                recv_cols<R, 2>(in + 3 * R * 64, tag, k->ctl, dead, q);
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    p[C - 3][r] = q[0][r];
-                    p[C - 2][r] = q[1][r];
-                }
-                recv_cols<R, 2>(in + 5 * R * 64, tag, k->ctl, dead, q);
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    w[C - 3][r] = q[0][r];
-                    w[C - 2][r] = q[1][r];
-                }
-            }
-            if (edge_l || edge_r) __builtin_amdgcn_s_setprio(0);
+            if (edge && exch)
+                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, fresh_args<FwdArgs>()->ctl, dead, u);
+            if (edge) __builtin_amdgcn_s_setprio(0);
             put_u();
             srcv = fresh_args<FwdArgs>()->d.dt * src_next;
             lds_barrier();
@@ -686,6 +686,533 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
         lds_barrier();               // the edges and the stage are rewritten by the next shot
     }
 }
+
+struct BwdArgs {
+    Dims d;
+    Cfg c;
+    int s0, ns;                 // shots s0 .. s0 + ns - 1
+    const float *co;            // coefficients as the forward's, adjoint regions (k_res_setup)
+    int ncol;
+    const float *fpx;
+    const ShotGeom *geo;
+    const float *src;           // [ns][nt]
+    const void *strips;         // rows [ns][nt][S]
+    int mode;                   // of the strips: 0 FP32, 1 FP16, 2 BF16
+    const uint32_t *smax;
+    const float *end;           // [ns][3][nx][nz] final forward state
+    // adjoint sources: window w of shot s takes dt times values base[s][w] + n of
+    // adj [ns][nt][ngmax]; n-th value's place in the injection stage itab [ns][P][2][64 W]
+    const float *adj;
+    const int *itab, *ibase;
+    unsigned long long imask;   // lanes of the injection stage
+    int layers;                 // receivers of one cell (1 or 2)
+    float *acc;                 // [ns][nxp][3][64 R] per-shot accumulators, zero at the start
+    u64 *msg;                   // [G P][2 slots][2 sides][2 fields][3 R][64]
+    Ctl *ctl;
+};
+
+// LDS of the backward: the waves' edge columns of both wavefields, then two sets (a step's
+// and the next one's) of: the strip rows' lanes [4][W C][R], w of row nz-1 [W C], the side
+// columns [6][64 R] (p of jx = 1, 2, nx-1, nx, u of jx = 1, nx-1), the injection stage
+// [layers][NI + 1][W C][R] (the last one zeros).
+__host__ __device__ inline int bwd_edge_floats(int W, int R) { return W * 12 * R * 64; }
+__host__ __device__ inline int bwd_set_floats(int W, int C, int R, int NI, int layers) {
+    return 4 * W * C * R + ((W * C + 3) & ~3) + 6 * 64 * R + layers * (NI + 1) * W * C * R;
+}
+
+// Reverse steps nt .. 2 (solver.f90:230-253) of every shot: reconstruction (fdcore.f90:
+// 202-289), adjoint step (:293-375) and imaging (solver.f90:237-239), both wavefields in
+// registers (6 R C <= 150 floats at two waves per SIMD).  A step is: velocities of both
+// fields from p (edges through LDS), strip values into the reconstructed u, w; then
+// pressures, strip values into the reconstructed p, injection and mirror of the adjoint p,
+// imaging.  Strip values and adjoint sources are loaded one step ahead and handed out
+// through LDS.  The accumulators are read and written in memory every step (they stay in
+// L2): the wavefields alone fill the registers.
+template <int R, int C>
+__global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
+    extern __shared__ float lds[];
+    __shared__ int sh_ticket;
+    constexpr int kCol = 64 * R * 4;                     // bytes of a column of one array
+    constexpr int NI6 = (6 * C + 63) / 64;               // strip values of the window's columns per thread
+    const int W = a.c.W, P = a.c.P, T = W * 64;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (threadIdx.x == 0) sh_ticket = (int)atomicAdd(&a.ctl->ticket, 1u);
+    __syncthreads();
+    const int t = __builtin_amdgcn_readfirstlane(sh_ticket);
+    const int grp = __builtin_amdgcn_readfirstlane(t / P), j = __builtin_amdgcn_readfirstlane(t % P);
+    const int WC = W * C, NI = __popcll(a.imask);
+    float *eP = lds;                                     // [W][2 fields][3][R][64]: first, second, last column of p
+    float *eU = eP + W * 6 * R * 64;                     // [W][2 fields][3][R][64]: first, last but one, last of u
+    const int set_floats = bwd_set_floats(W, C, R, NI, a.layers);
+    float *sets = eU + W * 6 * R * 64;
+    const int o_w = 4 * WC * R, o_side = o_w + ((WC + 3) & ~3), o_inj = o_side + 6 * 64 * R;
+    const int xw = window_x(W, C, j), x0w = xw + wave * C;
+    const bool has_l = j > 0, has_r = j + 1 < P;
+    const bool edge = (has_l && wave <= (2 * kH - 1) / C) || (has_r && wave >= W - 1 - (2 * kH - 1) / C);
+    const unsigned voff0 = lane * R * 4;
+    const bool wave_pml = x0w <= a.d.npml || x0w + C - 1 >= a.d.npml + a.d.nx;
+    const __amdgpu_buffer_rsrc_t co = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(a.co), 0, (int)((unsigned)(a.ncol + 1) * 5u * kCol), 0x00027000);
+    unsigned tag = 0;
+    bool dead = false;
+    float fpz[R];
+    buffer_rows<R>(co, voff0, 2 * kCol, fpz);
+    // lanes of the mirror row fs-1 (their first row), of the strips' rows, of the injection
+    const int lm = (a.d.fs - 1 - a.c.z0) / R;
+    const int lb = (a.d.npml + a.d.nz - 1 - a.c.z0) / R;           // row nz - 1
+    const bool mir_lane = lane == lm, mir_w = a.d.free_surface == 1 && lane == lm;
+    const int b_slot = lane <= lm + 1 ? max(lane - lm, 0) : min(max(lane - lb, 0) + 2, 3);
+    const int i_slot = (a.imask >> lane) & 1 ? __popcll(a.imask & ((1ull << lane) - 1)) : NI;
+    // rows of this lane: bit r: a strip row (jz 1..3, nz-1, nz); row nz - 1; bit: any interior row
+    unsigned brow = 0, wrow = 0;
+    bool inner = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int jz = a.c.z0 + lane * R + r - a.d.npml;
+        if ((jz >= 1 && jz <= 3) || jz == a.d.nz - 1 || jz == a.d.nz) brow |= 1u << r;
+        if (jz == a.d.nz - 1) wrow |= 1u << r;
+        inner = inner || (jz >= 1 && jz <= a.d.nz);
+    }
+    const unsigned acc_off = inner ? voff0 : 0x80000000u;          // past the buffer: loads 0, stores nothing
+
+    // ---- values of one step: strip values of the window's columns (n-th: column n / 6, value
+    // n % 6: p of jz = 1, 2, 3, nz, nz-1, w of nz-1), of the side columns, adjoint sources ----
+    struct Step {
+        uint32_t col[NI6], side[3];
+        float inj[2];
+        float scale;
+    };
+    // what thread item n of the side columns is: window column offset, strip place; false: none
+    auto side_item = [&](ArgPtr<BwdArgs> k, int n, int &q, int &jz, int &place) {
+        const int nz = k->d.nz;
+        const int v = n / (64 * R), row = n % (64 * R);
+        jz = k->c.z0 + row - k->d.npml;
+        if (v >= 6 || jz < 1 || jz > nz) return false;
+        // v: 0 p(1), 1 p(2), 2 p(nx-1), 3 p(nx), 4 u(1), 5 u(nx-1)
+        const int nx = k->d.nx;
+        const int jx = v == 0 || v == 4 ? 1 : v == 1 ? 2 : v == 3 ? nx : nx - 1;
+        const int x = k->d.npml + jx, xw_ = window_x(k->c.W, C, j);
+        q = v == 0 ? 0 : v == 1 ? 1 : v == 2 ? 4 : v == 3 ? 3 : v == 4 ? 2 : 5;
+        place = v * 64 * R + row;
+        return x >= xw_ && x < xw_ + k->c.W * C;
+    };
+    // The side columns of a window: left three (v = 0, 1, 4), right three, or both.  Items are
+    // the 6 x 64 R places, T at a time; windows without side columns take none.
+    const bool win_side = (xw <= a.d.npml + 2 && xw + WC > a.d.npml + 1) ||
+                          (xw <= a.d.npml + a.d.nx && xw + WC > a.d.npml + a.d.nx - 1);
+    auto load_step = [&](int s, int it, Step &v, int i0, int i1, int ib) {
+        const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
+        const int S = k->d.S, nx = k->d.nx, nz = k->d.nz;
+        const size_t row = (size_t)s * k->d.nt + (it - 2);
+        const int mode = k->mode;
+        const char *b = (const char *)k->strips + row * S * (mode == 0 ? 4 : 2);
+        auto get = [&](int i) -> uint32_t {
+            if (mode == 0) return ((const uint32_t *)b)[i];
+            return ((const uint16_t *)b)[i];
+        };
+        v.scale = mode ? strip_scale(k->smax[row]) : 1.0f;
+        const int top0 = 3 * nx + 6 * nz, xw_ = window_x(k->c.W, C, j), WC_ = k->c.W * C, T_ = k->c.W * 64;
+        unsigned tid = threadIdx.x;
+        opaque_v(tid);
+#pragma unroll
+        for (int i = 0; i < NI6; ++i) {
+            const int n = tid + i * T_, col = n / 6, q = n % 6, jx = xw_ + col - k->d.npml;
+            v.col[i] = 0;
+            if (col < WC_ && jx >= 1 && jx <= nx)
+                v.col[i] = get(q < 3 ? top0 + 6 * (jx - 1) + q : 3 * (jx - 1) + q - 3);
+        }
+        if (win_side) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                int q, jz, place;
+                v.side[i] = 0;
+                // places past 3 T (few waves): see store_step
+                if (side_item(k, tid + i * T_, q, jz, place)) v.side[i] = get(3 * nx + 6 * (jz - 1) + q);
+            }
+        }
+        const float *adj = k->adj + ((size_t)s * k->d.nt + (it - 1)) * k->d.ngmax + ib;
+        v.inj[0] = i0 >= 0 ? adj[tid] : 0.0f;
+        v.inj[1] = i1 >= 0 ? adj[tid + T_] : 0.0f;
+    };
+    auto decode = [&](int mode, uint32_t x, float scale) -> float {
+        if (mode == 0) return __uint_as_float(x);
+        return (mode == 1 ? strip_decode<1>((uint16_t)x) : strip_decode<2>((uint16_t)x)) * scale;
+    };
+    // values into set `par` of the LDS; i0, i1: this thread's injection places
+    auto store_step = [&](int s, int it, const Step &v, int par, int i0, int i1) {
+        const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
+        const int nz = k->d.nz, npml = k->d.npml, WC_ = k->c.W * C, T_ = k->c.W * 64, z0 = k->c.z0, mode = k->mode;
+        float *f = sets + par * set_floats;
+        unsigned tid = threadIdx.x;
+        opaque_v(tid);
+#pragma unroll
+        for (int i = 0; i < NI6; ++i) {
+            const int n = tid + i * T_, col = n / 6, q = n % 6;
+            if (col >= WC_) continue;
+            const float x = decode(mode, v.col[i], v.scale);
+            if (q == 5) {
+                f[o_w + col] = x;
+            } else {
+                const int row = (q < 3 ? q + 1 : q == 3 ? nz : nz - 1) + npml - z0, L = row / R;
+                f[((L <= lm + 1 ? L - lm : 2 + L - lb) * WC_ + col) * R + row % R] = x;
+            }
+        }
+        if (win_side) {
+            int q, jz, place;
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                if (side_item(k, tid + i * T_, q, jz, place)) f[o_side + place] = decode(mode, v.side[i], v.scale);
+            // the rest, for workgroups of few waves: loaded here
+            for (int n = tid + 3 * T_; n < 6 * 64 * R; n += T_)
+                if (side_item(k, n, q, jz, place)) {
+                    const size_t i = ((size_t)s * k->d.nt + (it - 2)) * k->d.S + 3 * k->d.nx + 6 * (jz - 1) + q;
+                    const uint32_t x = mode == 0 ? ((const uint32_t *)k->strips)[i] : ((const uint16_t *)k->strips)[i];
+                    f[o_side + place] = decode(mode, x, v.scale);
+                }
+        }
+        if (i0 >= 0) f[o_inj + i0] = k->d.dt * v.inj[0];
+        if (i1 >= 0) f[o_inj + i1] = k->d.dt * v.inj[1];
+    };
+
+    for (int s = a.s0 + grp; s < a.s0 + a.ns; s += a.c.G) {
+        const int isx = a.geo[s].isx_i + a.d.npml, isz = a.geo[s].isz_i + a.d.npml;   // padded cell
+        const bool src_in = a.geo[s].isx_i > 2 && a.geo[s].isx_i < a.d.nx - 1 && a.geo[s].isz_i > 3 &&
+                            a.geo[s].isz_i < a.d.nz - 1;
+        const float *src = a.src + (size_t)s * a.d.nt;
+        const int i0 = a.itab[((size_t)s * P + j) * 2 * T + threadIdx.x];
+        const int i1 = a.itab[((size_t)s * P + j) * 2 * T + T + threadIdx.x];
+        const int ib = a.ibase[s * P + j];
+        for (int i = threadIdx.x; i < 2 * set_floats; i += T) sets[i] = 0.0f;
+        float pr[C][R], ur[C][R], wr[C][R], pa[C][R], ua[C][R], wa[C][R];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int r = 0; r < R; ++r) pr[c][r] = ur[c][r] = wr[c][r] = pa[c][r] = ua[c][r] = wa[c][r] = 0.0f;
+        {
+            const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
+            int x0 = x0w;
+            unsigned voff = voff0;
+            opaque_s(x0);
+            opaque_v(voff);
+            const int npml = k->d.npml, nx = k->d.nx, nz = k->d.nz, ni = nx * nz;
+            const int jz0 = k->c.z0 + (int)(voff >> 2) - npml;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const int jx = x0 + c - npml;
+                if (jx < 1 || jx > nx) continue;
+                const float *f = k->end + (size_t)s * 3 * ni + (size_t)(jx - 1) * nz;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    if (jz0 + r < 1 || jz0 + r > nz) continue;
+                    const unsigned o = jz0 + r - 1;
+                    pr[c][r] = f[o];
+                    ur[c][r] = f[ni + o];
+                    wr[c][r] = f[2 * ni + o];
+                }
+            }
+        }
+        __syncthreads();
+        Step nxt;
+        load_step(s, a.d.nt, nxt, i0, i1, ib);
+        store_step(s, a.d.nt, nxt, a.d.nt & 1, i0, i1);
+        // p of the edge columns for the next step
+        auto put_p = [&]() {
+            float *e = eP + (size_t)wave * 6 * R * 64 + lane;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                e[r * 64] = pr[0][r];
+                e[(R + r) * 64] = pr[1][r];
+                e[(2 * R + r) * 64] = pr[C - 1][r];
+                e[(3 * R + r) * 64] = pa[0][r];
+                e[(4 * R + r) * 64] = pa[1][r];
+                e[(5 * R + r) * 64] = pa[C - 1][r];
+            }
+        };
+        // edge column `q` (0, 1, 2; + 3 for the adjoint) of a neighbouring wave, zero past the window
+        auto edge_rows = [&](const float *e, int w, int q, float (&v)[R]) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                v[r] = w >= 0 && w < W ? e[((w * 6 + q) * R + r) * 64 + lane] : 0.0f;
+        };
+        put_p();
+        lds_barrier();
+        for (int it = a.d.nt; it >= 2; --it) {
+            int x0 = x0w;
+            unsigned voff = voff0;
+            opaque_s(x0);
+            opaque_v(voff);
+            const float *set = sets + (it & 1) * set_floats;
+            if (it > 2) load_step(s, it - 1, nxt, i0, i1, ib);
+            float ssub;                                  // the reference's s(it+1), 0 past the end
+            {
+                const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
+                ssub = it + 1 <= k->d.nt ? k->d.dt * src[it] : 0.0f;
+            }
+            // ---- velocities: reconstruction (:221-247), adjoint (:310-326) ----
+            {
+                float kp[2][R], kv[2][R], fu[2][R], fw[2][R];
+                auto fetch = [&](int c) {
+                    const int f = wave_pml ? (x0 + c) * (5 * kCol) : 0;
+                    buffer_rows<R>(co, voff, (x0 + c) * (5 * kCol), kp[c & 1]);
+                    buffer_rows<R>(co, voff, (x0 + c) * (5 * kCol) + kCol, kv[c & 1]);
+                    buffer_rows<R>(co, voff, f + 3 * kCol, fu[c & 1]);
+                    buffer_rows<R>(co, voff, f + 4 * kCol, fw[c & 1]);
+                };
+                fetch(0);
+                float rl[R], al[R], r1[R], a1[R], r2[R], a2[R];
+                edge_rows(eP, wave - 1, 2, rl);
+                edge_rows(eP, wave - 1, 5, al);
+                edge_rows(eP, wave + 1, 0, r1);
+                edge_rows(eP, wave + 1, 3, a1);
+                edge_rows(eP, wave + 1, 1, r2);
+                edge_rows(eP, wave + 1, 4, a2);
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    if (c + 1 < C) fetch(c + 1);
+                    {
+                        const float pd = dn1(pr[c][R - 1]), pu0 = up1(pr[c][0]), pu1 = up1(pr[c][1]);
+#pragma unroll
+                        for (int r = 0; r < R; ++r) {
+                            const float xm = c >= 1 ? pr[c - (c >= 1)][r] : rl[r];
+                            const float xp = c + 1 < C ? pr[c + (c + 1 < C)][r] : r1[r];
+                            const float xq = c + 2 < C ? pr[c + (c + 2 < C ? 2 : 0)][r] : c + 2 == C ? r1[r] : r2[r];
+                            const float zm = r >= 1 ? pr[c][r - (r >= 1)] : pd;
+                            const float zp = r + 1 < R ? pr[c][r + (r + 1 < R)] : pu0;
+                            const float zq = r + 2 < R ? pr[c][r + (r + 2 < R ? 2 : 0)] : r + 2 == R ? pu0 : pu1;
+                            ur[c][r] = v_undo(ur[c][r], kp[c & 1][r], pr[c][r], xp, xq, xm);
+                            wr[c][r] = v_undo(wr[c][r], kp[c & 1][r], pr[c][r], zp, zq, zm);
+                        }
+                    }
+                    {
+                        const float pd = dn1(pa[c][R - 1]), pu0 = up1(pa[c][0]), pu1 = up1(pa[c][1]);
+#pragma unroll
+                        for (int r = 0; r < R; ++r) {
+                            const float xm = c >= 1 ? pa[c - (c >= 1)][r] : al[r];
+                            const float xp = c + 1 < C ? pa[c + (c + 1 < C)][r] : a1[r];
+                            const float xq = c + 2 < C ? pa[c + (c + 2 < C ? 2 : 0)][r] : c + 2 == C ? a1[r] : a2[r];
+                            const float zm = r >= 1 ? pa[c][r - (r >= 1)] : pd;
+                            const float zp = r + 1 < R ? pa[c][r + (r + 1 < R)] : pu0;
+                            const float zq = r + 2 < R ? pa[c][r + (r + 2 < R ? 2 : 0)] : r + 2 == R ? pu0 : pu1;
+                            ua[c][r] = v_update_f(ua[c][r], kv[c & 1][r], fu[c & 1][r], pa[c][r], xp, xq, xm);
+                            wa[c][r] = v_update_f(wa[c][r], kv[c & 1][r], fw[c & 1][r], pa[c][r], zp, zq, zm);
+                        }
+                    }
+                    if (mir_w) wa[c][0] = wa[c][1];
+                    // strip value of the reconstructed w, row nz - 1
+                    const float ws = set[o_w + wave * C + c];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        if (wrow & (1u << r)) wr[c][r] = ws;
+                        pin(ur[c][r]);
+                        pin(wr[c][r]);
+                        pin(ua[c][r]);
+                        pin(wa[c][r]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // strip values of the reconstructed u, columns jx = 1 and nx - 1
+            if (win_side) {
+                const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
+                const int c1 = k->d.npml + 1 - x0, cn = k->d.npml + k->d.nx - 1 - x0;
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+                    if (c == c1 || c == cn) {
+                        const float *q = set + o_side + (c == c1 ? 4 : 5) * 64 * R + voff / 4;
+#pragma unroll
+                        for (int r = 0; r < R; ++r) ur[c][r] = q[r];
+                    }
+            }
+            {
+                float *e = eU + (size_t)wave * 6 * R * 64 + lane;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    e[r * 64] = ur[0][r];
+                    e[(R + r) * 64] = ur[C - 2][r];
+                    e[(2 * R + r) * 64] = ur[C - 1][r];
+                    e[(3 * R + r) * 64] = ua[0][r];
+                    e[(4 * R + r) * 64] = ua[C - 2][r];
+                    e[(5 * R + r) * 64] = ua[C - 1][r];
+                }
+            }
+            // the reconstruction's source subtraction
+            if (src_in && (unsigned)(isx - x0) < (unsigned)C) {
+                const int zr = fresh_args<BwdArgs>()->c.z0 + (int)(voff >> 2);
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+                    if (x0 + c == isx) {
+#pragma unroll
+                        for (int r = 0; r < R; ++r)
+                            if (zr + r == isz) pr[c][r] = pr[c][r] - ssub;
+                    }
+            }
+            lds_barrier();
+            // ---- pressures: reconstruction (:250-287), adjoint (:336-373), imaging ----
+            if (edge) __builtin_amdgcn_s_setprio(3);
+            {
+                const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
+                const ArgPtr<float> fpx = (ArgPtr<float>)k->fpx + x0;
+                const int c1 = k->d.npml + 1 - x0, cn = k->d.npml + k->d.nx - x0;   // columns of jx = 1, nx
+                const int os = window_os(k->c.W, C, j), oe = window_oe(k->c.W, C, j, k->c.P, k->d.nxp);
+                const int ca = max(c1, os - x0), cb = min(cn, oe - x0);             // columns imaged here
+                const __amdgpu_buffer_rsrc_t ab = __builtin_amdgcn_make_buffer_rsrc(
+                    k->acc + (size_t)s * k->d.nxp * (3 * 64 * R), 0, (int)((unsigned)k->d.nxp * 3u * kCol), 0x00027000);
+                const unsigned ao = voff + (acc_off - voff0);
+                float kp[2][R], kv[2][R], g0[2][R], g1[2][R], g2[2][R];
+                auto fetch = [&](int c) {
+                    buffer_rows<R>(co, voff, (x0 + c) * (5 * kCol), kp[c & 1]);
+                    buffer_rows<R>(co, voff, (x0 + c) * (5 * kCol) + kCol, kv[c & 1]);
+                    if (c >= ca && c <= cb) {
+                        const int o = (x0 + c - 1) * (3 * kCol);
+                        buffer_rows<R>(ab, ao, o, g0[c & 1]);
+                        buffer_rows<R>(ab, ao, o + kCol, g1[c & 1]);
+                        buffer_rows<R>(ab, ao, o + 2 * kCol, g2[c & 1]);
+                    }
+                };
+                fetch(0);
+                float r2[R], a2[R], r1[R], a1[R], rr[R], ar[R];
+                edge_rows(eU, wave - 1, 1, r2);
+                edge_rows(eU, wave - 1, 4, a2);
+                edge_rows(eU, wave - 1, 2, r1);
+                edge_rows(eU, wave - 1, 5, a1);
+                edge_rows(eU, wave + 1, 0, rr);
+                edge_rows(eU, wave + 1, 3, ar);
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    if (c + 1 < C) fetch(c + 1);
+                    const float fx = fpx[c];
+                    {
+                        const float wd1 = dn1(wr[c][R - 1]), wd2 = dn1(wr[c][R - 2]), wu = up1(wr[c][0]);
+                        const float *q = set + (b_slot * WC + wave * C + c) * R;
+#pragma unroll
+                        for (int r = 0; r < R; ++r) {
+                            const float um1 = c >= 1 ? ur[c - (c >= 1)][r] : r1[r];
+                            const float um2 = c >= 2 ? ur[c - (c >= 2 ? 2 : 0)][r] : c == 1 ? r1[r] : r2[r];
+                            const float up = c + 1 < C ? ur[c + (c + 1 < C)][r] : rr[r];
+                            const float wm1 = r >= 1 ? wr[c][r - (r >= 1)] : wd1;
+                            const float wm2 = r >= 2 ? wr[c][r - (r >= 2 ? 2 : 0)] : r == 1 ? wd1 : wd2;
+                            const float wp1 = r + 1 < R ? wr[c][r + (r + 1 < R)] : wu;
+                            const float v = p_undo(pr[c][r], kv[c & 1][r], ur[c][r], um1, up, um2, wr[c][r], wm1, wp1,
+                                                   wm2);
+                            pr[c][r] = brow & (1u << r) ? q[r] : v;
+                        }
+                    }
+                    if (win_side && (c == c1 || c == c1 + 1 || c == cn - 1 || c == cn)) {
+                        const float *q = set + o_side + (c == c1 ? 0 : c == c1 + 1 ? 1 : c == cn ? 3 : 2) * 64 * R + voff / 4;
+#pragma unroll
+                        for (int r = 0; r < R; ++r) pr[c][r] = q[r];
+                    }
+                    float old[R];
+                    {
+                        const float wd1 = dn1(wa[c][R - 1]), wd2 = dn1(wa[c][R - 2]), wu = up1(wa[c][0]);
+                        const float *q = set + o_inj + (i_slot * WC + wave * C + c) * R;
+#pragma unroll
+                        for (int r = 0; r < R; ++r) {
+                            const float um1 = c >= 1 ? ua[c - (c >= 1)][r] : a1[r];
+                            const float um2 = c >= 2 ? ua[c - (c >= 2 ? 2 : 0)][r] : c == 1 ? a1[r] : a2[r];
+                            const float up = c + 1 < C ? ua[c + (c + 1 < C)][r] : ar[r];
+                            const float wm1 = r >= 1 ? wa[c][r - (r >= 1)] : wd1;
+                            const float wm2 = r >= 2 ? wa[c][r - (r >= 2 ? 2 : 0)] : r == 1 ? wd1 : wd2;
+                            const float wp1 = r + 1 < R ? wa[c][r + (r + 1 < R)] : wu;
+                            old[r] = pa[c][r];
+                            pa[c][r] = p_update_f(pa[c][r], kp[c & 1][r], fminf(fx, fpz[r]), ua[c][r], um1, up, um2,
+                                                  wa[c][r], wm1, wp1, wm2);
+                            pa[c][r] = pa[c][r] + q[r];
+                        }
+                        if (k->layers > 1) {
+                            const float *q2 = q + (NI + 1) * WC * R;
+#pragma unroll
+                            for (int r = 0; r < R; ++r) pa[c][r] = pa[c][r] + q2[r];
+                        }
+                        const float pm = R > 2 ? pa[c][R > 2 ? 2 : 0] : up1(pa[c][0]);
+                        if (mir_lane) pa[c][0] = -pm;
+                    }
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        pin(pr[c][r]);
+                        pin(pa[c][r]);
+                    }
+                    if (c >= ca && c <= cb) {
+                        const int o = (x0 + c - 1) * (3 * kCol);
+#pragma unroll
+                        for (int r = 0; r < R; ++r) {
+                            g0[c & 1][r] = g0[c & 1][r] + pr[c][r] * (old[r] - pa[c][r]);
+                            g1[c & 1][r] = g1[c & 1][r] + pr[c][r] * pr[c][r];
+                            g2[c & 1][r] = g2[c & 1][r] + pa[c][r] * pa[c][r];
+                        }
+                        buffer_store_rows<R>(ab, ao, o, g0[c & 1]);
+                        buffer_store_rows<R>(ab, ao, o + kCol, g1[c & 1]);
+                        buffer_store_rows<R>(ab, ao, o + 2 * kCol, g2[c & 1]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // ---- exchange of p, the next step's values ----
+            const bool exch = it > 2;
+            if (exch) ++tag;
+            constexpr int kMsg = 2 * kH * R * 64;
+            u64 *box = nullptr;
+            if (edge && exch) {
+                const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
+                box = k->msg + ((size_t)(grp * k->c.P + j) * 2 + (tag & 1)) * (2 * kMsg) + voff / (4 * R);
+                send_edges<R, C>(has_l, has_r, wave, W, box - 3 * kMsg, box + 4 * kMsg, tag, pr);
+                send_edges<R, C>(has_l, has_r, wave, W, box - 3 * kMsg + kMsg / 2, box + 4 * kMsg + kMsg / 2, tag, pa);
+            }
+            if (exch) store_step(s, it - 1, nxt, (it - 1) & 1, i0, i1);
+            if (edge && exch) {
+                const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
+                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, dead, pr);
+                recv_edges<R, C>(has_l, has_r, wave, W, box + kMsg / 2, box + kMsg + kMsg / 2, tag, k->ctl, dead, pa);
+            }
+            if (edge) __builtin_amdgcn_s_setprio(0);
+            put_p();
+            lds_barrier();
+        }
+    }
+}
+
+// Cross-shot FP64 sum of the resident backward's accumulators and g = -2 g / c (as
+// k_reduce_acc); NaN if a wait of the job ran out.
+__global__ void k_res_reduce(Dims d, int ns, int R, int z0, const float *__restrict__ vp, const float *__restrict__ acc,
+                             double *__restrict__ grad, double *__restrict__ fw, double *__restrict__ bk,
+                             const Ctl *ctl) {
+    const int jz = blockIdx.x * blockDim.x + threadIdx.x + 1, jx = blockIdx.y * blockDim.y + threadIdx.y + 1;
+    if (jz > d.nz || jx > d.nx) return;
+    const size_t n = (size_t)64 * R, per = (size_t)d.nxp * 3 * n;
+    const float *p = acc + (size_t)(jx + d.npml - 1) * 3 * n + (jz + d.npml - z0);
+    double g = 0.0, f = 0.0, b = 0.0;
+    for (int s = 0; s < ns; ++s, p += per) {
+        g += (double)p[0];
+        f += (double)p[n];
+        b += (double)p[2 * n];
+    }
+    const size_t k = iidx(d, jz, jx);
+    const double bad = ctl->err ? __longlong_as_double(0x7ff8000000000000ll) : 0.0;
+    grad[k] = -2.0 * g / (double)vp[k] + bad;
+    fw[k] = f + bad;
+    bk[k] = b + bad;
+}
+
+// Adjoint sources into slot order: out[s][t][n] = in[s][map[s][n]][t] (map -1: nothing).
+__global__ void k_res_adjsrc(int nt, int ngmax, const int *__restrict__ map, const float *__restrict__ in,
+                             float *__restrict__ out) {
+    __shared__ float tile[32][33];
+    const int s = blockIdx.z, n0 = blockIdx.x * 32, t0 = blockIdx.y * 32;
+    for (int k = threadIdx.y; k < 32; k += 8) {
+        const int n = n0 + k, t = t0 + threadIdx.x;
+        const int m = n < ngmax ? map[(size_t)s * ngmax + n] : -1;
+        if (m >= 0 && t < nt) tile[k][threadIdx.x] = in[((size_t)s * ngmax + m) * nt + t];
+    }
+    __syncthreads();
+    const int n = n0 + threadIdx.x;
+    const int m = n < ngmax ? map[(size_t)s * ngmax + n] : -1;
+    for (int k = threadIdx.y; k < 32; k += 8) {
+        const int t = t0 + k;
+        if (m >= 0 && t < nt) out[((size_t)s * nt + t) * ngmax + n] = tile[threadIdx.x][k];
+    }
+}
+
 
 // Coefficients of a configuration, column by column (1 .. ncol, past nxp zero):
 // {pressure update's, velocity updates', 1-kappa_p, 1-kappa_u, 1-kappa_w}[64 R rows from z0].

@@ -68,6 +68,19 @@ struct ResidentState {
     int *f_rbase = nullptr;      // [ns][P]
     int *f_map = nullptr;        // [ns][ngmax] receiver -> slot of seis_t
     int f_ncol = 0;
+    // the backward's
+    bool bwd = false;
+    rk::Cfg bc{};
+    size_t b_lds = 0;
+    float *b_co = nullptr, *b_fpx = nullptr;
+    int b_ncol = 0;
+    unsigned long long b_imask = 0;
+    int b_layers = 1;
+    int *b_itab = nullptr;       // [ns][P][2][64 W]
+    int *b_ibase = nullptr;      // [ns][P]
+    int *b_imap = nullptr;       // [ns][ngmax] slot -> receiver
+    float *b_acc = nullptr;      // [ns][nxp][3][64 R]
+    size_t b_msg = 0;
     rk::u64 *msg = nullptr;      // exchange words (shared by the plan's resident launches)
     size_t f_msg = 0;
     rk::Ctl *ctl = nullptr;
@@ -469,6 +482,8 @@ static int plain_adjoint(swit_plan *pl, const float *src, hipStream_t st) {
 
 static int resident_now(bool built, int use, hipStream_t st, bool *yes);
 static int resident_forward(swit_plan *pl, const float *src, float *seis, int save, hipStream_t st);
+static int resident_adjoint(swit_plan *pl, const float *src, const float *adjsrc, double *grad, double *fw, double *bk,
+                            hipStream_t st);
 
 // ---- public jobs -------------------------------------------------------------------
 
@@ -510,6 +525,9 @@ extern "C" int swit_adjoint(swit_plan *pl, const float *src, const float *adjsrc
     if (!pl->strips_valid)
         return set_err(SWIT_ESTATE, "no saved strips: run swit_forward with save_strips=1 first");
     const Dims &d = pl->d;
+    bool resident = false;
+    TRY(resident_now(pl->res.bwd, pl->res.use_bwd, stream, &resident));
+    if (resident) return resident_adjoint(pl, src, adjsrc, grad, illum_forw, illum_back, stream);
     // [ns][ngmax][nt] -> [ns][nt][ngmax]
     hipLaunchKernelGGL(k_transpose, dim3(cdiv(d.nt, 32), cdiv(d.ngmax, 32), pl->ns), dim3(32, 8), 0,
                        stream, d.ngmax, d.nt, adjsrc, pl->sadj_t);
@@ -1232,11 +1250,11 @@ struct FwdKernel {
 // above at two (256 registers, workgroups of at most 8 waves)
 #define SWIT_FWD(R, C) {R, C, {rk::k_fwd_resident<R, C, false>, rk::k_fwd_resident<R, C, true>}}
 const FwdKernel kFwdKernels[] = {
-    SWIT_FWD(2, 6), SWIT_FWD(2, 9), SWIT_FWD(2, 14), SWIT_FWD(2, 20), SWIT_FWD(2, 24),
-    SWIT_FWD(3, 6), SWIT_FWD(3, 9), SWIT_FWD(3, 12), SWIT_FWD(3, 14), SWIT_FWD(3, 16),
-    SWIT_FWD(4, 6), SWIT_FWD(4, 8), SWIT_FWD(4, 10), SWIT_FWD(4, 12),
-    SWIT_FWD(5, 6), SWIT_FWD(5, 8), SWIT_FWD(5, 10),
-    SWIT_FWD(6, 6), SWIT_FWD(6, 8), SWIT_FWD(7, 7), SWIT_FWD(8, 6),
+    SWIT_FWD(2, 3), SWIT_FWD(2, 6), SWIT_FWD(2, 9), SWIT_FWD(2, 14), SWIT_FWD(2, 20), SWIT_FWD(2, 24),
+    SWIT_FWD(3, 3), SWIT_FWD(3, 6), SWIT_FWD(3, 9), SWIT_FWD(3, 12), SWIT_FWD(3, 14), SWIT_FWD(3, 16),
+    SWIT_FWD(4, 3), SWIT_FWD(4, 5), SWIT_FWD(4, 8), SWIT_FWD(4, 10), SWIT_FWD(4, 12),
+    SWIT_FWD(5, 3), SWIT_FWD(5, 6), SWIT_FWD(5, 8),
+    SWIT_FWD(6, 3), SWIT_FWD(6, 6), SWIT_FWD(7, 3), SWIT_FWD(7, 5), SWIT_FWD(8, 3), SWIT_FWD(8, 4),
 };
 #undef SWIT_FWD
 constexpr int kCuLds = 160 * 1024;
@@ -1248,13 +1266,13 @@ size_t fwd_lds_bytes(const rk::Cfg &c, int NS) {
 
 // Estimated time of one resident step (us): the vector issue of the waves that share a
 // compute unit, with what their latency adds, and the exchange and the barriers.  Fitted to
-// the forward on grids of 201x81 to 481x141 (2.4 GHz): with one wave per SIMD 1.34 times the
-// issue time, with two or more 0.93 (36 operations are counted per cell, some waves have
-// fewer), plus 2.0 us with an exchange (one shot, R = 2, C = 6, W = 3: 2.97 measured, 2.96
-// estimated; 49 shots, R = 3, C = 16, W = 8: 7.37 and 7.36).
+// the forward on grids of 201x81 to 481x141 (2.4 GHz, 36 operations per cell): with one wave
+// per SIMD 1.34 times the issue time, with two or more 0.93, plus 1.45 us with an exchange
+// (one shot, R = 2, C = 3, W = 4: 1.99 measured, 1.93 estimated; C = 9: 2.95 and 2.90;
+// 49 shots, R = 3, C = 16, W = 8: 6.76 and 6.81).
 double resident_step_us(int waves_on_cu, double cell_ops, bool exchange) {
     const double issue = cdiv(waves_on_cu, 4) * cell_ops * 4 / 2400.0;
-    return (waves_on_cu > 4 ? 0.93 : 1.34) * issue + (exchange ? 2.0 : 0.9);
+    return (waves_on_cu > 4 ? 0.93 : 1.34) * issue + (exchange ? 1.45 : 0.9);
 }
 
 // Windows of the forward for ns shots on ncu compute units: of every (columns per wave,
@@ -1274,8 +1292,8 @@ bool choose_fwd(const Dims &d, int ns, int ncu, int NS, rk::Cfg *best) {
             c.z0 = d.fs - 1;
             const int cols = W * c.C;
             c.P = d.nxp <= cols ? 1 : cols > 2 * rk::kH ? cdiv(d.nxp - 2 * rk::kH, cols - 2 * rk::kH) : 0;
-            // a window's first and last six columns in one wave each, three own columns at least
-            if (c.P < 1 || (c.P > 1 && (c.C < 2 * rk::kH || cols < 3 * rk::kH))) continue;
+            // halo columns in one wave, three own columns at least
+            if (c.P < 1 || (c.P > 1 && (c.C < rk::kH || cols < 3 * rk::kH))) continue;
             const size_t lds = fwd_lds_bytes(c, NS);
             if (lds + 1024 > kCuLds) continue;
             const int per_cu = std::min(cu_waves / W, (int)(kCuLds / (lds + 1024)));
@@ -1373,14 +1391,182 @@ static void resident_receivers(const swit_plan *pl, const rk::Cfg &c, unsigned l
     }
 }
 
+
+// ---- the backward ----
+
+namespace {
+
+struct BwdKernel {
+    int R, C;
+    void (*fn)(rk::BwdArgs);
+};
+// 6 R C floats of state per thread of 256 registers
+#define SWIT_BWD(R, C) {R, C, rk::k_bwd_resident<R, C>}
+const BwdKernel kBwdKernels[] = {
+    SWIT_BWD(2, 3), SWIT_BWD(2, 6), SWIT_BWD(2, 12), SWIT_BWD(3, 3), SWIT_BWD(3, 6), SWIT_BWD(3, 8),
+    SWIT_BWD(4, 3), SWIT_BWD(4, 5), SWIT_BWD(4, 6), SWIT_BWD(5, 3), SWIT_BWD(5, 4), SWIT_BWD(6, 3), SWIT_BWD(6, 4),
+    SWIT_BWD(7, 3), SWIT_BWD(8, 3),
+};
+#undef SWIT_BWD
+
+size_t bwd_lds_bytes(const rk::Cfg &c, int NI, int layers) {
+    return sizeof(float) * (rk::bwd_edge_floats(c.W, c.R) + 2 * (size_t)rk::bwd_set_floats(c.W, c.C, c.R, NI, layers));
+}
+
+// Rows of the adjoint that a step changes or reads past its tile: 2 .. nzp-2.  z0 <= 2 puts
+// row fs - 1 on a lane's first row.
+void bwd_rows(const Dims &d, int R, int *z0, int *need) {
+    *z0 = 2 - (((2 - (d.fs - 1)) % R) + R) % R;
+    *need = d.nzp - 2 - *z0 + 1;
+}
+
+bool choose_bwd(const Dims &d, int ns, int ncu, int NI, int layers, rk::Cfg *best) {
+    double best_t = 1e30;
+    int R = 2, z0 = 0, need = 0;
+    for (;; ++R) {
+        bwd_rows(d, R, &z0, &need);
+        if (need <= 64 * R) break;
+        if (R > 8) return false;
+    }
+    for (const BwdKernel &kn : kBwdKernels) {
+        if (kn.R != R) continue;
+        for (int W = 1; W <= 8; ++W) {
+            rk::Cfg c{};
+            c.R = R;
+            c.C = kn.C;
+            c.W = W;
+            c.z0 = z0;
+            const int cols = W * c.C;
+            c.P = d.nxp <= cols ? 1 : cols > 2 * rk::kH ? cdiv(d.nxp - 2 * rk::kH, cols - 2 * rk::kH) : 0;
+            // halo columns in one wave, three own columns at least
+            if (c.P < 1 || (c.P > 1 && (c.C < rk::kH || cols < 3 * rk::kH))) continue;
+            const size_t lds = bwd_lds_bytes(c, NI, layers);
+            if (lds + 1024 > kCuLds) continue;
+            const int per_cu = std::min(8 / W, (int)(kCuLds / (lds + 1024)));
+            if (c.P > per_cu * ncu) continue;
+            const int rounds = cdiv(ns, std::min(ns, per_cu * ncu / c.P));
+            c.G = cdiv(ns, rounds);
+            const double t = rounds * resident_step_us(W * cdiv(c.G * c.P, ncu), 80.0 * c.C * R, c.P > 1);
+            if (t < best_t) {
+                best_t = t;
+                *best = c;
+            }
+        }
+    }
+    return best_t < 1e30;
+}
+
+const BwdKernel *find_bwd(int R, int C) {
+    for (const BwdKernel &k : kBwdKernels)
+        if (k.R == R && k.C == C) return &k;
+    return nullptr;
+}
+
+}  // namespace
+
+// The backward's configuration and adjoint-source tables.  Receivers go through an LDS stage
+// of the lanes that hold injection cells (up to 8, up to two receivers in a cell and two per
+// thread of a window); other acquisitions keep the step kernels.
+static int resident_init_bwd(swit_plan *pl, int ncu) {
+    ResidentState &rs = pl->res;
+    const Dims &d = pl->d;
+    rs.bwd = false;
+    if (pl->flags & SWIT_PLAN_NO_STRIPS) return SWIT_OK;
+    rk::Cfg c{};
+    int layers = 1;
+    for (int s = 0; s < pl->ns && layers <= 2; ++s) {
+        std::vector<int> q(pl->rec_cells_inj.begin() + (size_t)s * d.ngmax,
+                           pl->rec_cells_inj.begin() + (size_t)s * d.ngmax + pl->geo_h[s].ng);
+        std::sort(q.begin(), q.end());
+        for (size_t k = 0, m = 1; k + 1 < q.size(); ++k) {
+            m = q[k] == q[k + 1] ? m + 1 : 1;
+            layers = std::max(layers, (int)m);
+        }
+    }
+    if (layers > 2 || !choose_bwd(d, pl->ns, ncu, 8, layers, &c)) return SWIT_OK;
+    unsigned long long mask = 0;
+    for (int s = 0; s < pl->ns; ++s)
+        for (int r = 0; r < pl->geo_h[s].ng; ++r)
+            mask |= 1ull << ((pl->rec_cells_inj[(size_t)s * d.ngmax + r] % d.ld + 1 - c.z0) / c.R);
+    const int NI = __builtin_popcountll(mask);
+    if (NI > 8) return SWIT_OK;
+    const int T = c.W * 64, WC = c.W * c.C;
+    std::vector<int> itab((size_t)pl->ns * c.P * 2 * T, -1), ibase((size_t)pl->ns * c.P, 0),
+        imap((size_t)pl->ns * d.ngmax, -1);
+    struct Item {
+        int j, col, row, r;
+    };
+    std::vector<Item> item;
+    for (int s = 0; s < pl->ns; ++s) {
+        item.clear();
+        for (int r = 0; r < pl->geo_h[s].ng; ++r) {
+            const int o = pl->rec_cells_inj[(size_t)s * d.ngmax + r];
+            const int z = o % d.ld + 1, x = o / d.ld + 1;
+            int j = 0;
+            while (x > rk::window_oe(c.W, c.C, j, c.P, d.nxp)) ++j;
+            item.push_back(Item{j, x - rk::window_x(c.W, c.C, j), z - c.z0, r});
+        }
+        std::stable_sort(item.begin(), item.end(), [](const Item &x, const Item &y) {
+            return x.j != y.j ? x.j < y.j : x.col != y.col ? x.col < y.col : x.row < y.row;
+        });
+        int first = 0, layer = 0;
+        for (size_t k = 0; k < item.size(); ++k) {
+            const Item &q = item[k];
+            const bool same = k && item[k - 1].j == q.j && item[k - 1].col == q.col && item[k - 1].row == q.row;
+            layer = same ? layer + 1 : 0;
+            if (!k || item[k - 1].j != q.j) {
+                first = (int)k;
+                ibase[(size_t)s * c.P + q.j] = first;
+            }
+            const int n = (int)k - first;
+            if (n >= 2 * T) return SWIT_OK;
+            const int slot = __builtin_popcountll(mask & ((1ull << (q.row / c.R)) - 1));
+            itab[((size_t)s * c.P + q.j) * 2 * T + n] = ((layer * (NI + 1) + slot) * WC + q.col) * c.R + q.row % c.R;
+            imap[(size_t)s * d.ngmax + k] = q.r;
+        }
+    }
+    rs.bc = c;
+    rs.b_imask = mask;
+    rs.b_layers = layers;
+    rs.b_lds = bwd_lds_bytes(c, NI, layers);
+    HIP_TRY(hipFuncSetAttribute((const void *)find_bwd(c.R, c.C)->fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)rs.b_lds));
+    rs.b_ncol = d.nxp + WC;
+    const size_t col = (size_t)64 * c.R;
+    TRY(pl->alloc(&rs.b_co, (rs.b_ncol + 1) * 5 * col));
+    TRY(pl->alloc(&rs.b_fpx, rs.b_ncol + 1));
+    TRY(pl->alloc(&rs.b_itab, itab.size()));
+    TRY(pl->alloc(&rs.b_ibase, ibase.size()));
+    TRY(pl->alloc(&rs.b_imap, imap.size()));
+    TRY(pl->alloc(&rs.b_acc, (size_t)pl->ns * d.nxp * 3 * col));
+    HIP_TRY(hipMemcpy(rs.b_itab, itab.data(), sizeof(int) * itab.size(), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(rs.b_ibase, ibase.data(), sizeof(int) * ibase.size(), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(rs.b_imap, imap.data(), sizeof(int) * imap.size(), hipMemcpyHostToDevice));
+    rs.b_msg = c.P > 1 ? (size_t)c.G * c.P * 8 * rk::kH * c.R * 64 : 0;
+    rs.bwd = true;
+    return SWIT_OK;
+}
+
+static int resident_init_fwd(swit_plan *pl);
+
 static int resident_init(swit_plan *pl) {
     ResidentState &rs = pl->res;
     const Dims &d = pl->d;
     int dev = 0, ncu = 0;
     HIP_TRY(hipGetDevice(&dev));
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    TRY(resident_init_bwd(pl, ncu));
     rs.fwd = choose_fwd(d, pl->ns, ncu, 8, &rs.fc);
-    if (!rs.fwd) return SWIT_OK;
+    if (rs.fwd) TRY(resident_init_fwd(pl));
+    if (!rs.fwd && !rs.bwd) return SWIT_OK;
+    TRY(pl->alloc(&rs.msg, std::max(rs.f_msg, rs.b_msg)));
+    TRY(pl->alloc(&rs.ctl, 1));
+    return SWIT_OK;
+}
+
+static int resident_init_fwd(swit_plan *pl) {
+    ResidentState &rs = pl->res;
+    const Dims &d = pl->d;
     const rk::Cfg &c = rs.fc;
     bool direct = false;
     rs.f_pmask = resident_stage_lanes(pl, c.R, c.z0, &direct);
@@ -1405,9 +1591,7 @@ static int resident_init(swit_plan *pl) {
     TRY(pl->alloc(&rs.f_map, map.size()));
     HIP_TRY(hipMemcpy(rs.f_rbase, rbase.data(), sizeof(int) * rbase.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(rs.f_map, map.data(), sizeof(int) * map.size(), hipMemcpyHostToDevice));
-    rs.f_msg = c.P > 1 ? (size_t)c.G * c.P * 4 * rk::kFromRight * c.R * 64 : 0;
-    TRY(pl->alloc(&rs.msg, rs.f_msg));
-    TRY(pl->alloc(&rs.ctl, 1));
+    rs.f_msg = c.P > 1 ? (size_t)c.G * c.P * 4 * rk::kH * c.R * 64 : 0;
     return SWIT_OK;
 }
 
@@ -1418,6 +1602,11 @@ static int resident_set_model(swit_plan *pl, hipStream_t st) {
     if (rs.fwd) {
         hipLaunchKernelGGL(rk::k_res_setup, dim3(rs.fc.R, rs.f_ncol + 1), dim3(64), 0, st, d, rs.fc.R, rs.fc.z0,
                            rs.f_ncol, d.fs + 1, d.fs, 0, bs.KB, bs.CP, bs.CV, rs.f_co, rs.f_fpx);
+        LAUNCH_CHECK();
+    }
+    if (rs.bwd) {
+        hipLaunchKernelGGL(rk::k_res_setup, dim3(rs.bc.R, rs.b_ncol + 1), dim3(64), 0, st, d, rs.bc.R, rs.bc.z0,
+                           rs.b_ncol, 3, 2, 1, bs.KB, bs.CP, bs.CV, rs.b_co, rs.b_fpx);
         LAUNCH_CHECK();
     }
     return SWIT_OK;
@@ -1525,6 +1714,64 @@ static int resident_forward(swit_plan *pl, const float *src, float *seis, int sa
     return resident_traces(pl, seis, st);
 }
 
+// The reverse loop of every shot in one launch (adj: adjoint sources in slot order).
+static int resident_backward_steps(swit_plan *pl, const float *src, const float *adj, hipStream_t st) {
+    ResidentState &rs = pl->res;
+    BatchedState &bs = pl->bat;
+    const Dims &d = pl->d;
+    TRY(resident_begin(pl, rs.b_msg, true, st));
+    TRY(fill(rs.b_acc, (size_t)pl->ns * d.nxp * 3 * 64 * rs.bc.R, st));
+    rk::BwdArgs a{};
+    a.d = d;
+    a.c = rs.bc;
+    a.s0 = 0;
+    a.ns = pl->ns;
+    a.co = rs.b_co;
+    a.ncol = rs.b_ncol;
+    a.fpx = rs.b_fpx;
+    a.geo = pl->geo;
+    a.src = src;
+    a.strips = bs.strip_mode == 0 ? static_cast<const void *>(pl->strips) : static_cast<const void *>(bs.strips16);
+    a.mode = bs.strip_mode;
+    a.smax = bs.smax;
+    a.end = bs.end;
+    a.adj = adj;
+    a.itab = rs.b_itab;
+    a.ibase = rs.b_ibase;
+    a.imask = rs.b_imask;
+    a.layers = rs.b_layers;
+    a.acc = rs.b_acc;
+    a.msg = rs.msg;
+    a.ctl = rs.ctl;
+    hipLaunchKernelGGL(find_bwd(rs.bc.R, rs.bc.C)->fn, dim3(rs.bc.G * rs.bc.P), dim3(64 * rs.bc.W), rs.b_lds, st, a);
+    LAUNCH_CHECK();
+    return SWIT_OK;
+}
+
+// The whole adjoint job, outputs straight into the caller's arrays.
+static int resident_adjoint(swit_plan *pl, const float *src, const float *adjsrc, double *grad, double *fw, double *bk,
+                            hipStream_t st) {
+    ResidentState &rs = pl->res;
+    BatchedState &bs = pl->bat;
+    const Dims &d = pl->d;
+    BatchedState::Timed t{1, (long long)d.nt - 1, nullptr, nullptr};
+    hipLaunchKernelGGL(rk::k_res_adjsrc, dim3(cdiv(d.ngmax, 32), cdiv(d.nt, 32), pl->ns), dim3(32, 8), 0, st, d.nt,
+                       d.ngmax, rs.b_imap, adjsrc, pl->sadj_t);
+    LAUNCH_CHECK();
+    if (bs.profile) {
+        TRY(pool_event(bs, &t.e0));
+        TRY(pool_event(bs, &t.e1));
+        bs.pending.push_back(t);
+        HIP_TRY(hipEventRecord(t.e0, st));
+    }
+    TRY(resident_backward_steps(pl, src, pl->sadj_t, st));
+    if (bs.profile) HIP_TRY(hipEventRecord(t.e1, st));
+    hipLaunchKernelGGL(rk::k_res_reduce, dim3(cdiv(d.nz, 64), cdiv(d.nx, 4)), dim3(64, 4), 0, st, d, pl->ns, rs.bc.R,
+                       rs.bc.z0, pl->c_int, rs.b_acc, grad, fw, bk, rs.ctl);
+    LAUNCH_CHECK();
+    return SWIT_OK;
+}
+
 // The resident loops against the step kernels' best times us[0] (forward), us[1] (backward)
 // per time step: each is used where it is faster, and us gets its time.  A job of up to 200
 // steps is timed (best of three).
@@ -1532,14 +1779,14 @@ static int resident_autotune(swit_plan *pl, double *us, hipStream_t st) {
     ResidentState &rs = pl->res;
     BatchedState &bs = pl->bat;
     const Dims &d = pl->d;
-    if (!rs.fwd) return SWIT_OK;
+    if (!rs.fwd && !rs.bwd) return SWIT_OK;
     hipEvent_t e0, e1;
     TRY(pool_event(bs, &e0));
     TRY(pool_event(bs, &e1));
     const int it1 = std::min(d.nt, 201);
     const int save = (pl->flags & SWIT_PLAN_NO_STRIPS) ? 0 : 1;
     double best = 1e30;
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < 4 && rs.fwd; ++k) {
         HIP_TRY(hipEventRecord(e0, st));
         TRY(resident_forward_steps(pl, 2, it1, bs.src, save, DSave{nullptr, 0, 0}, nullptr, nullptr, nullptr, true, st));
         HIP_TRY(hipEventRecord(e1, st));
@@ -1550,6 +1797,21 @@ static int resident_autotune(swit_plan *pl, double *us, hipStream_t st) {
     }
     rs.use_fwd = best < us[0];
     if (rs.use_fwd) us[0] = best;
+    if (rs.bwd) {
+        best = 1e30;
+        // the loop always runs from nt to 2: one job, its adjoint sources whatever is there
+        for (int k = 0; k < 3; ++k) {
+            HIP_TRY(hipEventRecord(e0, st));
+            TRY(resident_backward_steps(pl, bs.src, pl->sadj_t, st));
+            HIP_TRY(hipEventRecord(e1, st));
+            HIP_TRY(hipEventSynchronize(e1));
+            float ms = 0.0f;
+            HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
+            if (k) best = std::min(best, 1000.0 * ms / (d.nt - 1));
+        }
+        rs.use_bwd = best < us[1];
+        if (rs.use_bwd) us[1] = best;
+    }
     bs.ev_pool.push_back(e0);
     bs.ev_pool.push_back(e1);
     return SWIT_OK;
