@@ -218,11 +218,12 @@ int swit_adjoint_exact(swit_plan *plan, const float *gseis, double *grad, hipStr
 int swit_misfit(int kind, int ntraces, int nt, float dt, const float *obs, const float *syn, float *adj,
                 double *work, double *misfit, hipStream_t stream);
 
-/* ---- plan groups: uneven grids in one launch ------------------------------------
+/* ---- plan groups: uneven grids as one job -----------------------------------------
  * A group runs several batched plans (different grids, shot counts, record lengths,
- * strip precisions) as one job: each group forward / adjoint is a single hipGraph
- * launch holding every plan's whole time loop on its own branch, so plans with short
- * records fill the GPU while long ones finish.  No counterpart in the reference (one
+ * strip precisions) as one job.  Where every plan takes the resident time loops they run
+ * one after the other, each filling the chip; otherwise each group forward / adjoint is a
+ * single hipGraph launch holding every plan's step kernels on its own branch, so plans with
+ * short records fill the GPU while long ones finish.  No counterpart in the reference (one
  * fd2dmpi job per grid, toolbox/solver.py:24-92); results are those of
  * swit_forward / swit_adjoint on each plan alone.  The arrays below hold one entry
  * per plan, in the order of `plans`; each entry is what the single-plan call takes.
@@ -237,13 +238,11 @@ int swit_group_adjoint(swit_group *group, const float *const *src, const float *
                        hipStream_t stream);
 int swit_group_destroy(swit_group *group);
 
-/* A whole gradient of every plan in one graph launch: each plan's branch runs the
- * strip-saving forward (seismograms to seis), the misfit and adjoint source `kind`
+/* A whole gradient of every plan in one call: each plan runs the strip-saving forward (seismograms to seis), the misfit and adjoint source `kind`
  * (SWIT_MISFIT_*) against obs, exactly as swit_misfit computes them (adjoint source to
  * adj, per-trace misfits to work, their sum to misfit), and the adjoint (grad,
  * illum_forw, illum_back).  Each plan's results equal swit_forward, swit_misfit and
- * swit_adjoint run one after the other.  The branches overlap, so one plan's adjoint
- * runs beside another's forward.  Per plan: obs, seis, adj [ns][ngmax][nt]; work
+ * swit_adjoint run one after the other.  Per plan: obs, seis, adj [ns][ngmax][nt]; work
  * [ns*ngmax] doubles; misfit one double; grad, illum_* [nx][nz] doubles.  No counterpart in the
  * reference (toolbox/inversion.py:48-60 runs these steps one after the other, through files). */
 int swit_group_gradient(swit_group *group, int kind, const float *const *src, const float *const *obs,

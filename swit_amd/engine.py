@@ -234,8 +234,10 @@ class Plan:
 
 class PlanGroup:
     """Several batched plans (uneven grids, shot counts, record lengths) run as one job:
-    each forward / adjoint is a single hipGraph launch with every plan's time loop on
-    its own branch.  Results equal those of each plan run alone."""
+    where every plan takes the resident time loops they run one after the other, each
+    filling the chip, otherwise each forward / adjoint is a single hipGraph launch with
+    every plan's step kernels on a branch of its own.  Results equal those of each plan
+    run alone."""
 
     def __init__(self, plans):
         self.plans = list(plans)
@@ -276,7 +278,7 @@ class PlanGroup:
         return [tuple(o) for o in outs]
 
     def gradient(self, srcs, obs, kind):
-        """Every plan's whole gradient in one graph launch (swit_group_gradient): forward
+        """Every plan's whole gradient in one call (swit_group_gradient): forward
         with strips, misfit `kind` and adjoint source against obs[i], adjoint.  Returns
         (misfits, seismograms, (grad, illum_forw, illum_back) per plan); each plan's
         results equal forward, engine.misfit and adjoint run one after the other.  The
