@@ -1214,6 +1214,347 @@ __global__ void k_res_adjsrc(int nt, int ngmax, const int *__restrict__ map, con
 }
 
 
+struct ExArgs {
+    Dims d;
+    Cfg c;
+    int ns;
+    int it0, it1;               // reverse steps it1 .. it0
+    const float *co;            // the forward's coefficients (k_res_setup)
+    int ncol;
+    const float *fpx;
+    const float *g;             // [ns][nt][ngmax] dJ/dseis
+    const int2 *itab;           // [ns][P][2][64 W] {place in the injection stage, receiver}, -1 none
+    unsigned long long imask;   // lanes of the injection stage
+    int layers;                 // most receivers of one cell (1 or 2)
+    DSave hist;                 // divergence history
+    const float *in;            // null (zero state) or [ns][3][nxp][ld]: adjoint fields after step it1 + 1
+    float *out;                 // null or [ns][3][nxp][ld]
+    float *gk;                  // [ns][nxp][ld] K-gradient so far, zero outside the p region
+    int add;                    // 0: it is zero
+    u64 *msg;                   // as the forward's
+    Ctl *ctl;
+};
+
+// LDS of the exact reverse loop: the waves' edge columns of q and r, two injection stages.
+__host__ __device__ inline int ex_set_floats(int W, int C, int R, int NI, int layers) { return layers * NI * W * C * R; }
+
+// Reverse steps it1 .. it0 of the exact adjoint (the transpose of the forward step, written
+// out in fd_exact.hip) of every shot, the three adjoint fields, the K-gradient, K and B in
+// registers.  qu = B lu takes the place of the forward's u and r = K lp that of its p: lp
+// needs qu at x-2..x+1 and lu needs r at x-1..x+2, so fresh lu in the halo after every step
+// keeps the rest that is needed right, receivers in the halo included.
+// Bound by vector issue, 34 operations per cell and step and about as many again for shifts,
+// the divergence history (one 4-byte load per cell and step, in flight through the first
+// part) and the exchange.  Forward and reverse of 161x61x1500, 8 shots, whole history: 31.2 ms
+// by the step kernels (a launch each per step), 9.2 ms here; of 301x101, 21 shots, with
+// checkpoints (an additional forward): 81.8 and 19.0 ms.
+template <int R, int C>
+__global__ __launch_bounds__(512) void k_ex_resident(ExArgs a) {
+    extern __shared__ float lds[];
+    __shared__ int sh_ticket;
+    constexpr int kCol = 64 * R * 4;
+    const int W = a.c.W, P = a.c.P, T = W * 64;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (threadIdx.x == 0) sh_ticket = (int)atomicAdd(&a.ctl->ticket, 1u);
+    __syncthreads();
+    const int t = __builtin_amdgcn_readfirstlane(sh_ticket);
+    const int grp = __builtin_amdgcn_readfirstlane(t / P), j = __builtin_amdgcn_readfirstlane(t % P);
+    const int NI = __popcll(a.imask);
+    float *eQ = lds;                                     // [W][3][R][64]: first, last but one, last column of qu
+    float *eR = eQ + W * 3 * R * 64;                     // [W][3][R][64]: first, second, last column of r
+    float *sets = eR + W * 3 * R * 64;
+    const int set_floats = ex_set_floats(W, C, R, NI, a.layers), layer_floats = NI * W * C * R;
+    const int x0w = window_x(W, C, j) + wave * C;
+    const bool has_l = j > 0, has_r = j + 1 < P;
+    const bool edge = (has_l && wave <= (2 * kH - 1) / C) || (has_r && wave >= W - 1 - (2 * kH - 1) / C);
+    const unsigned voff0 = lane * R * 4;
+    const bool mirror = a.d.free_surface == 1 && lane == 0;
+    const bool mirror1 = a.d.free_surface == 1 && lane == 1;
+    const bool wave_pml = x0w <= a.d.npml || x0w + C - 1 >= a.d.npml + a.d.nx;
+    const __amdgpu_buffer_rsrc_t co = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(a.co), 0, (int)((unsigned)(a.ncol + 1) * 5u * kCol), 0x00027000);
+    const bool i_lane = (a.imask >> lane) & 1;
+    const int i_off = (__popcll(a.imask & ((1ull << lane) - 1)) * W + wave) * (C * R);
+    unsigned tag = 0;
+    bool dead = false;
+    float K[C][R], B[C][R], fpz[R];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        buffer_rows<R>(co, voff0, (x0w + c) * (5 * kCol), K[c]);
+        buffer_rows<R>(co, voff0, (x0w + c) * (5 * kCol) + kCol, B[c]);
+    }
+    buffer_rows<R>(co, voff0, 2 * kCol, fpz);
+
+    for (int s = grp; s < a.ns; s += a.c.G) {
+        float lp[C][R], lu[C][R], lw[C][R], gk[C][R];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int r = 0; r < R; ++r) lp[c][r] = lu[c][r] = lw[c][r] = gk[c][r] = 0.0f;
+        if (a.in || a.add) {
+            const ArgPtr<ExArgs> k = fresh_args<ExArgs>();
+            int x0 = x0w;
+            unsigned voff = voff0;
+            opaque_s(x0);
+            opaque_v(voff);
+            const int zr = k->c.z0 + (int)(voff >> 2), ld = k->d.ld, np = k->d.nxp * ld;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                if (x0 + c > k->d.nxp) continue;
+                const float *f = k->in + (size_t)s * 3 * np + (size_t)(x0 + c - 1) * ld;
+                const float *g = k->gk + (size_t)s * np + (size_t)(x0 + c - 1) * ld;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    if (zr + r > k->d.nzp) continue;
+                    const unsigned o = zr + r - 1;
+                    if (k->in) {
+                        lp[c][r] = f[o];
+                        lu[c][r] = f[np + o];
+                        lw[c][r] = f[2 * np + o];
+                    }
+                    if (k->add) gk[c][r] = g[o];
+                }
+            }
+        }
+        const int2 *tab = a.itab + ((size_t)s * P + j) * 2 * T + threadIdx.x;
+        const int2 i0 = tab[0], i1 = tab[T];
+        for (int n = threadIdx.x; n < 2 * set_floats; n += T) sets[n] = 0.0f;
+        // qu of the edge columns for the next step
+        auto put_q = [&]() {
+            float *e = eQ + (size_t)wave * 3 * R * 64 + lane;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                e[r * 64] = B[0][r] * lu[0][r];
+                e[(R + r) * 64] = B[C - 2][r] * lu[C - 2][r];
+                e[(2 * R + r) * 64] = B[C - 1][r] * lu[C - 1][r];
+            }
+        };
+        __syncthreads();
+        const int ngmax = a.d.ngmax;
+        const float *grow = a.g + ((size_t)s * a.d.nt + (a.it1 - 1)) * ngmax;
+        {
+            float *f = sets + (a.it1 & 1) * set_floats;
+            if (i0.x >= 0) f[i0.x] = grow[i0.y];
+            if (i1.x >= 0) f[i1.x] = grow[i1.y];
+        }
+        put_q();
+        __syncthreads();
+        const int it0 = a.it0;
+        for (int it = a.it1; it >= it0; --it) {
+            int x0 = x0w;
+            unsigned voff = voff0;
+            opaque_s(x0);
+            opaque_v(voff);
+            // D(it) of the window's columns (past the grid: the last column's, for cells that
+            // are never stored) and the next step's injection
+            float D[C][R];
+            {
+                const ArgPtr<ExArgs> k = fresh_args<ExArgs>();
+                const int ld = k->d.ld, nxp = k->d.nxp, np = nxp * ld;
+                const __amdgpu_buffer_rsrc_t h = __builtin_amdgcn_make_buffer_rsrc(
+                    k->hist.p + ((size_t)s * k->hist.slots + (it - 1 - k->hist.base)) * np, 0, np * 4, 0x00027000);
+                const unsigned zo = voff + (k->c.z0 - 1) * 4;
+#pragma unroll
+                for (int c = 0; c < C; ++c) buffer_rows<R>(h, zo, (min(x0 + c, nxp) - 1) * ld * 4, D[c]);
+            }
+            grow -= ngmax;
+            float gn0 = 0.0f, gn1 = 0.0f;
+            if (it > it0) {
+                if (i0.x >= 0) gn0 = grow[i0.y];
+                if (i1.x >= 0) gn1 = grow[i1.y];
+            }
+            // ---- lp += g at the receivers, in receiver order ----
+            if (i_lane) {
+                const float *q = sets + (it & 1) * set_floats + i_off;
+                for (int l = a.layers; l > 0; --l, q += layer_floats) {
+#pragma unroll
+                    for (int c = 0; c < C; ++c)
+#pragma unroll
+                        for (int r = 0; r < R; ++r) lp[c][r] = lp[c][r] + q[c * R + r];
+                }
+            }
+            // ---- lp -= Gx^T qu + Gz^T qw; gK -= lp D; qu of the columns x0-2, x0-1, x0+C ----
+            {
+                float ql2[R], ql1[R], qr1[R], q[C][R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float *e = eQ + lane;
+                    ql2[r] = wave > 0 ? e[(((wave - 1) * 3 + 1) * R + r) * 64] : 0.0f;
+                    ql1[r] = wave > 0 ? e[(((wave - 1) * 3 + 2) * R + r) * 64] : 0.0f;
+                    qr1[r] = wave + 1 < W ? e[((wave + 1) * 3 * R + r) * 64] : 0.0f;
+                    q[0][r] = B[0][r] * lu[0][r];
+                }
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    if (c + 1 < C) {
+#pragma unroll
+                        for (int r = 0; r < R; ++r) q[c + (c + 1 < C)][r] = B[c + (c + 1 < C)][r] * lu[c + (c + 1 < C)][r];
+                    }
+                    // w mirror transposed: rows fs-1, fs are lane 0's first two
+                    const float wf = lw[c][1] + lw[c][0];
+                    lw[c][1] = mirror ? wf : lw[c][1];
+                    lw[c][0] = mirror ? 0.0f : lw[c][0];
+                    float qw[R];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) qw[r] = B[c][r] * lw[c][r];
+                    const float d1 = dn1(qw[R - 1]), d2 = dn1(qw[R - 2]), un = up1(qw[0]);
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float xm1 = c >= 1 ? q[c - (c >= 1)][r] : ql1[r];
+                        const float xm2 = c >= 2 ? q[c - (c >= 2 ? 2 : 0)][r] : c == 1 ? ql1[r] : ql2[r];
+                        const float xp1 = c + 1 < C ? q[c + (c + 1 < C)][r] : qr1[r];
+                        const float zm1 = r >= 1 ? qw[r - (r >= 1)] : d1;
+                        const float zm2 = r >= 2 ? qw[r - (r >= 2 ? 2 : 0)] : r == 1 ? d1 : d2;
+                        const float zp1 = r + 1 < R ? qw[r + (r + 1 < R)] : un;
+                        const float gx = kC1 * (xm1 - q[c][r]) + kC2 * (xm2 - xp1);
+                        const float gz = kC1 * (zm1 - qw[r]) + kC2 * (zm2 - zp1);
+                        lp[c][r] = lp[c][r] - gx - gz;
+                    }
+                    // p mirror transposed: row fs+1 (lane 1's first when R = 2) -= row fs-1
+                    if constexpr (R > 2) {
+                        const float pf = lp[c][R > 2 ? 2 : 0] - lp[c][0];
+                        lp[c][R > 2 ? 2 : 0] = mirror ? pf : lp[c][R > 2 ? 2 : 0];
+                    } else {
+                        const float pf = lp[c][0] - dn1(lp[c][0]);
+                        lp[c][0] = mirror1 ? pf : lp[c][0];
+                    }
+                    lp[c][0] = mirror ? 0.0f : lp[c][0];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        gk[c][r] = gk[c][r] - lp[c][r] * D[c][r];
+                        pin(lp[c][r]);
+                        pin(lw[c][r]);
+                        pin(gk[c][r]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // ---- r = K lp; lu -= Dx^T r, lw -= Dz^T r; lp *= fp; r of x0-1, x0+C, x0+C+1 ----
+            float cfu[2][R], cfw[2][R];
+            auto fetch_v = [&](int c) {
+                const int f = wave_pml ? (x0 + c) * (5 * kCol) : 0;
+                buffer_rows<R>(co, voff, f + 3 * kCol, cfu[c % 2]);
+                buffer_rows<R>(co, voff, f + 4 * kCol, cfw[c % 2]);
+            };
+            fetch_v(0);
+            float rc[C][R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                rc[0][r] = K[0][r] * lp[0][r];
+                rc[1][r] = K[1][r] * lp[1][r];
+            }
+            {
+                float *e = eR + (size_t)wave * 3 * R * 64 + lane;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    e[r * 64] = rc[0][r];
+                    e[(R + r) * 64] = rc[1][r];
+                    e[(2 * R + r) * 64] = K[C - 1][r] * lp[C - 1][r];
+                }
+            }
+            lds_barrier();
+            if (edge) __builtin_amdgcn_s_setprio(3);
+            {
+                const ArgPtr<float> fpx = (ArgPtr<float>)fresh_args<ExArgs>()->fpx + x0;
+                float rl1[R], rr1[R], rr2[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float *e = eR + lane;
+                    rl1[r] = wave > 0 ? e[(((wave - 1) * 3 + 2) * R + r) * 64] : 0.0f;
+                    rr1[r] = wave + 1 < W ? e[((wave + 1) * 3 * R + r) * 64] : 0.0f;
+                    rr2[r] = wave + 1 < W ? e[(((wave + 1) * 3 + 1) * R + r) * 64] : 0.0f;
+                }
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    if (c + 1 < C) fetch_v(c + 1);
+                    const float fx = fpx[c];
+                    if (c + 2 < C) {
+#pragma unroll
+                        for (int r = 0; r < R; ++r)
+                            rc[c + (c + 2 < C ? 2 : 0)][r] = K[c + (c + 2 < C ? 2 : 0)][r] * lp[c + (c + 2 < C ? 2 : 0)][r];
+                    }
+                    const float d1 = dn1(rc[c][R - 1]), un1 = up1(rc[c][0]), un2 = up1(rc[c][1]);
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float xm = c >= 1 ? rc[c - (c >= 1)][r] : rl1[r];
+                        const float xp = c + 1 < C ? rc[c + (c + 1 < C)][r] : rr1[r];
+                        const float xq = c + 2 < C ? rc[c + (c + 2 < C ? 2 : 0)][r] : c + 2 == C ? rr1[r] : rr2[r];
+                        const float zm = r >= 1 ? rc[c][r - (r >= 1)] : d1;
+                        const float zp = r + 1 < R ? rc[c][r + (r + 1 < R)] : un1;
+                        const float zq = r + 2 < R ? rc[c][r + (r + 2 < R ? 2 : 0)] : r + 2 == R ? un1 : un2;
+                        const float dx = kC1 * (rc[c][r] - xp) + kC2 * (xm - xq);
+                        const float dz = kC1 * (rc[c][r] - zp) + kC2 * (zm - zq);
+                        lu[c][r] = cfu[c % 2][r] * lu[c][r] - dx;
+                        lw[c][r] = cfw[c % 2][r] * lw[c][r] - dz;
+                        lp[c][r] = fminf(fx, fpz[r]) * lp[c][r];
+                    }
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        pin(lu[c][r]);
+                        pin(lw[c][r]);
+                        pin(lp[c][r]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // ---- exchange lu, hand out the next step's injection ----
+            const bool exch = it > it0;
+            if (exch) ++tag;
+            constexpr int kMsg = kH * R * 64;
+            u64 *box = nullptr;
+            if (edge && exch) {
+                const ArgPtr<ExArgs> k = fresh_args<ExArgs>();
+                box = k->msg + ((size_t)(grp * k->c.P + j) * 2 + (tag & 1)) * (2 * kMsg) + voff / (4 * R);
+                send_edges<R, C>(has_l, has_r, wave, W, box - 3 * kMsg, box + 4 * kMsg, tag, lu);
+            }
+            {
+                float *f = sets + ((it - 1) & 1) * set_floats;
+                if (i0.x >= 0) f[i0.x] = gn0;
+                if (i1.x >= 0) f[i1.x] = gn1;
+            }
+            if (edge && exch)
+                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, fresh_args<ExArgs>()->ctl, dead, lu);
+            if (edge) __builtin_amdgcn_s_setprio(0);
+            put_q();
+            lds_barrier();
+        }
+        // own columns out
+        {
+            const ArgPtr<ExArgs> k = fresh_args<ExArgs>();
+            int x0 = x0w;
+            unsigned voff = voff0;
+            opaque_s(x0);
+            opaque_v(voff);
+            const int nxp = k->d.nxp, nzp = k->d.nzp, ld = k->d.ld, np = nxp * ld, fs = k->d.fs;
+            const int zr = k->c.z0 + (int)(voff >> 2);
+            const int os_ = window_os(k->c.W, C, j), oe_ = window_oe(k->c.W, C, j, k->c.P, nxp);
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const int x = x0 + c;
+                if (x < os_ || x > oe_) continue;
+                float *g = k->gk + (size_t)s * np + (size_t)(x - 1) * ld;
+                const bool in_x = x >= 3 && x <= nxp - 2;
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (in_x && zr + r >= fs + 1 && zr + r <= nzp - 2) g[zr + r - 1] = gk[c][r];
+                if (k->out) {
+                    float *f = k->out + (size_t)s * 3 * np + (size_t)(x - 1) * ld;
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (zr + r <= nzp) {
+                            const unsigned o = zr + r - 1;
+                            f[o] = lp[c][r];
+                            f[np + o] = lu[c][r];
+                            f[2 * np + o] = lw[c][r];
+                        }
+                }
+            }
+        }
+        lds_barrier();               // the edges and the stages are rewritten by the next shot
+    }
+}
+
 // Coefficients of a configuration, column by column (1 .. ncol, past nxp zero):
 // {pressure update's, velocity updates', 1-kappa_p, 1-kappa_u, 1-kappa_w}[64 R rows from z0].
 // The forward's pressure coefficient is K and its velocity coefficient B, the adjoint's the

@@ -11,6 +11,7 @@
 #include <cstdlib>
 #include <mutex>
 #include <utility>
+#include <set>
 #include <vector>
 
 #include "swit_fd.h"
@@ -81,6 +82,14 @@ struct ResidentState {
     int *b_imap = nullptr;       // [ns][ngmax] slot -> receiver
     float *b_acc = nullptr;      // [ns][nxp][3][64 R]
     size_t b_msg = 0;
+    // the exact reverse loop's (coefficients: the forward's)
+    bool ex = false;
+    rk::Cfg xc{};
+    size_t x_lds = 0;
+    unsigned long long x_imask = 0;
+    int x_layers = 1;
+    int2 *x_itab = nullptr;      // [ns][P][2][64 W]
+    size_t x_msg = 0;
     rk::u64 *msg = nullptr;      // exchange words (shared by the plan's resident launches)
     size_t f_msg = 0;
     rk::Ctl *ctl = nullptr;
@@ -1470,6 +1479,123 @@ const BwdKernel *find_bwd(int R, int C) {
 
 }  // namespace
 
+namespace {
+
+struct ExKernel {
+    int R, C;
+    void (*fn)(rk::ExArgs);
+};
+#define SWIT_EX(R, C) {R, C, rk::k_ex_resident<R, C>}
+const ExKernel kExKernels[] = {
+    SWIT_EX(2, 3), SWIT_EX(2, 6), SWIT_EX(2, 9), SWIT_EX(2, 12), SWIT_EX(3, 3), SWIT_EX(3, 4), SWIT_EX(3, 5), SWIT_EX(3, 6),
+    SWIT_EX(3, 8), SWIT_EX(4, 3), SWIT_EX(4, 4), SWIT_EX(4, 6), SWIT_EX(5, 3), SWIT_EX(5, 4), SWIT_EX(6, 3), SWIT_EX(7, 3),
+    SWIT_EX(8, 3),
+};
+#undef SWIT_EX
+
+size_t ex_lds_bytes(const rk::Cfg &c, int NI, int layers) {
+    return sizeof(float) * (rk::lds_edge_floats(c.W, c.R) + 2 * (size_t)rk::ex_set_floats(c.W, c.C, c.R, NI, layers));
+}
+
+// As choose_fwd (the same rows and so the same R).
+bool choose_ex(const Dims &d, int ns, int ncu, int NI, int layers, rk::Cfg *best) {
+    const int R = std::max(2, cdiv(d.nzp - (d.fs - 1) + 1, 64));
+    double best_t = 1e30;
+    for (const ExKernel &kn : kExKernels) {
+        if (kn.R != R) continue;
+        for (int W = 1; W <= 8; ++W) {
+            rk::Cfg c{};
+            c.R = R;
+            c.C = kn.C;
+            c.W = W;
+            c.z0 = d.fs - 1;
+            const int cols = W * c.C;
+            c.P = d.nxp <= cols ? 1 : cols > 2 * rk::kH ? cdiv(d.nxp - 2 * rk::kH, cols - 2 * rk::kH) : 0;
+            if (c.P < 1 || (c.P > 1 && cols < 3 * rk::kH)) continue;
+            const size_t lds = ex_lds_bytes(c, NI, layers);
+            if (lds + 1024 > kCuLds) continue;
+            const int per_cu = std::min(8 / W, (int)(kCuLds / (lds + 1024)));
+            if (c.P > max_windows(per_cu, ncu)) continue;
+            const int rounds = cdiv(ns, std::min(ns, per_cu * ncu / c.P));
+            c.G = cdiv(ns, rounds);
+            const double t = rounds * resident_step_us(W * cdiv(c.G * c.P, ncu), 60.0 * c.C * R, c.P > 1);
+            if (t < best_t) {
+                best_t = t;
+                *best = c;
+            }
+        }
+    }
+    return best_t < 1e30;
+}
+
+const ExKernel *find_ex(int R, int C) {
+    for (const ExKernel &k : kExKernels)
+        if (k.R == R && k.C == C) return &k;
+    return nullptr;
+}
+
+}  // namespace
+
+// The exact reverse loop's configuration and injection tables: every window takes the
+// receivers of all its columns, halo included, in receiver order within a cell.  The same
+// limits as the backward's; other acquisitions keep the step kernels.
+static int resident_init_ex(swit_plan *pl, int ncu) {
+    ResidentState &rs = pl->res;
+    BatchedState &bs = pl->bat;
+    const Dims &d = pl->d;
+    rs.ex = false;
+    if (!(pl->flags & (SWIT_PLAN_EXACT | SWIT_PLAN_EXACT_CKPT))) return SWIT_OK;
+    // the resident loops write checkpoints from row fs - 1 on
+    if (bs.ckpt) HIP_TRY(hipMemset(bs.ckpt, 0, sizeof(float) * bs.nck * pl->ns * 3 * d.nxp * d.ld));
+    if (!rs.fwd) return SWIT_OK;
+    unsigned long long mask = 0;
+    int layers = 1;
+    for (int s = 0; s < pl->ns; ++s) {
+        std::vector<int> q(pl->rec_cells_fwd.begin() + (size_t)s * d.ngmax,
+                           pl->rec_cells_fwd.begin() + (size_t)s * d.ngmax + pl->geo_h[s].ng);
+        for (int o : q) mask |= 1ull << ((o % d.ld + 1 - rs.fc.z0) / rs.fc.R);
+        std::sort(q.begin(), q.end());
+        for (size_t k = 0, m = 1; k + 1 < q.size(); ++k) {
+            m = q[k] == q[k + 1] ? m + 1 : 1;
+            layers = std::max(layers, (int)m);
+        }
+    }
+    const int NI = __builtin_popcountll(mask);
+    rk::Cfg c{};
+    if (layers > 2 || NI > 8 || !choose_ex(d, pl->ns, ncu, NI, layers, &c)) return SWIT_OK;
+    const int T = c.W * 64, WC = c.W * c.C;
+    std::vector<int2> itab((size_t)pl->ns * c.P * 2 * T, make_int2(-1, 0));
+    std::vector<int> n(c.P);
+    for (int s = 0; s < pl->ns; ++s) {
+        std::fill(n.begin(), n.end(), 0);
+        const int *cell = &pl->rec_cells_fwd[(size_t)s * d.ngmax];
+        std::set<int> taken;
+        for (int r = 0; r < pl->geo_h[s].ng; ++r) {
+            const int z = cell[r] % d.ld + 1 - c.z0, x = cell[r] / d.ld + 1;
+            const int layer = taken.insert(cell[r]).second ? 0 : 1;
+            const int slot = __builtin_popcountll(mask & ((1ull << (z / c.R)) - 1));
+            for (int j = 0; j < c.P; ++j) {
+                const int col = x - rk::window_x(c.W, c.C, j);
+                if (col < 0 || col >= WC) continue;
+                if (n[j] >= 2 * T) return SWIT_OK;
+                itab[((size_t)s * c.P + j) * 2 * T + n[j]++] =
+                    make_int2(((layer * NI + slot) * WC + col) * c.R + z % c.R, r);
+            }
+        }
+    }
+    rs.xc = c;
+    rs.x_imask = mask;
+    rs.x_layers = layers;
+    rs.x_lds = ex_lds_bytes(c, NI, layers);
+    HIP_TRY(hipFuncSetAttribute((const void *)find_ex(c.R, c.C)->fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)rs.x_lds));
+    TRY(pl->alloc(&rs.x_itab, itab.size()));
+    HIP_TRY(hipMemcpy(rs.x_itab, itab.data(), sizeof(int2) * itab.size(), hipMemcpyHostToDevice));
+    rs.x_msg = c.P > 1 ? (size_t)c.G * c.P * 4 * rk::kH * c.R * 64 : 0;
+    rs.ex = true;
+    return SWIT_OK;
+}
+
 // The backward's configuration and adjoint-source tables.  Receivers go through an LDS stage
 // of the lanes that hold injection cells (up to 8, up to two receivers in a cell and two per
 // thread of a window); other acquisitions keep the step kernels.
@@ -1563,9 +1689,10 @@ static int resident_init(swit_plan *pl) {
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     TRY(resident_init_bwd(pl, ncu));
     rs.fwd = choose_fwd(d, pl->ns, ncu, 8, &rs.fc);
+    TRY(resident_init_ex(pl, ncu));
     if (rs.fwd) TRY(resident_init_fwd(pl));
     if (!rs.fwd && !rs.bwd) return SWIT_OK;
-    TRY(pl->alloc(&rs.msg, std::max(rs.f_msg, rs.b_msg)));
+    TRY(pl->alloc(&rs.msg, std::max(rs.f_msg, std::max(rs.b_msg, rs.x_msg))));
     TRY(pl->alloc(&rs.ctl, 1));
     return SWIT_OK;
 }
@@ -1579,7 +1706,7 @@ static int resident_init_fwd(swit_plan *pl) {
     rs.f_lds = fwd_lds_bytes(c, __builtin_popcountll(rs.f_pmask));
     for (auto *fn : find_fwd(c.R, c.C)->fn)
         HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rs.f_lds));
-    rs.f_ncol = d.nxp + c.W * c.C;
+    rs.f_ncol = d.nxp + std::max(c.W * c.C, rs.ex ? rs.xc.W * rs.xc.C : 0);
     const size_t col = (size_t)64 * c.R;
     TRY(pl->alloc(&rs.f_co, (rs.f_ncol + 1) * 5 * col));
     TRY(pl->alloc(&rs.f_fpx, rs.f_ncol + 1));
@@ -1751,6 +1878,74 @@ static int resident_backward_steps(swit_plan *pl, const float *src, const float 
     a.ctl = rs.ctl;
     hipLaunchKernelGGL(find_bwd(rs.bc.R, rs.bc.C)->fn, dim3(rs.bc.G * rs.bc.P), dim3(64 * rs.bc.W), rs.b_lds, st, a);
     LAUNCH_CHECK();
+    return SWIT_OK;
+}
+
+// Exact forward: the divergence history of all steps, or a checkpoint every ck steps (the
+// state goes from checkpoint to checkpoint).
+static int resident_forward_exact(swit_plan *pl, float *seis, hipStream_t st) {
+    BatchedState &bs = pl->bat;
+    const Dims &d = pl->d;
+    hipLaunchKernelGGL(k_zero_rows, dim3(pl->ns), dim3(256), 0, st, pl->seis_t, (size_t)d.nt * d.ngmax, d.ngmax);
+    LAUNCH_CHECK();
+    const DSave none{nullptr, 0, 0};
+    if (!bs.ck) {
+        TRY(resident_forward_steps(pl, 2, d.nt, bs.src_ex, 0, DSave{bs.dhist, d.nt, 0}, nullptr, nullptr, nullptr, true, st));
+    } else {
+        const size_t chunk = (size_t)pl->ns * 3 * d.nxp * d.ld;
+        TRY(fill(bs.ckpt, chunk, st));
+        for (int j = 0; j < bs.nck; ++j) {
+            const int a = 1 + j * bs.ck, b = std::min(a + bs.ck, d.nt);
+            float *ck = bs.ckpt + j * chunk;
+            TRY(resident_forward_steps(pl, a + 1, b, bs.src_ex, 0, none, j ? ck : nullptr,
+                                       j + 1 < bs.nck ? ck + chunk : nullptr, nullptr, j == 0, st));
+        }
+    }
+    return resident_traces(pl, seis, st);
+}
+
+// Exact adjoint from the K-gradient zero: from the full history, or segment by segment (each
+// segment's history is recomputed first; the adjoint fields stay in lam in between).
+static int resident_adjoint_exact(swit_plan *pl, const float *gseis, hipStream_t st) {
+    ResidentState &rs = pl->res;
+    BatchedState &bs = pl->bat;
+    const Dims &d = pl->d;
+    hipLaunchKernelGGL(k_transpose, dim3(cdiv(d.nt, 32), cdiv(d.ngmax, 32), pl->ns), dim3(32, 8), 0, st, d.ngmax, d.nt,
+                       gseis, bs.gseis);
+    LAUNCH_CHECK();
+    TRY(fill(bs.gk, (size_t)pl->ns * d.nxp * d.ld, st));
+    rk::ExArgs x{};
+    x.d = d;
+    x.c = rs.xc;
+    x.ns = pl->ns;
+    x.co = rs.f_co;
+    x.ncol = rs.f_ncol;
+    x.fpx = rs.f_fpx;
+    x.g = bs.gseis;
+    x.itab = rs.x_itab;
+    x.imask = rs.x_imask;
+    x.layers = rs.x_layers;
+    x.gk = bs.gk;
+    x.msg = rs.msg;
+    x.ctl = rs.ctl;
+    const size_t chunk = (size_t)pl->ns * 3 * d.nxp * d.ld;
+    const int nseg = bs.ck ? bs.nck : 1;
+    for (int j = nseg - 1; j >= 0; --j) {
+        const bool first = j == nseg - 1;
+        const int a = bs.ck ? 1 + j * bs.ck : 1, b = bs.ck ? std::min(a + bs.ck, d.nt) : d.nt;
+        x.hist = bs.ck ? DSave{bs.dhist, bs.ck, a} : DSave{bs.dhist, d.nt, 0};
+        if (bs.ck)
+            TRY(resident_forward_steps(pl, a + 1, b, bs.src_ex, 0, x.hist, j ? bs.ckpt + j * chunk : nullptr, nullptr,
+                                       nullptr, first, st));
+        TRY(resident_begin(pl, rs.x_msg, first && !bs.ck, st));
+        x.it0 = a + 1;
+        x.it1 = b;
+        x.in = first ? nullptr : bs.lam;
+        x.add = !first;
+        x.out = j ? bs.lam : nullptr;
+        hipLaunchKernelGGL(find_ex(rs.xc.R, rs.xc.C)->fn, dim3(rs.xc.G * rs.xc.P), dim3(64 * rs.xc.W), rs.x_lds, st, x);
+        LAUNCH_CHECK();
+    }
     return SWIT_OK;
 }
 
@@ -2600,11 +2795,17 @@ extern "C" int swit_forward_exact(swit_plan *pl, const float *src, float *seis, 
     const Dims &d = pl->d;
     bs.exact_valid = false;
     HIP_TRY(hipMemcpyAsync(bs.src_ex, src, sizeof(float) * pl->ns * d.nt, hipMemcpyDeviceToDevice, stream));
-    TRY(forward_prologue(pl, 0, stream));
-    TRY(exact_run(pl, 0, stream));
-    hipLaunchKernelGGL(k_transpose, dim3(cdiv(d.ngmax, 32), cdiv(d.nt, 32), pl->ns), dim3(32, 8), 0, stream, d.nt,
-                       d.ngmax, pl->seis_t, seis);
-    LAUNCH_CHECK();
+    bool resident = false;
+    TRY(resident_now(pl->res.ex, pl->res.use_exact, stream, &resident));
+    if (resident) {
+        TRY(resident_forward_exact(pl, seis, stream));
+    } else {
+        TRY(forward_prologue(pl, 0, stream));
+        TRY(exact_run(pl, 0, stream));
+        hipLaunchKernelGGL(k_transpose, dim3(cdiv(d.ngmax, 32), cdiv(d.nt, 32), pl->ns), dim3(32, 8), 0, stream, d.nt,
+                           d.ngmax, pl->seis_t, seis);
+        LAUNCH_CHECK();
+    }
     bs.exact_valid = true;
     ++bs.exact_gen;
     return SWIT_OK;
@@ -2624,16 +2825,22 @@ extern "C" int swit_adjoint_exact(swit_plan *pl, const float *gseis, double *gra
     const Dims &d = pl->d;
     const int ns = pl->ns;
     const size_t np = (size_t)d.nxp * d.ld;
-    HIP_TRY(hipMemcpyAsync(bs.gseis, gseis, sizeof(float) * ns * d.ngmax * d.nt, hipMemcpyDeviceToDevice, stream));
-    TRY(fill(bs.lam, 3 * np * ns, stream));
-    TRY(fill(bs.lam2, 3 * np * ns, stream));
-    TRY(fill(bs.gk, np * ns, stream));
-    TRY(exact_run(pl, 1, stream));
+    bool resident = false;
+    TRY(resident_now(pl->res.ex, pl->res.use_exact, stream, &resident));
+    if (resident) {
+        TRY(resident_adjoint_exact(pl, gseis, stream));
+    } else {
+        HIP_TRY(hipMemcpyAsync(bs.gseis, gseis, sizeof(float) * ns * d.ngmax * d.nt, hipMemcpyDeviceToDevice, stream));
+        TRY(fill(bs.lam, 3 * np * ns, stream));
+        TRY(fill(bs.lam2, 3 * np * ns, stream));
+        TRY(fill(bs.gk, np * ns, stream));
+        TRY(exact_run(pl, 1, stream));
+    }
     hipLaunchKernelGGL(ex::k_ex_shotsum, dim3((unsigned)std::min<size_t>(cdiv((int)np, 256), 4096)), dim3(256), 0,
                        stream, d, ns, bs.gk, bs.gsum);
     LAUNCH_CHECK();
     hipLaunchKernelGGL(ex::k_ex_fold, dim3(cdiv(d.nz, 64), cdiv(d.nx, 4)), dim3(64, 4), 0, stream, d, pl->c_int,
-                       pl->rho_int, bs.gsum, grad);
+                       pl->rho_int, bs.gsum, resident ? &pl->res.ctl->err : nullptr, grad);
     LAUNCH_CHECK();
     return SWIT_OK;
 }

@@ -111,3 +111,63 @@ def test_seismograms_against_the_oracle():
     p.set_model(torch.from_numpy(w.vp_init), torch.from_numpy(workloads.gardner(w.vp_init)))
     np.testing.assert_array_equal(p.forward(torch.from_numpy(src)).cpu().numpy(), f["seis"])
     p.close()
+
+
+def _exact_outputs(w, kind, resident, free_surface=1):
+    import torch
+    from swit_amd.engine import Plan
+    p = Plan(w.nx, w.nz, w.dx, w.dt, w.nt, w.npml, w.src_xz, w.rec_xz, strips="none", exact=kind,
+             free_surface=free_surface)
+    p.set_model(torch.from_numpy(w.vp_init), torch.from_numpy(workloads.gardner(w.vp_init)))
+    p.set_option("resident", resident)
+    src = torch.from_numpy(integrated_sources(w))
+    out = []
+    for _ in range(2):
+        syn = p.forward_exact(src)
+        g = torch.flip(syn, (2,)) + syn
+        out.append([syn.cpu().numpy(), p.adjoint_exact(g.contiguous()).cpu().numpy()])
+    p.close()
+    return out
+
+
+def _check_exact(w, kind, free_surface=1):
+    """The reverse loop's operations and their order are the step kernels': equal but for the
+    sign of zeros (cells outside an update region multiply by 0 there, here they are skipped)."""
+    ref, got = (_exact_outputs(w, kind, r, free_surface) for r in (0, 1))
+    assert np.abs(ref[0][0]).max() > 0
+    for a, b in zip(ref, got):
+        np.testing.assert_array_equal(b[0], a[0])
+        np.testing.assert_array_equal(b[1], a[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nz,npml", [(117, 10), (118, 10), (181, 10), (182, 10), (246, 9), (310, 10), (373, 10),
+                                     (438, 9), (501, 10)])
+def test_exact_rows_per_lane(nz, npml):
+    w = workloads.small(seed=nz, nx=70, nz=nz, npml=npml, nt=90, ns=2)
+    _check_exact(w, True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx", [8, 9, 34, 49, 50, 51, 52, 53, 61, 121, 240])
+def test_exact_widths(nx):
+    w = workloads.small(seed=nx, nx=nx, nz=40, npml=10, nt=70, ns=2)
+    _check_exact(w, "checkpoint" if nx % 3 else True, free_surface=nx % 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nt", [2, 3, 5, 49, 50, 101])
+def test_exact_checkpoint_segments(nt):
+    """Records of one segment, of a last segment of one step, of full segments."""
+    w = workloads.small(seed=nt, nx=60, nz=30, npml=8, nt=nt, ns=3)
+    _check_exact(w, "checkpoint")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [True, "checkpoint"])
+def test_exact_shared_cells_and_many_shots(kind):
+    w = workloads.small(seed=6, nx=130, nz=50, npml=10, nt=80, ns=70)
+    rec = [[x * w.dx, z * w.dx] for x in range(w.nx) for z in (1.0, 9.0)]
+    rec += [[17 * w.dx, w.dx], [18 * w.dx, 9.0 * w.dx], [29 * w.dx, w.dx]]
+    w.rec_xz = [np.asarray(rec[:len(rec) - i], np.float32) for i in range(w.ns)]
+    _check_exact(w, kind)
