@@ -77,6 +77,8 @@ __host__ __device__ inline int window_oe(int W, int C, int j, int P, int nxp) {
     return j + 1 < P ? window_x(W, C, j) + W * C - 1 - kH : nxp;
 }
 
+constexpr int kHistPad = 64 * 8;    // floats past the divergence history: a column's lanes past the grid read them
+
 struct Ctl {
     unsigned ticket;
     int err;
@@ -706,18 +708,26 @@ struct BwdArgs {
     const int *itab, *ibase;
     unsigned long long imask;   // lanes of the injection stage
     int layers;                 // receivers of one cell (1 or 2)
+    int ring;                   // steps whose values are held (a power of two)
+    int ninj, sides;            // most receivers, most side layers (1 or 2) of a window
     float *acc;                 // [ns][nxp][3][64 R] per-shot accumulators, zero at the start
     u64 *msg;                   // [G P][2 slots][2 sides][2 fields][3 R][64]
     Ctl *ctl;
 };
 
-// LDS of the backward: the waves' edge columns of both wavefields, then two sets (a step's
-// and the next one's) of: the strip rows' lanes [4][W C][R], w of row nz-1 [W C], the side
-// columns [6][64 R] (p of jx = 1, 2, nx-1, nx, u of jx = 1, nx-1), the injection stage
-// [layers][NI + 1][W C][R] (the last one zeros).
-__host__ __device__ inline int bwd_edge_floats(int W, int R) { return W * 12 * R * 64; }
+// LDS of the backward: the waves' edge columns of both wavefields (p, then u: with R >= 5 in
+// one place, with a barrier between the last read and the first write); two sets (a step's and
+// the next one's) of the strip rows' lanes [4][W C][R], w of row nz-1 [W C], the injection
+// stage [layers][NI + 1][W C][R] (the last one zeros); the values of `ring` steps as they
+// come: [ring][6 W C strip values of the columns, ninj adjoint sources]; the side columns of
+// `ring` steps [ring][sides][p, next p, u][64 R].
+constexpr bool bwd_one_edge_set(int R) { return R >= 5; }
+__host__ __device__ inline int bwd_edge_floats(int W, int R) { return W * (bwd_one_edge_set(R) ? 6 : 12) * R * 64; }
 __host__ __device__ inline int bwd_set_floats(int W, int C, int R, int NI, int layers) {
-    return 4 * W * C * R + ((W * C + 3) & ~3) + 6 * 64 * R + layers * (NI + 1) * W * C * R;
+    return 4 * W * C * R + ((W * C + 3) & ~3) + layers * (NI + 1) * W * C * R;
+}
+__host__ __device__ inline int bwd_step_floats(int W, int C, int R, int ninj, int sides) {
+    return 6 * W * C + ninj + sides * 3 * 64 * R;
 }
 
 // Reverse steps nt .. 2 (solver.f90:230-253) of every shot: reconstruction (fdcore.f90:
@@ -725,9 +735,17 @@ __host__ __device__ inline int bwd_set_floats(int W, int C, int R, int NI, int l
 // registers (6 R C <= 150 floats at two waves per SIMD).  A step is: velocities of both
 // fields from p (edges through LDS), strip values into the reconstructed u, w; then
 // pressures, strip values into the reconstructed p, injection and mirror of the adjoint p,
-// imaging.  Strip values and adjoint sources are loaded one step ahead and handed out
-// through LDS.  The accumulators are read and written in memory every step (they stay in
+// imaging.  Strip values and adjoint sources come from HBM, and loads complete in order: one
+// value of the step that is fetched makes every later load of the wave wait for HBM.  So the
+// values of ring - 1 steps are fetched at once, and handed out through LDS step by step.  The accumulators are read and written in memory every step (they stay in
 // L2): the wavefields alone fill the registers.
+// Per time step (481x141, 49 shots, in three rounds of 17; the step kernel 86 us): 33.9 us with
+// values fetched one step ahead, 30.9 with the ring, 27.5 with the accumulators' loads and
+// stores free of branches (a wait has to assume the fewest loads in flight that any path
+// leaves, and so waited for the stores of the column before).  One shot of 201x81: 7.5 us by
+// the step kernel, 6.4, 5.2, 5.1; 801x267, 81 shots: 432 by the step kernel, 224, 186, 180
+// (R = 6: eight waves fit since the edges of p and u share their place).  Vector issue is 5.9 of
+// the 9.2 us of a round of the 49 shots.
 template <int R, int C>
 __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
     extern __shared__ float lds[];
@@ -743,10 +761,14 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
     const int grp = __builtin_amdgcn_readfirstlane(t / P), j = __builtin_amdgcn_readfirstlane(t % P);
     const int WC = W * C, NI = __popcll(a.imask);
     float *eP = lds;                                     // [W][2 fields][3][R][64]: first, second, last column of p
-    float *eU = eP + W * 6 * R * 64;                     // [W][2 fields][3][R][64]: first, last but one, last of u
+    // [W][2 fields][3][R][64]: first, last but one, last of u
+    float *eU = bwd_one_edge_set(R) ? eP : eP + W * 6 * R * 64;
     const int set_floats = bwd_set_floats(W, C, R, NI, a.layers);
-    float *sets = eU + W * 6 * R * 64;
-    const int o_w = 4 * WC * R, o_side = o_w + ((WC + 3) & ~3), o_inj = o_side + 6 * 64 * R;
+    const int ring = a.ring, nraw = 6 * WC + a.ninj;
+    float *sets = lds + bwd_edge_floats(W, R);
+    float *raw = sets + 2 * set_floats;
+    float *side_ring = raw + ring * nraw;
+    const int o_w = 4 * WC * R, o_inj = o_w + ((WC + 3) & ~3);
     const int xw = window_x(W, C, j), x0w = xw + wave * C;
     const bool has_l = j > 0, has_r = j + 1 < P;
     const bool edge = (has_l && wave <= (2 * kH - 1) / C) || (has_r && wave >= W - 1 - (2 * kH - 1) / C);
@@ -776,103 +798,111 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
     }
     const unsigned acc_off = inner ? voff0 : 0x80000000u;          // past the buffer: loads 0, stores nothing
 
-    // ---- values of one step: strip values of the window's columns (n-th: column n / 6, value
-    // n % 6: p of jz = 1, 2, 3, nz, nz-1, w of nz-1), of the side columns, adjoint sources ----
-    struct Step {
-        uint32_t col[NI6], side[3];
-        float inj[2];
-        float scale;
-    };
-    // what thread item n of the side columns is: window column offset, strip place; false: none
-    auto side_item = [&](ArgPtr<BwdArgs> k, int n, int &q, int &jz, int &place) {
-        const int nz = k->d.nz;
-        const int v = n / (64 * R), row = n % (64 * R);
-        jz = k->c.z0 + row - k->d.npml;
-        if (v >= 6 || jz < 1 || jz > nz) return false;
-        // v: 0 p(1), 1 p(2), 2 p(nx-1), 3 p(nx), 4 u(1), 5 u(nx-1)
-        const int nx = k->d.nx;
-        const int jx = v == 0 || v == 4 ? 1 : v == 1 ? 2 : v == 3 ? nx : nx - 1;
-        const int x = k->d.npml + jx, xw_ = window_x(k->c.W, C, j);
-        q = v == 0 ? 0 : v == 1 ? 1 : v == 2 ? 4 : v == 3 ? 3 : v == 4 ? 2 : 5;
-        place = v * 64 * R + row;
-        return x >= xw_ && x < xw_ + k->c.W * C;
-    };
-    // The side columns of a window: left three (v = 0, 1, 4), right three, or both.  Items are
-    // the 6 x 64 R places, T at a time; windows without side columns take none.
-    const bool win_side = (xw <= a.d.npml + 2 && xw + WC > a.d.npml + 1) ||
-                          (xw <= a.d.npml + a.d.nx && xw + WC > a.d.npml + a.d.nx - 1);
-    auto load_step = [&](int s, int it, Step &v, int i0, int i1, int ib) {
+    // ---- values of a step: strip values of the window's columns (n-th: column n / 6, value
+    // n % 6: p of jz = 1, 2, 3, nz, nz-1, w of nz-1), the thread's own at n = tid + i T, to
+    // place col_dst of a set; adjoint sources; side columns ----
+    int col_dst[NI6];
+    {
+        const int nx = a.d.nx, nz = a.d.nz, npml = a.d.npml;
+#pragma unroll
+        for (int i = 0; i < NI6; ++i) {
+            const int n = threadIdx.x + i * T, col = n / 6, q = n % 6, jx = xw + col - npml;
+            const int row = (q < 3 ? q + 1 : q == 3 ? nz : nz - 1) + npml - a.c.z0, L = row / R;
+            col_dst[i] = col >= WC || jx < 1 || jx > nx ? -1
+                         : q == 5                       ? o_w + col
+                                                        : ((L <= lm + 1 ? L - lm : 2 + L - lb) * WC + col) * R + row % R;
+        }
+    }
+    const bool side_l = xw <= a.d.npml + 2 && xw + WC > a.d.npml + 1;
+    const bool side_r = xw <= a.d.npml + a.d.nx && xw + WC > a.d.npml + a.d.nx - 1;
+    constexpr int kSide = 64 * R;
+    const int side_floats = a.sides * 3 * kSide, o_right = side_l ? 3 * kSide : 0;
+    const int c1 = a.d.npml + 1 - x0w, cn = a.d.npml + a.d.nx - x0w;      // this wave's columns of jx = 1, nx
+    const bool wave_side = (c1 < C && c1 >= -1) || (cn >= 0 && cn <= C);
+    // values of steps t, t-1, .. (ring - 1 of them, down to step 2) into the ring
+    auto fetch_steps = [&](int s, int t, int i0, int i1, int ib) {
+        constexpr int U = 4;                             // steps in flight
         const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
-        const int S = k->d.S, nx = k->d.nx, nz = k->d.nz;
-        const size_t row = (size_t)s * k->d.nt + (it - 2);
-        const int mode = k->mode;
-        const char *b = (const char *)k->strips + row * S * (mode == 0 ? 4 : 2);
-        auto get = [&](int i) -> uint32_t {
-            if (mode == 0) return ((const uint32_t *)b)[i];
-            return ((const uint16_t *)b)[i];
+        const int nx = k->d.nx, nz = k->d.nz, mode = k->mode, WC_ = k->c.W * C, T_ = k->c.W * 64;
+        const size_t S = k->d.S, row0 = (size_t)s * k->d.nt + (t - 2), ngmax = k->d.ngmax;
+        const int cnt = min(ring - 1, t - 1);
+        unsigned tid = threadIdx.x;
+        opaque_v(tid);
+        auto get = [&](size_t i, float scale) -> float {
+            if (mode == 0) return ((const float *)k->strips)[i];
+            const uint16_t x = ((const uint16_t *)k->strips)[i];
+            return (mode == 1 ? strip_decode<1>(x) : strip_decode<2>(x)) * scale;
         };
-        v.scale = mode ? strip_scale(k->smax[row]) : 1.0f;
-        const int top0 = 3 * nx + 6 * nz, xw_ = window_x(k->c.W, C, j), WC_ = k->c.W * C, T_ = k->c.W * 64;
-        unsigned tid = threadIdx.x;
-        opaque_v(tid);
+        // lane l: the scale of the l-th row (16-bit strips)
+        const float scales = mode ? strip_scale(k->smax[row0 - min(lane, cnt - 1)]) : 1.0f;
+        auto scale_of = [&](int n) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(scales), n)); };
+        const float *adj = k->adj + (row0 + 1) * ngmax + ib + tid;
+        for (int b = 0; b < cnt; b += U) {
+            float v[U][NI6], g0[U], g1[U];
 #pragma unroll
-        for (int i = 0; i < NI6; ++i) {
-            const int n = tid + i * T_, col = n / 6, q = n % 6, jx = xw_ + col - k->d.npml;
-            v.col[i] = 0;
-            if (col < WC_ && jx >= 1 && jx <= nx)
-                v.col[i] = get(q < 3 ? top0 + 6 * (jx - 1) + q : 3 * (jx - 1) + q - 3);
-        }
-        if (win_side) {
+            for (int u = 0; u < U; ++u) {
+                if (b + u >= cnt) break;
+                const size_t row = row0 - (b + u);
+                const float scale = scale_of(b + u);
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                int q, jz, place;
-                v.side[i] = 0;
-                // places past 3 T (few waves): see store_step
-                if (side_item(k, tid + i * T_, q, jz, place)) v.side[i] = get(3 * nx + 6 * (jz - 1) + q);
-            }
-        }
-        const float *adj = k->adj + ((size_t)s * k->d.nt + (it - 1)) * k->d.ngmax + ib;
-        v.inj[0] = i0 >= 0 ? adj[tid] : 0.0f;
-        v.inj[1] = i1 >= 0 ? adj[tid + T_] : 0.0f;
-    };
-    auto decode = [&](int mode, uint32_t x, float scale) -> float {
-        if (mode == 0) return __uint_as_float(x);
-        return (mode == 1 ? strip_decode<1>((uint16_t)x) : strip_decode<2>((uint16_t)x)) * scale;
-    };
-    // values into set `par` of the LDS; i0, i1: this thread's injection places
-    auto store_step = [&](int s, int it, const Step &v, int par, int i0, int i1) {
-        const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
-        const int nz = k->d.nz, npml = k->d.npml, WC_ = k->c.W * C, T_ = k->c.W * 64, z0 = k->c.z0, mode = k->mode;
-        float *f = sets + par * set_floats;
-        unsigned tid = threadIdx.x;
-        opaque_v(tid);
-#pragma unroll
-        for (int i = 0; i < NI6; ++i) {
-            const int n = tid + i * T_, col = n / 6, q = n % 6;
-            if (col >= WC_) continue;
-            const float x = decode(mode, v.col[i], v.scale);
-            if (q == 5) {
-                f[o_w + col] = x;
-            } else {
-                const int row = (q < 3 ? q + 1 : q == 3 ? nz : nz - 1) + npml - z0, L = row / R;
-                f[((L <= lm + 1 ? L - lm : 2 + L - lb) * WC_ + col) * R + row % R] = x;
-            }
-        }
-        if (win_side) {
-            int q, jz, place;
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-                if (side_item(k, tid + i * T_, q, jz, place)) f[o_side + place] = decode(mode, v.side[i], v.scale);
-            // the rest, for workgroups of few waves: loaded here
-            for (int n = tid + 3 * T_; n < 6 * 64 * R; n += T_)
-                if (side_item(k, n, q, jz, place)) {
-                    const size_t i = ((size_t)s * k->d.nt + (it - 2)) * k->d.S + 3 * k->d.nx + 6 * (jz - 1) + q;
-                    const uint32_t x = mode == 0 ? ((const uint32_t *)k->strips)[i] : ((const uint16_t *)k->strips)[i];
-                    f[o_side + place] = decode(mode, x, v.scale);
+                for (int i = 0; i < NI6; ++i) {
+                    const int n = tid + i * T_, col = n / 6, q = n % 6, jx = window_x(k->c.W, C, j) + col - k->d.npml;
+                    v[u][i] = 0.0f;
+                    if (col < WC_ && jx >= 1 && jx <= nx)
+                        v[u][i] = get(row * S + (q < 3 ? 3 * nx + 6 * nz + 6 * (jx - 1) + q : 3 * (jx - 1) + q - 3), scale);
                 }
+                g0[u] = i0 >= 0 ? adj[0] : 0.0f;
+                g1[u] = i1 >= 0 ? adj[T_] : 0.0f;
+                adj -= ngmax;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (b + u >= cnt) break;
+                float *q = raw + ((t - b - u) & (ring - 1)) * nraw + tid;
+#pragma unroll
+                for (int i = 0; i < NI6; ++i)
+                    if ((int)tid + i * T_ < 6 * WC_) q[i * T_] = v[u][i];
+                if (i0 >= 0) q[6 * WC_] = k->d.dt * g0[u];
+                if (i1 >= 0) q[6 * WC_ + T_] = k->d.dt * g1[u];
+            }
         }
-        if (i0 >= 0) f[o_inj + i0] = k->d.dt * v.inj[0];
-        if (i1 >= 0) f[o_inj + i1] = k->d.dt * v.inj[1];
+        if (side_l || side_r) {
+            const int n1 = side_l && side_r ? 2 * kSide : kSide;
+            for (int n = tid; n < n1; n += T_) {
+                const int right = side_l ? n / kSide : 1, row_ = n % kSide, jz = k->c.z0 + row_ - k->d.npml;
+                if (jz < 1 || jz > nz) continue;
+                const size_t o = 3 * nx + 6 * (jz - 1) + 3 * right;
+                float *to = side_ring + (right ? o_right : 0) + row_;
+                for (int b = 0; b < cnt; b += U) {
+                    float v[U][3];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        if (b + u >= cnt) break;
+                        const size_t row = row0 - (b + u);
+                        const float scale = scale_of(b + u);
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) v[u][q] = get(row * S + o + q, scale);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        if (b + u >= cnt) break;
+                        float *f = to + ((t - b - u) & (ring - 1)) * side_floats;
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) f[q * kSide] = v[u][q];
+                    }
+                }
+            }
+        }
+    };
+    // step t's own values from the ring into its set
+    auto hand_out = [&](int t, int i0, int i1) {
+        float *f = sets + (t & 1) * set_floats;
+        const float *q = raw + (t & (ring - 1)) * nraw + threadIdx.x;
+#pragma unroll
+        for (int i = 0; i < NI6; ++i)
+            if (col_dst[i] >= 0) f[col_dst[i]] = q[i * T];
+        if (i0 >= 0) f[o_inj + i0] = q[6 * WC];
+        if (i1 >= 0) f[o_inj + i1] = q[6 * WC + T];
     };
 
     for (int s = a.s0 + grp; s < a.s0 + a.ns; s += a.c.G) {
@@ -883,7 +913,7 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
         const int i0 = a.itab[((size_t)s * P + j) * 2 * T + threadIdx.x];
         const int i1 = a.itab[((size_t)s * P + j) * 2 * T + T + threadIdx.x];
         const int ib = a.ibase[s * P + j];
-        for (int i = threadIdx.x; i < 2 * set_floats; i += T) sets[i] = 0.0f;
+        for (int i = threadIdx.x; i < 2 * set_floats + ring * (nraw + side_floats); i += T) sets[i] = 0.0f;
         float pr[C][R], ur[C][R], wr[C][R], pa[C][R], ua[C][R], wa[C][R];
 #pragma unroll
         for (int c = 0; c < C; ++c)
@@ -913,9 +943,10 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
             }
         }
         __syncthreads();
-        Step nxt;
-        load_step(s, a.d.nt, nxt, i0, i1, ib);
-        store_step(s, a.d.nt, nxt, a.d.nt & 1, i0, i1);
+        int left = a.d.nt;                               // first step whose values are not fetched
+        fetch_steps(s, left, i0, i1, ib);
+        left -= ring - 1;
+        hand_out(a.d.nt, i0, i1);
         // p of the edge columns for the next step
         auto put_p = [&]() {
             float *e = eP + (size_t)wave * 6 * R * 64 + lane;
@@ -943,7 +974,11 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
             opaque_s(x0);
             opaque_v(voff);
             const float *set = sets + (it & 1) * set_floats;
-            if (it > 2) load_step(s, it - 1, nxt, i0, i1, ib);
+            if (it - 1 == left && it > 2) {
+                fetch_steps(s, left, i0, i1, ib);
+                left -= ring - 1;
+            }
+            const float *side = side_ring + (it & (ring - 1)) * side_floats + voff / 4;
             float ssub;                                  // the reference's s(it+1), 0 past the end
             {
                 const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
@@ -967,6 +1002,7 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
                 edge_rows(eP, wave + 1, 3, a1);
                 edge_rows(eP, wave + 1, 1, r2);
                 edge_rows(eP, wave + 1, 4, a2);
+                if constexpr (bwd_one_edge_set(R)) lds_barrier();
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
                     if (c + 1 < C) fetch(c + 1);
@@ -1013,13 +1049,11 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
                 }
             }
             // strip values of the reconstructed u, columns jx = 1 and nx - 1
-            if (win_side) {
-                const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
-                const int c1 = k->d.npml + 1 - x0, cn = k->d.npml + k->d.nx - 1 - x0;
+            if (wave_side) {
 #pragma unroll
                 for (int c = 0; c < C; ++c)
-                    if (c == c1 || c == cn) {
-                        const float *q = set + o_side + (c == c1 ? 4 : 5) * 64 * R + voff / 4;
+                    if (c == c1 || c == cn - 1) {
+                        const float *q = side + (c == c1 ? 0 : o_right) + 2 * kSide;
 #pragma unroll
                         for (int r = 0; r < R; ++r) ur[c][r] = q[r];
                     }
@@ -1053,7 +1087,6 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
             {
                 const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
                 const ArgPtr<float> fpx = (ArgPtr<float>)k->fpx + x0;
-                const int c1 = k->d.npml + 1 - x0, cn = k->d.npml + k->d.nx - x0;   // columns of jx = 1, nx
                 const int os = window_os(k->c.W, C, j), oe = window_oe(k->c.W, C, j, k->c.P, k->d.nxp);
                 const int ca = max(c1, os - x0), cb = min(cn, oe - x0);             // columns imaged here
                 const __amdgpu_buffer_rsrc_t ab = __builtin_amdgcn_make_buffer_rsrc(
@@ -1063,12 +1096,14 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
                 auto fetch = [&](int c) {
                     buffer_rows<R>(co, voff, (x0 + c) * (5 * kCol), kp[c & 1]);
                     buffer_rows<R>(co, voff, (x0 + c) * (5 * kCol) + kCol, kv[c & 1]);
-                    if (c >= ca && c <= cb) {
-                        const int o = (x0 + c - 1) * (3 * kCol);
-                        buffer_rows<R>(ab, ao, o, g0[c & 1]);
-                        buffer_rows<R>(ab, ao, o + kCol, g1[c & 1]);
-                        buffer_rows<R>(ab, ao, o + 2 * kCol, g2[c & 1]);
-                    }
+                    // no branch (the loads and stores in flight stay countable): past the buffer
+                    // where nothing is imaged
+                    const bool im = c >= ca && c <= cb;
+                    const int o = im ? (x0 + c - 1) * (3 * kCol) : 0;
+                    const unsigned aoc = ao | (im ? 0u : 0x80000000u);
+                    buffer_rows<R>(ab, aoc, o, g0[c & 1]);
+                    buffer_rows<R>(ab, aoc, o + kCol, g1[c & 1]);
+                    buffer_rows<R>(ab, aoc, o + 2 * kCol, g2[c & 1]);
                 };
                 fetch(0);
                 float r2[R], a2[R], r1[R], a1[R], rr[R], ar[R];
@@ -1078,6 +1113,7 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
                 edge_rows(eU, wave - 1, 5, a1);
                 edge_rows(eU, wave + 1, 0, rr);
                 edge_rows(eU, wave + 1, 3, ar);
+                if constexpr (bwd_one_edge_set(R)) lds_barrier();
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
                     if (c + 1 < C) fetch(c + 1);
@@ -1098,8 +1134,8 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
                             pr[c][r] = brow & (1u << r) ? q[r] : v;
                         }
                     }
-                    if (win_side && (c == c1 || c == c1 + 1 || c == cn - 1 || c == cn)) {
-                        const float *q = set + o_side + (c == c1 ? 0 : c == c1 + 1 ? 1 : c == cn ? 3 : 2) * 64 * R + voff / 4;
+                    if (wave_side && (c == c1 || c == c1 + 1 || c == cn - 1 || c == cn)) {
+                        const float *q = side + (c == c1 || c == c1 + 1 ? 0 : o_right) + (c == c1 || (c != c1 + 1 && c == cn) ? 0 : kSide);
 #pragma unroll
                         for (int r = 0; r < R; ++r) pr[c][r] = q[r];
                     }
@@ -1133,17 +1169,19 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
                         pin(pr[c][r]);
                         pin(pa[c][r]);
                     }
-                    if (c >= ca && c <= cb) {
-                        const int o = (x0 + c - 1) * (3 * kCol);
+                    {
+                        const bool im = c >= ca && c <= cb;
+                        const int o = im ? (x0 + c - 1) * (3 * kCol) : 0;
+                        const unsigned aoc = ao | (im ? 0u : 0x80000000u);
 #pragma unroll
                         for (int r = 0; r < R; ++r) {
                             g0[c & 1][r] = g0[c & 1][r] + pr[c][r] * (old[r] - pa[c][r]);
                             g1[c & 1][r] = g1[c & 1][r] + pr[c][r] * pr[c][r];
                             g2[c & 1][r] = g2[c & 1][r] + pa[c][r] * pa[c][r];
                         }
-                        buffer_store_rows<R>(ab, ao, o, g0[c & 1]);
-                        buffer_store_rows<R>(ab, ao, o + kCol, g1[c & 1]);
-                        buffer_store_rows<R>(ab, ao, o + 2 * kCol, g2[c & 1]);
+                        buffer_store_rows<R>(ab, aoc, o, g0[c & 1]);
+                        buffer_store_rows<R>(ab, aoc, o + kCol, g1[c & 1]);
+                        buffer_store_rows<R>(ab, aoc, o + 2 * kCol, g2[c & 1]);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -1159,7 +1197,7 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
                 send_edges<R, C>(has_l, has_r, wave, W, box - 3 * kMsg, box + 4 * kMsg, tag, pr);
                 send_edges<R, C>(has_l, has_r, wave, W, box - 3 * kMsg + kMsg / 2, box + 4 * kMsg + kMsg / 2, tag, pa);
             }
-            if (exch) store_step(s, it - 1, nxt, (it - 1) & 1, i0, i1);
+            if (exch) hand_out(it - 1, i0, i1);
             if (edge && exch) {
                 const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
                 recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, dead, pr);

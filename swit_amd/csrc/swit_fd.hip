@@ -76,7 +76,7 @@ struct ResidentState {
     float *b_co = nullptr, *b_fpx = nullptr;
     int b_ncol = 0;
     unsigned long long b_imask = 0;
-    int b_layers = 1;
+    int b_layers = 1, b_ring = 2, b_ninj = 0, b_sides = 1;
     int *b_itab = nullptr;       // [ns][P][2][64 W]
     int *b_ibase = nullptr;      // [ns][P]
     int *b_imap = nullptr;       // [ns][ngmax] slot -> receiver
@@ -798,9 +798,9 @@ static int batched_init(swit_plan *pl) {
             bs.ck = std::max(1, (int)std::lround(std::sqrt((double)d.nt)));
             bs.nck = cdiv(d.nt - 1, bs.ck);
             TRY(pl->alloc(&bs.ckpt, (size_t)bs.nck * ns * 3 * np));
-            TRY(pl->alloc(&bs.dhist, (size_t)ns * bs.ck * np));
+            TRY(pl->alloc(&bs.dhist, (size_t)ns * bs.ck * np + rk::kHistPad));
         } else {
-            TRY(pl->alloc(&bs.dhist, (size_t)ns * d.nt * np));
+            TRY(pl->alloc(&bs.dhist, (size_t)ns * d.nt * np + rk::kHistPad));
         }
         TRY(pl->alloc(&bs.lam, (size_t)ns * 3 * np));
         TRY(pl->alloc(&bs.lam2, (size_t)ns * 3 * np));
@@ -1274,14 +1274,16 @@ size_t fwd_lds_bytes(const rk::Cfg &c, int NS) {
 }
 
 // Estimated time of one resident step (us): the vector issue of the waves that share a
-// compute unit, with what their latency adds, and the exchange and the barriers.  Fitted to
-// the forward on grids of 201x81 to 481x141 (2.4 GHz, 36 operations per cell): with one wave
-// per SIMD 1.34 times the issue time, with two or more 0.93, plus 1.45 us with an exchange
-// (one shot, R = 2, C = 3, W = 4: 1.99 measured, 1.93 estimated; C = 9: 2.95 and 2.90;
-// 49 shots, R = 3, C = 16, W = 8: 6.76 and 6.81).
-double resident_step_us(int waves_on_cu, double cell_ops, bool exchange) {
+// compute unit (2.4 GHz, 4 cycles an operation), with what their latency adds, and a fixed part
+// for the exchange, the barriers and what is read and written per step.  Fitted to the forward
+// on grids of 201x81 to 481x141 (36 operations per cell, fixed 1.45 us with an exchange, 0.9
+// without): one shot, R = 2, C = 3, W = 4: 1.99 measured, 1.93 estimated, C = 9: 2.95 and 2.90;
+// 49 shots, R = 3, C = 16, W = 8: 6.76 and 6.81.  Backward (80 operations, fixed 3.4 us):
+// one shot, R = 3, C = 3, W = 3: 5.1 and 5.1, W = 8: 5.4 and 5.6; 49 shots, R = 4, W = 8, C = 6: 9.2
+// and 9.4, C = 5: 8.2 and 8.4.
+double resident_step_us(int waves_on_cu, double cell_ops, double fixed) {
     const double issue = cdiv(waves_on_cu, 4) * cell_ops * 4 / 2400.0;
-    return (waves_on_cu > 4 ? 0.93 : 1.34) * issue + (exchange ? 1.45 : 0.9);
+    return (waves_on_cu > 4 ? 0.93 : 1.34) * issue + fixed;
 }
 
 // Most windows of a shot.  The windows of a group wait for each other, and of every launch
@@ -1315,7 +1317,7 @@ bool choose_fwd(const Dims &d, int ns, int ncu, int NS, rk::Cfg *best) {
             if (c.P > max_windows(per_cu, ncu)) continue;
             const int rounds = cdiv(ns, std::min(ns, per_cu * ncu / c.P));
             c.G = cdiv(ns, rounds);
-            const double t = rounds * resident_step_us(W * cdiv(c.G * c.P, ncu), 36.0 * c.C * R, c.P > 1);
+            const double t = rounds * resident_step_us(W * cdiv(c.G * c.P, ncu), 36.0 * c.C * R, c.P > 1 ? 1.45 : 0.9);
             if (t < best_t) {
                 best_t = t;
                 *best = c;
@@ -1419,13 +1421,40 @@ struct BwdKernel {
 #define SWIT_BWD(R, C) {R, C, rk::k_bwd_resident<R, C>}
 const BwdKernel kBwdKernels[] = {
     SWIT_BWD(2, 3), SWIT_BWD(2, 6), SWIT_BWD(2, 12), SWIT_BWD(3, 3), SWIT_BWD(3, 6), SWIT_BWD(3, 8),
-    SWIT_BWD(4, 3), SWIT_BWD(4, 5), SWIT_BWD(4, 6), SWIT_BWD(5, 3), SWIT_BWD(5, 4), SWIT_BWD(6, 3), SWIT_BWD(6, 4),
+    SWIT_BWD(4, 3), SWIT_BWD(4, 5), SWIT_BWD(4, 6), SWIT_BWD(5, 3), SWIT_BWD(5, 4), SWIT_BWD(6, 3),
     SWIT_BWD(7, 3), SWIT_BWD(8, 3),
 };
 #undef SWIT_BWD
 
-size_t bwd_lds_bytes(const rk::Cfg &c, int NI, int layers) {
-    return sizeof(float) * (rk::bwd_edge_floats(c.W, c.R) + 2 * (size_t)rk::bwd_set_floats(c.W, c.C, c.R, NI, layers));
+// Most receivers (of `cells`, all shots) in one window's own columns.
+int bwd_window_receivers(const swit_plan *pl, const rk::Cfg &c) {
+    const Dims &d = pl->d;
+    std::vector<int> n(c.P);
+    int most = 0;
+    for (int s = 0; s < pl->ns; ++s) {
+        std::fill(n.begin(), n.end(), 0);
+        for (int r = 0; r < pl->geo_h[s].ng; ++r) {
+            const int x = pl->rec_cells_inj[(size_t)s * d.ngmax + r] / d.ld + 1;
+            const int j = c.P == 1 ? 0 : std::min(c.P - 1, std::max(0, x - 1 - rk::kH) / (c.W * c.C - 2 * rk::kH));
+            most = std::max(most, ++n[j]);
+        }
+    }
+    return most;
+}
+
+// Most side layers (0 to 2) of the strips in one window.
+int bwd_window_sides(const Dims &d, const rk::Cfg &c) {
+    int most = 0;
+    for (int j = 0; j < c.P; ++j) {
+        const int a = rk::window_x(c.W, c.C, j) - d.npml, b = a + c.W * c.C;       // interior columns a .. b - 1
+        most = std::max(most, (a <= 2 && b > 1) + (a <= d.nx && b > d.nx - 1));
+    }
+    return most;
+}
+
+size_t bwd_lds_bytes(const rk::Cfg &c, int NI, int layers, int ring, int ninj, int sides) {
+    return sizeof(float) * (rk::bwd_edge_floats(c.W, c.R) + 2 * (size_t)rk::bwd_set_floats(c.W, c.C, c.R, NI, layers) +
+                            (size_t)ring * rk::bwd_step_floats(c.W, c.C, c.R, ninj, sides));
 }
 
 // Rows of the adjoint that a step changes or reads past its tile: 2 .. nzp-2.  z0 <= 2 puts
@@ -1435,14 +1464,16 @@ void bwd_rows(const Dims &d, int R, int *z0, int *need) {
     *need = d.nzp - 2 - *z0 + 1;
 }
 
-bool choose_bwd(const Dims &d, int ns, int ncu, int NI, int layers, rk::Cfg *best) {
+struct BwdRing {
+    int ring, ninj, sides;
+};
+
+// As choose_fwd.  ring: the values of up to 15 steps fetched at once, fewer where the LDS is full
+// (a fetch waits about 2 us).
+bool choose_bwd(const swit_plan *pl, int ncu, int NI, int layers, int R, int z0, rk::Cfg *best, BwdRing *best_ring) {
+    const Dims &d = pl->d;
+    const int ns = pl->ns;
     double best_t = 1e30;
-    int R = 2, z0 = 0, need = 0;
-    for (;; ++R) {
-        bwd_rows(d, R, &z0, &need);
-        if (need <= 64 * R) break;
-        if (R > 8) return false;
-    }
     for (const BwdKernel &kn : kBwdKernels) {
         if (kn.R != R) continue;
         for (int W = 1; W <= 8; ++W) {
@@ -1455,16 +1486,19 @@ bool choose_bwd(const Dims &d, int ns, int ncu, int NI, int layers, rk::Cfg *bes
             c.P = d.nxp <= cols ? 1 : cols > 2 * rk::kH ? cdiv(d.nxp - 2 * rk::kH, cols - 2 * rk::kH) : 0;
             // halo columns in one wave, three own columns at least
             if (c.P < 1 || (c.P > 1 && (c.C < rk::kH || cols < 3 * rk::kH))) continue;
-            const size_t lds = bwd_lds_bytes(c, NI, layers);
+            BwdRing q{16, bwd_window_receivers(pl, c), bwd_window_sides(d, c)};
+            while (q.ring > 2 && bwd_lds_bytes(c, NI, layers, q.ring, q.ninj, q.sides) + 1024 > kCuLds) q.ring /= 2;
+            const size_t lds = bwd_lds_bytes(c, NI, layers, q.ring, q.ninj, q.sides);
             if (lds + 1024 > kCuLds) continue;
             const int per_cu = std::min(8 / W, (int)(kCuLds / (lds + 1024)));
             if (c.P > max_windows(per_cu, ncu)) continue;
             const int rounds = cdiv(ns, std::min(ns, per_cu * ncu / c.P));
             c.G = cdiv(ns, rounds);
-            const double t = rounds * resident_step_us(W * cdiv(c.G * c.P, ncu), 80.0 * c.C * R, c.P > 1);
+            const double t = rounds * (resident_step_us(W * cdiv(c.G * c.P, ncu), 80.0 * c.C * R, c.P > 1 ? 3.4 : 2.0) + 2.0 / (q.ring - 1));
             if (t < best_t) {
                 best_t = t;
                 *best = c;
+                *best_ring = q;
             }
         }
     }
@@ -1518,7 +1552,7 @@ bool choose_ex(const Dims &d, int ns, int ncu, int NI, int layers, rk::Cfg *best
             if (c.P > max_windows(per_cu, ncu)) continue;
             const int rounds = cdiv(ns, std::min(ns, per_cu * ncu / c.P));
             c.G = cdiv(ns, rounds);
-            const double t = rounds * resident_step_us(W * cdiv(c.G * c.P, ncu), 60.0 * c.C * R, c.P > 1);
+            const double t = rounds * resident_step_us(W * cdiv(c.G * c.P, ncu), 60.0 * c.C * R, c.P > 1 ? 1.45 : 0.9);
             if (t < best_t) {
                 best_t = t;
                 *best = c;
@@ -1615,13 +1649,19 @@ static int resident_init_bwd(swit_plan *pl, int ncu) {
             layers = std::max(layers, (int)m);
         }
     }
-    if (layers > 2 || !choose_bwd(d, pl->ns, ncu, 8, layers, &c)) return SWIT_OK;
+    int z0 = 0, need = 0, R = 2;
+    for (;; ++R) {
+        bwd_rows(d, R, &z0, &need);
+        if (need <= 64 * R) break;
+        if (R > 8) return SWIT_OK;
+    }
     unsigned long long mask = 0;
     for (int s = 0; s < pl->ns; ++s)
         for (int r = 0; r < pl->geo_h[s].ng; ++r)
-            mask |= 1ull << ((pl->rec_cells_inj[(size_t)s * d.ngmax + r] % d.ld + 1 - c.z0) / c.R);
+            mask |= 1ull << ((pl->rec_cells_inj[(size_t)s * d.ngmax + r] % d.ld + 1 - z0) / R);
     const int NI = __builtin_popcountll(mask);
-    if (NI > 8) return SWIT_OK;
+    BwdRing ring{};
+    if (layers > 2 || NI > 8 || !choose_bwd(pl, ncu, NI, layers, R, z0, &c, &ring)) return SWIT_OK;
     const int T = c.W * 64, WC = c.W * c.C;
     std::vector<int> itab((size_t)pl->ns * c.P * 2 * T, -1), ibase((size_t)pl->ns * c.P, 0),
         imap((size_t)pl->ns * d.ngmax, -1);
@@ -1660,7 +1700,10 @@ static int resident_init_bwd(swit_plan *pl, int ncu) {
     rs.bc = c;
     rs.b_imask = mask;
     rs.b_layers = layers;
-    rs.b_lds = bwd_lds_bytes(c, NI, layers);
+    rs.b_ring = ring.ring;
+    rs.b_ninj = ring.ninj;
+    rs.b_sides = ring.sides;
+    rs.b_lds = bwd_lds_bytes(c, NI, layers, ring.ring, ring.ninj, ring.sides);
     HIP_TRY(hipFuncSetAttribute((const void *)find_bwd(c.R, c.C)->fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)rs.b_lds));
     rs.b_ncol = d.nxp + WC;
@@ -1873,6 +1916,9 @@ static int resident_backward_steps(swit_plan *pl, const float *src, const float 
     a.ibase = rs.b_ibase;
     a.imask = rs.b_imask;
     a.layers = rs.b_layers;
+    a.ring = rs.b_ring;
+    a.ninj = rs.b_ninj;
+    a.sides = rs.b_sides;
     a.acc = rs.b_acc;
     a.msg = rs.msg;
     a.ctl = rs.ctl;
