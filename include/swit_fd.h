@@ -346,7 +346,9 @@ int swit_process_work(const swit_process_params *p, size_t *bytes);
  *            first break from the data (the first sample above 0.1 % of the trace
  *            maximum, preprocess.py:140-142, 203-209) and shifts it by
  *            ceil(|mute_late_window| / dt);
- *   work:    device memory of swit_process_work bytes.
+ *   work:    device memory of swit_process_work bytes.  That holds 16384 traces of the
+ *            filter's forward output (8 (nt + 6 filter_taps) bytes each); with more, up to
+ *            65536, more are filtered at once.
  * The filter needs nt > 3 * filter_taps (scipy's padding). */
 int swit_process(const swit_process_params *p, const float *offsets, const double *mute_win, const double *taper,
                  const int32_t *picks, float *data, void *work, size_t work_bytes, hipStream_t stream);

