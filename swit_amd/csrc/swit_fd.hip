@@ -2930,62 +2930,49 @@ int precond_run(const swit_precond *p, const float *grad, const float *forw, con
     const int smax = precond_spans(p, &sill);
     double *A = static_cast<double *>(work), *B = A + n, *C = B + n, *T = C + n;
     double *f_ill = T + n, *f_grad = f_ill + (2 * smax + 1), *f_tap = f_grad + (2 * smax + 1);
-    double *M = f_tap + (2 * smax + 1);                // maxima: forw, back, precond, taper, |grad|
-    const dim3 b2(256), g2(cdiv(nz, 256), nx);
-    const int ge = (int)std::min<size_t>(cdiv((int)std::min<size_t>(n, (size_t)1 << 30), 256), 2048);
-    // smooth2d of the field in X (in place through T), rows z0.. nz-1
-    auto smooth = [&](double *X, int z0, int span, const double *f) -> int {
-        const dim3 g(cdiv(nz - z0, 256), nx);
-        hipLaunchKernelGGL(pc::k_smooth_z, g, b2, 0, stream, nx, nz, z0, span, f, X, T);
-        hipLaunchKernelGGL(pc::k_smooth_x, g, b2, 0, stream, nx, nz, z0, span, f, T, X);
-        LAUNCH_CHECK();
-        return SWIT_OK;
+    pc::u64 *M = reinterpret_cast<pc::u64 *>(f_tap + (2 * smax + 1));
+    const dim3 blk(pc::kT), ge((unsigned)std::min<size_t>((n + pc::kT - 1) / pc::kT, 512));
+    // taper (postprocess.py:56-58, 88-111): marine zeroes the rows above the mute, land damps
+    // them with a smoothed Hamming ramp
+    const int kind = p->grad_mute > 0 ? (p->marine ? 1 : 2) : 0;
+    const int z0 = p->marine ? p->grad_mute : 0;       // gradient smoothing: below the mute for marine data
+    const bool smooth = p->grad_smooth > 0 && z0 < nz;
+    auto pass_z = [&](const pc::Passes &ps, int count, int z) {
+        hipLaunchKernelGGL(pc::k_smooth_z, dim3(cdiv(nz - z, 64), cdiv(nx, pc::kT / 64), count), blk, 0, stream, nx, nz, ps);
     };
-    hipLaunchKernelGGL(pc::k_weights, dim3(1), dim3(1), 0, stream, sill, f_ill);
-    // illumination preconditioner (postprocess.py:62-75)
-    hipLaunchKernelGGL(pc::k_to_double, dim3(ge), dim3(256), 0, stream, n, forw, A);
-    hipLaunchKernelGGL(pc::k_to_double, dim3(ge), dim3(256), 0, stream, n, back, B);
+    auto pass_x = [&](const pc::Passes &ps, int count) {
+        hipLaunchKernelGGL(pc::k_smooth_x, dim3(cdiv(nz, 64), cdiv(nx, pc::kT / 64 * pc::kCols), count), blk, 0, stream, nx,
+                           nz, ps);
+    };
+    const pc::Weights w{{sill, p->grad_smooth, p->grad_mute / 2}, {f_ill, f_grad, f_tap}};
+    hipLaunchKernelGGL(pc::k_weights, dim3(3), blk, 0, stream, w, M);
+    // illumination preconditioner (postprocess.py:62-75): the fields through T and C to A and B;
+    // the land taper's column stands in out for a while
+    pc::Passes z{}, x{};
+    z.p[0] = pc::Pass{nullptr, forw, 0, T, f_ill, sill, 0, nullptr, 0, nullptr};
+    z.p[1] = pc::Pass{nullptr, back, 0, C, f_ill, sill, 0, nullptr, 0, nullptr};
+    z.p[2] = pc::Pass{nullptr, nullptr, p->grad_mute, out, f_tap, p->grad_mute / 2, 0, nullptr, 0, nullptr};
+    pass_z(z, kind == 2 ? 3 : 2, 0);
+    x.p[0] = pc::Pass{T, nullptr, 0, A, f_ill, sill, 0, M + pc::kMaxForw, 0, nullptr};
+    x.p[1] = pc::Pass{C, nullptr, 0, B, f_ill, sill, 0, M + pc::kMaxBack, 0, nullptr};
+    pass_x(x, 2);
     LAUNCH_CHECK();
-    TRY(smooth(A, 0, sill, f_ill));
-    TRY(smooth(B, 0, sill, f_ill));
-    hipLaunchKernelGGL(pc::k_max, dim3(1), dim3(pc::kMaxThreads), 0, stream, n, A, 0, M);
-    hipLaunchKernelGGL(pc::k_max, dim3(1), dim3(pc::kMaxThreads), 0, stream, n, B, 0, M + 1);
-    hipLaunchKernelGGL(pc::k_precond_sum, dim3(ge), dim3(256), 0, stream, n, A, B, M, C);
-    hipLaunchKernelGGL(pc::k_max, dim3(1), dim3(pc::kMaxThreads), 0, stream, n, C, 0, M + 2);
-    LAUNCH_CHECK();
-    // taper (postprocess.py:56-58, 88-111): marine zeroes the rows above the mute, land
-    // damps them with a smoothed Hamming ramp
-    int kind = 0;
-    if (p->grad_mute > 0) {
-        if (p->marine) {
-            kind = 1;
-        } else {
-            kind = 2;
-            const int ts = p->grad_mute;
-            hipLaunchKernelGGL(pc::k_weights, dim3(1), dim3(1), 0, stream, ts / 2, f_tap);
-            hipLaunchKernelGGL(pc::k_taper0, g2, b2, 0, stream, nx, nz, ts, A);
-            LAUNCH_CHECK();
-            TRY(smooth(A, 0, ts / 2, f_tap));
-            hipLaunchKernelGGL(pc::k_max, dim3(1), dim3(pc::kMaxThreads), 0, stream, n, A, 0, M + 3);
-            hipLaunchKernelGGL(pc::k_taper_land, dim3(ge), dim3(256), 0, stream, n, (double)p->grad_thred, M + 3, A);
-            LAUNCH_CHECK();
-        }
+    hipLaunchKernelGGL(pc::k_precond_sum, ge, blk, 0, stream, n, A, B, M, C);
+    if (kind == 2) {
+        x.p[0] = pc::Pass{out, nullptr, p->grad_mute, A, f_tap, p->grad_mute / 2, 0, M + pc::kMaxTaper, 0, nullptr};
+        pass_x(x, 1);
     }
-    hipLaunchKernelGGL(pc::k_apply, g2, b2, 0, stream, nx, nz, kind, p->grad_mute, grad, A, C, M, out);
+    hipLaunchKernelGGL(pc::k_apply, ge, blk, 0, stream, nz, n, kind, p->grad_mute, (double)p->grad_thred, smooth ? 0 : 1,
+                       grad, A, C, mask, M, out);
     LAUNCH_CHECK();
-    // gradient smoothing (postprocess.py:77-83): below the mute for marine data
-    if (p->grad_smooth > 0) {
-        const int z0 = p->marine ? p->grad_mute : 0;
-        hipLaunchKernelGGL(pc::k_weights, dim3(1), dim3(1), 0, stream, p->grad_smooth, f_grad);
-        LAUNCH_CHECK();
-        if (z0 < nz) TRY(smooth(out, z0, p->grad_smooth, f_grad));
-    }
-    if (mask) {
-        hipLaunchKernelGGL(pc::k_mul, dim3(ge), dim3(256), 0, stream, n, mask, out);
+    if (smooth) {                                       // postprocess.py:77-83
+        z.p[0] = pc::Pass{out, nullptr, 0, T, f_grad, p->grad_smooth, z0, nullptr, 0, nullptr};
+        x.p[0] = pc::Pass{T, nullptr, 0, out, f_grad, p->grad_smooth, z0, M + pc::kMaxOut, 1, mask};
+        pass_z(z, 1, z0);
+        pass_x(x, 1);
         LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(pc::k_max, dim3(1), dim3(pc::kMaxThreads), 0, stream, n, out, 1, M + 4);
-    hipLaunchKernelGGL(pc::k_scale, dim3(ge), dim3(256), 0, stream, n, p->vpmax, M + 4, out);
+    hipLaunchKernelGGL(pc::k_scale, ge, blk, 0, stream, n, p->vpmax, M, out);
     LAUNCH_CHECK();
     return SWIT_OK;
 }

@@ -53,3 +53,26 @@ def test_device_grad_precond_matches_numpy(nx, nz, marine, mute, thred, smooth, 
     land_taper = not marine and mute > 0
     assert err <= (1e-8 if land_taper else 1e-12)
     assert np.abs(got).max() == pytest.approx(3500.0, rel=1e-15)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,nz,marine,mute,thred,smooth,use_mask", [
+    (4, 65, True, 3, 0.0, 1, False),         # fewer columns than a wave takes; 64 rows and one
+    (17, 64, False, 9, 0.02, 0, True),       # no smoothing pass: the mask rides on the product
+    (70, 131, True, 67, 0.0, 6, True),       # smoothing from a row inside the second 64
+    (140, 150, True, 2, 0.0, 128, False),    # the largest staged span
+    (140, 150, True, 2, 0.0, 129, False),    # past it
+    (50, 60, True, 60, 0.0, 3, False),       # everything muted: no row is left to smooth
+])
+def test_edges_of_the_passes(nx, nz, marine, mute, thred, smooth, use_mask):
+    from swit_amd.engine import grad_precond
+    grad, forw, back = _case(nx, nz, nx + nz + mute)
+    mask = np.random.default_rng(3).random((nx, nz)) if use_mask else None
+    if marine and mute >= nz:
+        got = grad_precond(grad, forw, back, 3500.0, marine, mute, thred, smooth, mask).cpu().numpy()
+        assert np.isnan(got).all()           # 0 * (vpmax / max 0)
+        return
+    ref = P.precondition(grad, forw, back, 3500.0, marine, mute, thred, smooth, mask).ravel()
+    got = grad_precond(grad, forw, back, 3500.0, marine, mute, thred, smooth, mask).cpu().numpy().ravel()
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert err <= (1e-8 if not marine and mute > 0 else 1e-12)
