@@ -12,6 +12,7 @@
 #include <mutex>
 #include <utility>
 #include <set>
+#include <type_traits>
 #include <vector>
 
 #include "swit_fd.h"
