@@ -177,6 +177,10 @@ int swit_plan_autotune(swit_plan *plan, int steps, int *choice, double *us, hipS
  * back in between); this call waits for the loops recorded so far to finish. */
 int swit_plan_kernel_time(swit_plan *plan, int which, double *total_ms, int64_t *launches);
 
+/* 1 if the plan's forward (which = 0), backward (1) or exact (2) loops outside a stream
+ * capture run resident in registers (SWIT_OPT_RESIDENT), 0 if one launch per step or two. */
+int swit_plan_resident(const swit_plan *plan, int which);
+
 /* The saved boundary strips of the last strip-saving forward, decoded to FP32:
  * out[ns][nt][S] (device), S = 9nx+6nz, row it-1 = step it, the layout of the
  * reference's boundary.bin per shot (fdcore.f90:130-159,166-176).
@@ -238,8 +242,8 @@ int swit_group_adjoint(swit_group *group, const float *const *src, const float *
                        hipStream_t stream);
 int swit_group_destroy(swit_group *group);
 
-/* A whole gradient of every plan in one call: each plan runs the strip-saving forward (seismograms to seis), the misfit and adjoint source `kind`
- * (SWIT_MISFIT_*) against obs, exactly as swit_misfit computes them (adjoint source to
+/* A whole gradient of every plan in one call: each plan runs the strip-saving forward
+ * (seismograms to seis), the misfit and adjoint source `kind` (SWIT_MISFIT_*) against obs, exactly as swit_misfit computes them (adjoint source to
  * adj, per-trace misfits to work, their sum to misfit), and the adjoint (grad,
  * illum_forw, illum_back).  Each plan's results equal swit_forward, swit_misfit and
  * swit_adjoint run one after the other.  Per plan: obs, seis, adj [ns][ngmax][nt]; work

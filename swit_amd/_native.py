@@ -47,6 +47,7 @@ EXPORTS = (
     "swit_group_gradient",
     "swit_plan_set_option",
     "swit_plan_kernel_time",
+    "swit_plan_resident",
     "swit_grad_precond_work",
     "swit_grad_precond",
     "swit_grad_precond_noalloc",
@@ -190,6 +191,8 @@ def load(path: str | None = None):
     L.swit_plan_kernel_time.argtypes = [vp, ctypes.c_int, ctypes.POINTER(ctypes.c_double),
                                         ctypes.POINTER(ctypes.c_int64)]
     L.swit_plan_kernel_time.restype = ctypes.c_int
+    L.swit_plan_resident.argtypes = [vp, ctypes.c_int]
+    L.swit_plan_resident.restype = ctypes.c_int
     if path is None:
         _lib = L
     return L

@@ -2291,6 +2291,12 @@ extern "C" int swit_plan_set_option(swit_plan *pl, int option, int value) {
     }
 }
 
+extern "C" int swit_plan_resident(const swit_plan *pl, int which) {
+    if (!pl) return 0;
+    const ResidentState &rs = pl->res;
+    return which == 0 ? rs.fwd && rs.use_fwd : which == 1 ? rs.bwd && rs.use_bwd : which == 2 ? rs.ex && rs.use_exact : 0;
+}
+
 extern "C" int swit_plan_kernel_time(swit_plan *pl, int which, double *total_ms, int64_t *launches) {
     g_err[0] = 0;
     if (!pl || which < 0 || which > 1 || !total_ms || !launches) return set_err(SWIT_EINVAL, "bad arguments");
@@ -2375,8 +2381,9 @@ static int group_capture(swit_group *gr, int which, int save, hipGraphExec_t *ex
 
 // Whether every plan of the group takes the resident loops in the given directions.  They
 // then run one after the other: each fills the chip for its whole job.  501x171x2500 with 22
-// shots, 481x121x2000 with 21 and 300x102x1500 with 21, forward, misfit and adjoint: 147 ms, on
-// concurrent streams 149 to 179 ms, as one graph of the step kernels 329 ms.
+// shots, 481x121x2000 with 21 and 300x102x1500 with 21, forward, misfit and adjoint: 119 ms, as
+// one graph of the step kernels 329 ms (with an earlier reverse loop 147 ms one after the other,
+// 149 to 179 ms on concurrent streams).
 static int group_resident(swit_group *gr, bool fwd, bool bwd, hipStream_t stream, bool *yes) {
     for (swit_plan *pl : gr->plans) {
         const ResidentState &rs = pl->res;

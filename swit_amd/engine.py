@@ -119,7 +119,10 @@ class Plan:
     def set_option(self, option, value):
         """option: 'graph' | 'profile' | 'fwd_group' | 'fwd_colgroup' | 'bwd_colgroup' |
         'bwd_steps' | 'bwd_tile_x' | 'bwd_balance' | 'exact_fused' | 'streams' | 'resident'
-        (batched path).  'streams' 2 runs the two halves of the shots on two streams; 'bwd_balance'
+        (batched path).  'resident' 1 (the default) keeps the wavefields in registers, one launch
+        for many steps, where the plan allows it; an option of a direction's step kernels selects
+        these for it.  'streams' 2 runs the two halves of the shots on two streams (step kernels;
+        a resident loop takes all shots); 'bwd_balance'
         splits the one-step backward kernel's work over the XCDs by estimated cost (1, the
         default) or by item count (0).  None of them changes results."""
         code = {"graph": _native.SWIT_OPT_GRAPH, "profile": _native.SWIT_OPT_PROFILE,
@@ -135,7 +138,8 @@ class Plan:
     def autotune(self, steps=20):
         """Time the batched step kernels for every candidate forward shots-per-workgroup
         and column-group order (backward: steps per launch, the one-step kernel's tile
-        width and column-group order) and keep the fastest.  Invalidates saved strips.
+        width and column-group order), then the resident loops, and keep the fastest.  Invalidates
+        saved strips.
         Returns {'fwd_group', 'fwd_colgroup', 'bwd_colgroup', 'bwd_steps', 'bwd_tile_x',
         'bwd_balance', 'fwd_us', 'bwd_us'} (times per time step)."""
         choice = (ctypes.c_int * 6)()
@@ -155,6 +159,10 @@ class Plan:
         _native.check(self._lib.swit_plan_kernel_time(self._h, {"forward": 0, "backward": 1}[which],
                                                       ctypes.byref(ms), ctypes.byref(n)))
         return ms.value, n.value
+
+    def resident(self, which):
+        """Whether the 'forward', 'backward' or 'exact' time loop runs resident in registers."""
+        return bool(self._lib.swit_plan_resident(self._h, {"forward": 0, "backward": 1, "exact": 2}[which]))
 
     # -- jobs ---------------------------------------------------------------------
     def set_model(self, vp, rho):
@@ -324,8 +332,10 @@ class Lanes:
     """The shots of one job split into `lanes` batched plans (contiguous shot ranges),
     each running its whole job on a stream of its own.  The lanes' step kernels run side
     by side and fill each other's idle workgroup slots: at 481x141x4000 with 49 shots a
-    gradient on two lanes runs in 473-480 ms against 511-514 ms for one plan (three or
-    four lanes, or a second lane started after the first's forward, were slower).  Gradients
+    gradient by step kernels on two lanes runs in 473-480 ms against 511-514 ms for one plan
+    (three or four lanes, or a second lane started after the first's forward, were slower).
+    Resident time loops fill the chip by themselves: two lanes take 177 ms, one plan 147 ms.
+    Gradients
     and illuminations are the lanes' FP64 sums added in lane order, so they equal the
     one-plan result to FP64 rounding.  Plan keyword arguments (strips, ...) apply to
     every lane."""
