@@ -202,23 +202,22 @@ struct FftFactors {
     int radix[kFftMaxStages];
 };
 
-// Threads per workgroup: 512, so that two workgroups of up to 4096 points share a CU
-// (each barrier of one overlaps the other's work).
-template <int NMAX>
-constexpr int fft_threads() { return 512; }
-
-template <int NMAX>
+// Threads per workgroup T: 512, so that two workgroups of up to 4096 points share a CU (each
+// barrier of one overlaps the other's work).  Up to 2048 points also 256, four workgroups a CU:
+// a radix-10 stage has 200 butterflies at 2000 points, so half of 512 threads wait.  23569
+// traces of 2000 samples: envelope 1298 us with 512 threads, 999 with 256 (traveltime 920 and
+// 675), 603 traces 56 and 51; but 100 traces, which leave compute units idle, 26 and 30, and 603
+// of 2003 samples (a prime: a gather stage) 3568 and 4120 (launch_misfit has the rule).
+template <int NMAX, int T>
 struct FftLds {
-    static constexpr int T = fft_threads<NMAX>();
     double2 x[NMAX];
     double2 ta[kTwA], tb[kTwB];      // exp(-2 pi i a kTwB / n), exp(-2 pi i b / n)
     double sh[T / 64];
     int ish[T / 64];
 };
 
-template <int NMAX>
-__device__ void fft_twiddles(FftLds<NMAX> &L, const FftFactors &f) {
-    constexpr int T = fft_threads<NMAX>();
+template <int NMAX, int T>
+__device__ void fft_twiddles(FftLds<NMAX, T> &L, const FftFactors &f) {
     const int na = (f.n + kTwB - 1) / kTwB;
     for (int i = threadIdx.x; i < na + kTwB; i += T) {
         const int e = i < na ? i * kTwB : i - na;
@@ -230,8 +229,8 @@ __device__ void fft_twiddles(FftLds<NMAX> &L, const FftFactors &f) {
 }
 
 // W^e (conjugated for the inverse), 0 <= e < n
-template <int NMAX, bool INV>
-__device__ __forceinline__ double2 fft_w(const FftLds<NMAX> &L, int e) {
+template <int NMAX, int T, bool INV>
+__device__ __forceinline__ double2 fft_w(const FftLds<NMAX, T> &L, int e) {
     const double2 a = L.ta[e >> kTwShift], b = L.tb[e & (kTwB - 1)];
     const double re = a.x * b.x - a.y * b.y, im = a.x * b.y + a.y * b.x;
     return make_double2(re, INV ? -im : im);
@@ -343,9 +342,8 @@ template <> __device__ __forceinline__ void dft_small<10, true>(const double2 *z
 
 // One butterfly stage of radix R (2..5, 10), in place: all reads, barrier, all writes,
 // barrier.
-template <int NMAX, bool INV, int R>
-__device__ void fft_stage_bfly(FftLds<NMAX> &L, int n, int ns) {
-    constexpr int T = fft_threads<NMAX>();
+template <int NMAX, int T, bool INV, int R>
+__device__ void fft_stage_bfly(FftLds<NMAX, T> &L, int n, int ns) {
     constexpr int BPT = (NMAX / R + T - 1) / T;      // butterflies per thread
     const int nb = n / R, mult = nb / ns;            // n / (ns R)
     double2 y[BPT][R];
@@ -359,7 +357,7 @@ __device__ void fft_stage_bfly(FftLds<NMAX> &L, int n, int ns) {
             o0[k] = (b - jm) * R + jm;
             // twiddle powers w^q from w = W^(jm n/(ns R)) by products
             double2 z[R];
-            const double2 w1 = fft_w<NMAX, INV>(L, jm * mult);
+            const double2 w1 = fft_w<NMAX, T, INV>(L, jm * mult);
             double2 wq = w1;
             z[0] = L.x[b];
 #pragma unroll
@@ -383,9 +381,9 @@ __device__ void fft_stage_bfly(FftLds<NMAX> &L, int n, int ns) {
 
 // One stage of any radix as a gather over outputs, in place (reads, barrier, writes,
 // barrier).
-template <int NMAX, bool INV>
-__device__ void fft_stage_gather(FftLds<NMAX> &L, int n, int R, int ns) {
-    constexpr int T = fft_threads<NMAX>(), E = (NMAX + T - 1) / T;
+template <int NMAX, int T, bool INV>
+__device__ void fft_stage_gather(FftLds<NMAX, T> &L, int n, int R, int ns) {
+    constexpr int E = (NMAX + T - 1) / T;
     const int nr = n / R, span = ns * R, mult = n / span;
     double2 acc[E];
 #pragma unroll
@@ -395,7 +393,7 @@ __device__ void fft_stage_gather(FftLds<NMAX> &L, int n, int R, int ns) {
         if (o < n) {
             const int jm = o % ns, q = (o / ns) % R;
             const int j = (o / span) * ns + jm;
-            const double2 w1 = fft_w<NMAX, INV>(L, (jm + q * ns) * mult);     // step < n
+            const double2 w1 = fft_w<NMAX, T, INV>(L, (jm + q * ns) * mult);     // step < n
             double wr = 1.0, wi = 0.0;
             for (int r = 0; r < R; ++r) {
                 const double2 v = L.x[j + r * nr];
@@ -419,20 +417,20 @@ __device__ void fft_stage_gather(FftLds<NMAX> &L, int n, int R, int ns) {
 
 // In-place DFT of L.x[0..n) (INV: inverse without the 1/n factor).  Begins and ends
 // with a barrier.
-template <int NMAX, bool INV>
-__device__ void fft_lds(FftLds<NMAX> &L, const FftFactors &f) {
+template <int NMAX, int T, bool INV>
+__device__ void fft_lds(FftLds<NMAX, T> &L, const FftFactors &f) {
     const int n = f.n;
     int ns = 1;
     __syncthreads();
     for (int st = 0; st < f.nst; ++st) {
         const int R = f.radix[st];
         switch (R) {
-        case 2: fft_stage_bfly<NMAX, INV, 2>(L, n, ns); break;
-        case 3: fft_stage_bfly<NMAX, INV, 3>(L, n, ns); break;
-        case 4: fft_stage_bfly<NMAX, INV, 4>(L, n, ns); break;
-        case 5: fft_stage_bfly<NMAX, INV, 5>(L, n, ns); break;
-        case 10: fft_stage_bfly<NMAX, INV, 10>(L, n, ns); break;
-        default: fft_stage_gather<NMAX, INV>(L, n, R, ns); break;
+        case 2: fft_stage_bfly<NMAX, T, INV, 2>(L, n, ns); break;
+        case 3: fft_stage_bfly<NMAX, T, INV, 3>(L, n, ns); break;
+        case 4: fft_stage_bfly<NMAX, T, INV, 4>(L, n, ns); break;
+        case 5: fft_stage_bfly<NMAX, T, INV, 5>(L, n, ns); break;
+        case 10: fft_stage_bfly<NMAX, T, INV, 10>(L, n, ns); break;
+        default: fft_stage_gather<NMAX, T, INV>(L, n, R, ns); break;
         }
         ns *= R;
     }
@@ -441,9 +439,8 @@ __device__ void fft_lds(FftLds<NMAX> &L, const FftFactors &f) {
 // x <- -i sgn(k) x, sgn as scipy.signal.hilbert's h - 1: 0 at k = 0 (and k = n/2 for
 // even n), +1 below n/2, -1 above.  After the inverse transform, the real and
 // imaginary parts are the Hilbert transforms of the two packed real traces.
-template <int NMAX>
-__device__ void hilbert_multiplier(FftLds<NMAX> &L, int n) {
-    constexpr int T = fft_threads<NMAX>();
+template <int NMAX, int T>
+__device__ void hilbert_multiplier(FftLds<NMAX, T> &L, int n) {
     for (int k = threadIdx.x; k < n; k += T) {
         const double sg = (k == 0 || 2 * k == n) ? 0.0 : (2 * k < n ? 1.0 : -1.0);
         const double2 v = L.x[k];
@@ -452,15 +449,15 @@ __device__ void hilbert_multiplier(FftLds<NMAX> &L, int n) {
 }
 
 // Envelope misfit (power 2) of one trace per workgroup.
-template <int NMAX>
-__global__ __launch_bounds__(fft_threads<NMAX>())
+template <int NMAX, int T>
+__global__ __launch_bounds__(T)
 __attribute__((amdgpu_waves_per_eu(NMAX <= 4096 ? 4 : 1, 8))) void k_misfit_envelope(FftFactors f, float dt,
                                                                  const float *__restrict__ obs,
                                                                  const float *__restrict__ syn,
                                                                  float *__restrict__ adj,
                                                                  double *__restrict__ tmis) {
-    constexpr int T = fft_threads<NMAX>(), E = (NMAX + T - 1) / T;
-    __shared__ FftLds<NMAX> L;
+    constexpr int E = (NMAX + T - 1) / T;
+    __shared__ FftLds<NMAX, T> L;
     const int n = f.n;
     const size_t base = (size_t)blockIdx.x * n;
     const float *o = obs + base, *s = syn + base;
@@ -480,9 +477,9 @@ __attribute__((amdgpu_waves_per_eu(NMAX <= 4096 ? 4 : 1, 8))) void k_misfit_enve
         if (threadIdx.x == 0) tmis[blockIdx.x] = 0.0;
         return;
     }
-    fft_lds<NMAX, false>(L, f);
+    fft_lds<NMAX, T, false>(L, f);
     hilbert_multiplier(L, n);
-    fft_lds<NMAX, true>(L, f);
+    fft_lds<NMAX, T, true>(L, f);
     const double inv_n = 1.0 / n;
     double part[E];
     double r2 = 0.0;
@@ -501,9 +498,9 @@ __attribute__((amdgpu_waves_per_eu(NMAX <= 4096 ? 4 : 1, 8))) void k_misfit_enve
         }
     }
     r2 = block_sum<T>(r2, L.sh);
-    fft_lds<NMAX, false>(L, f);
+    fft_lds<NMAX, T, false>(L, f);
     hilbert_multiplier(L, n);
-    fft_lds<NMAX, true>(L, f);
+    fft_lds<NMAX, T, true>(L, f);
 #pragma unroll
     for (int k = 0; k < E; ++k) {
         const int i = threadIdx.x + k * T;
@@ -513,15 +510,15 @@ __attribute__((amdgpu_waves_per_eu(NMAX <= 4096 ? 4 : 1, 8))) void k_misfit_enve
 }
 
 // Cross-correlation traveltime misfit of one trace per workgroup.
-template <int NMAX>
-__global__ __launch_bounds__(fft_threads<NMAX>())
+template <int NMAX, int T>
+__global__ __launch_bounds__(T)
 __attribute__((amdgpu_waves_per_eu(NMAX <= 4096 ? 4 : 1, 8))) void k_misfit_traveltime(FftFactors f, float dt,
                                                                    const float *__restrict__ obs,
                                                                    const float *__restrict__ syn,
                                                                    float *__restrict__ adj,
                                                                    double *__restrict__ tmis) {
-    constexpr int T = fft_threads<NMAX>(), E = (NMAX + T - 1) / T;
-    __shared__ FftLds<NMAX> L;
+    constexpr int E = (NMAX + T - 1) / T;
+    __shared__ FftLds<NMAX, T> L;
     const int n = f.n;
     const size_t base = (size_t)blockIdx.x * n;
     const float *o = obs + base, *s = syn + base;
@@ -549,7 +546,7 @@ __attribute__((amdgpu_waves_per_eu(NMAX <= 4096 ? 4 : 1, 8))) void k_misfit_trav
         if (threadIdx.x == 0) tmis[blockIdx.x] = 0.0;
         return;
     }
-    fft_lds<NMAX, false>(L, f);
+    fft_lds<NMAX, T, false>(L, f);
     // Z = O + i S  ->  P = O * conj(-S), with O = (Z_k + conj Z_-k)/2, S = (Z_k - conj Z_-k)/(2i);
     // P_-k = conj P_k.
     double2 pk[E];
@@ -574,7 +571,7 @@ __attribute__((amdgpu_waves_per_eu(NMAX <= 4096 ? 4 : 1, 8))) void k_misfit_trav
             if (i != 0) L.x[n - i] = make_double2(pk[k].x, -pk[k].y);
         }
     }
-    fft_lds<NMAX, true>(L, f);
+    fft_lds<NMAX, T, true>(L, f);
     // first index of the largest |cc| (numpy argmax)
     double best = -1.0;
     int bi = 0;

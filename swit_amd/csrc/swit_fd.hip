@@ -2554,14 +2554,14 @@ static FftFactors fft_factors(int n) {
     return f;
 }
 
-template <int NMAX>
+template <int NMAX, int T>
 static void launch_fft_misfit(int kind, const FftFactors &f, int ntraces, float dt, const float *obs,
                               const float *syn, float *adj, double *work, hipStream_t stream) {
     if (kind == SWIT_MISFIT_ENVELOPE)
-        hipLaunchKernelGGL(k_misfit_envelope<NMAX>, dim3(ntraces), dim3(fft_threads<NMAX>()), 0, stream, f, dt, obs, syn,
+        hipLaunchKernelGGL((k_misfit_envelope<NMAX, T>), dim3(ntraces), dim3(T), 0, stream, f, dt, obs, syn,
                            adj, work);
     else
-        hipLaunchKernelGGL(k_misfit_traveltime<NMAX>, dim3(ntraces), dim3(fft_threads<NMAX>()), 0, stream, f, dt, obs, syn,
+        hipLaunchKernelGGL((k_misfit_traveltime<NMAX, T>), dim3(ntraces), dim3(T), 0, stream, f, dt, obs, syn,
                            adj, work);
 }
 
@@ -2586,9 +2586,15 @@ static int launch_misfit(int kind, int ntraces, int nt, float dt, const float *o
                            work);
     } else {
         const FftFactors f = fft_factors(nt);
-        if (nt <= 2048) launch_fft_misfit<2048>(kind, f, ntraces, dt, obs, syn, adj, work, stream);
-        else if (nt <= 4096) launch_fft_misfit<4096>(kind, f, ntraces, dt, obs, syn, adj, work, stream);
-        else launch_fft_misfit<kFftMaxN>(kind, f, ntraces, dt, obs, syn, adj, work, stream);
+        // 256 threads a trace where more traces than two per compute unit share the chip and
+        // every stage is a register butterfly (FftLds has both sides' times)
+        bool bfly = true;
+        for (int k = 0; k < f.nst; ++k) bfly = bfly && (f.radix[k] <= 5 || f.radix[k] == 10);
+        if (nt <= 2048 && ntraces > 2 * 256 && bfly)
+            launch_fft_misfit<2048, 256>(kind, f, ntraces, dt, obs, syn, adj, work, stream);
+        else if (nt <= 2048) launch_fft_misfit<2048, 512>(kind, f, ntraces, dt, obs, syn, adj, work, stream);
+        else if (nt <= 4096) launch_fft_misfit<4096, 512>(kind, f, ntraces, dt, obs, syn, adj, work, stream);
+        else launch_fft_misfit<kFftMaxN, 512>(kind, f, ntraces, dt, obs, syn, adj, work, stream);
     }
     LAUNCH_CHECK();
     hipLaunchKernelGGL(k_sum_fixed, dim3(1), dim3(kMisfitThreads), 0, stream, ntraces, work, misfit);

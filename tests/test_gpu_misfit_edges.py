@@ -44,3 +44,27 @@ def test_infinite_sample():
     adj = misfit("Globalcorrelation", torch.from_numpy(obs).cuda(), torch.from_numpy(syn).cuda(), 0.002)[1].cpu().numpy()
     np.testing.assert_array_equal(adj[[0, 2]], clean[[0, 2]])
     assert np.isnan(adj[1, 7]) and np.all(np.delete(adj[1], 7) == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["Envelope", "Traveltime"])
+@pytest.mark.parametrize("nt", [2, 8, 200, 1000, 2000, 2048, 2003, 1001])
+def test_fft_misfits_of_many_traces(nt, kind):
+    """More than 512 traces (256 threads each where every stage is a register butterfly) against
+    the same traces in calls of 100 (512 threads each): the transforms' operations are the same,
+    the FP64 sums over a trace go in another order."""
+    import torch
+    from swit_amd.engine import misfit
+    rng = np.random.default_rng(nt)
+    t = np.arange(nt) * 0.002
+    obs = (np.sin(2 * np.pi * (3.0 + rng.random((700, 1))) * t) + 0.1 * rng.standard_normal((700, nt))).astype(np.float32)
+    syn = np.roll(obs, 3, axis=1) * np.float32(1.2)
+    obs[5] = 0.0
+    o, s = torch.from_numpy(obs).cuda(), torch.from_numpy(syn).cuda()
+    J, adj, per = misfit(kind, o, s, 0.002)
+    parts = [misfit(kind, o[a:a + 100].contiguous(), s[a:a + 100].contiguous(), 0.002) for a in range(0, 700, 100)]
+    want = np.concatenate([p[1].cpu().numpy() for p in parts])
+    np.testing.assert_allclose(adj.cpu().numpy(), want, rtol=0, atol=2e-7 * max(np.abs(want).max(), 1e-30))
+    wper = np.concatenate([p[2].cpu().numpy() for p in parts])
+    np.testing.assert_allclose(per.cpu().numpy(), wper, rtol=1e-12, atol=1e-300)
+    assert float(J) == pytest.approx(wper.sum(), rel=1e-12)
