@@ -369,6 +369,28 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
             if (sv_lds[i] >= 0) q[sv_slot[i]] = sv[sv_lds[i]];
     };
 
+    // HIST: a column's divergence terms of step it.  Few cells a thread (kLate): all of them at the
+    // step's end, where nothing is loaded until they have arrived behind the next pressure phase;
+    // more would not fit the registers, and go out as they are made, which the velocity
+    // coefficients then wait for (loads complete after every earlier store).  161x61, 8 shots:
+    // 2.84 us a step stored at once, 2.52 us late.
+    constexpr bool kLate = HIST && R * C <= 12;
+    auto store_hist = [&](int s, int it, int x, unsigned voff, const float (&dv)[R]) {
+        const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+        const int zr = k->c.z0 + (int)(voff >> 2), nzp = k->d.nzp;
+        if (x < window_os(k->c.W, C, j) || x > window_oe(k->c.W, C, j, k->c.P, k->d.nxp)) return;
+        float *h = k->hist.p + ((size_t)s * k->hist.slots + (it - 1 - k->hist.base)) * (k->d.nxp * k->d.ld) +
+                   (size_t)(x - 1) * k->d.ld;
+        const unsigned o = zr - 1;
+        if (zr + R - 1 <= nzp) {
+            __builtin_memcpy(h + o, dv, sizeof(float) * R);
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (zr + r <= nzp) h[o + r] = dv[r];
+        }
+    };
+
     for (int s = a.s0 + grp; s < a.s0 + a.ns; s += a.c.G) {
         const int isx = a.geo[s].isx, isz = a.geo[s].isz;
         const float *src = a.src + (size_t)s * a.d.nt;
@@ -448,6 +470,7 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
             unsigned voff = voff0;
             opaque_s(x0);
             opaque_v(voff);
+            float hd[kLate ? C : 1][R];
             // ---- p: u of the neighbouring waves' columns x0-2, x0-1 and x0+C ----
             {
                 const ArgPtr<float> fpx = (ArgPtr<float>)fresh_args<FwdArgs>()->fpx + x0;
@@ -477,20 +500,15 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
                     }
 #pragma unroll
                     for (int r = 0; r < R; ++r) pin(p[c][r]);
-                    if (HIST) {
-                        const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
-                        const int x = x0 + c, zr = k->c.z0 + (int)(voff >> 2), nzp = k->d.nzp;
-                        if (x >= window_os(k->c.W, C, j) && x <= window_oe(k->c.W, C, j, k->c.P, k->d.nxp)) {
-                            float *h = k->hist.p + ((size_t)s * k->hist.slots + (it - 1 - k->hist.base)) *
-                                                       (k->d.nxp * k->d.ld) + (size_t)(x - 1) * k->d.ld;
-                            const unsigned o = zr - 1;
-                            if (zr + R - 1 <= nzp) {
-                                __builtin_memcpy(h + o, dv, sizeof(float) * R);
-                            } else {
+                    if constexpr (HIST) {
+                        if constexpr (kLate) {
 #pragma unroll
-                                for (int r = 0; r < R; ++r)
-                                    if (zr + r <= nzp) h[o + r] = dv[r];
+                            for (int r = 0; r < R; ++r) {
+                                hd[c][r] = dv[r];
+                                pin(hd[c][r]);
                             }
+                        } else {
+                            store_hist(s, it, x0 + c, voff, dv);
                         }
                     }
                     __builtin_amdgcn_sched_barrier(0);
@@ -641,6 +659,10 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
             if (edge && exch)
                 recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, fresh_args<FwdArgs>()->ctl, dead, u);
             if (edge) __builtin_amdgcn_s_setprio(0);
+            if constexpr (kLate) {
+#pragma unroll
+                for (int c = 0; c < C; ++c) store_hist(s, it, x0 + c, voff, hd[c]);
+            }
             put_u();
             srcv = fresh_args<FwdArgs>()->d.dt * src_next;
             lds_barrier();
