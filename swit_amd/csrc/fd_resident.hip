@@ -33,7 +33,8 @@
 // consecutive tickets form the group of one shot.  So at any time at most one group of a
 // launch is incomplete, and it waits only for workgroups that are dispatched next; complete
 // groups run to their end.  Several such launches at once hold at most P - 1 waiting
-// workgroups each, far fewer than the chip's slots, so one of them always completes.  Every
+// workgroups each, P at most a quarter of the chip's places, so with up to four at once (the
+// hardware queues of a process) one of them always completes.  Every
 // wait is bounded by the clock all the same: past kWaitTicks a wave stops waiting for good,
 // sets *err, and the job's outputs are overwritten with NaN.
 //
@@ -1306,8 +1307,8 @@ __host__ __device__ inline int ex_set_floats(int W, int C, int R, int NI, int la
 // Bound by vector issue, 34 operations per cell and step and about as many again for shifts,
 // the divergence history (one 4-byte load per cell and step, in flight through the first
 // part) and the exchange.  Forward and reverse of 161x61x1500, 8 shots, whole history: 31.2 ms
-// by the step kernels (a launch each per step), 9.2 ms here; of 301x101, 21 shots, with
-// checkpoints (an additional forward): 81.8 and 19.0 ms.
+// by the step kernels (a launch each per step), 8.5 ms here; of 301x101, 21 shots, with
+// checkpoints (an additional forward): 81.8 and 18.5 ms.
 template <int R, int C>
 __global__ __launch_bounds__(512) void k_ex_resident(ExArgs a) {
     extern __shared__ float lds[];
