@@ -155,6 +155,10 @@ const char *swit_last_error(void);
                                    An option of a direction's step kernels selects these
                                    for it; the autotuner takes the faster.  Calls on a
                                    capturing stream take the step kernels               */
+#define SWIT_OPT_RESIDENT_WAIT 2048  /* ms (default 30000) after which a workgroup of a
+                                   resident loop stops waiting for a neighbour that runs
+                                   (20 times that for one that has no room to start yet);
+                                   its job's outputs are then NaN                       */
 int swit_plan_set_option(swit_plan *plan, int option, int value);
 
 /* Autotuner (no counterpart in the reference): times `steps` back-to-back launches of

@@ -71,6 +71,7 @@ SWIT_OPT_BWD_TILE_X = 128
 SWIT_OPT_STREAMS = 256
 SWIT_OPT_BWD_BALANCE = 512
 SWIT_OPT_RESIDENT = 1024
+SWIT_OPT_RESIDENT_WAIT = 2048
 
 
 class SwitPrecond(ctypes.Structure):

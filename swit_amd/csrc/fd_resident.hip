@@ -35,14 +35,15 @@
 // groups run to their end.  Several such launches at once hold at most P - 1 waiting
 // workgroups each, P at most a quarter of the chip's places, so with up to four at once (the
 // hardware queues of a process) one of them always completes.  Every
-// wait is bounded by the clock all the same: past kWaitTicks a wave stops waiting for good,
-// sets *err, and the job's outputs are overwritten with NaN.
+// wait is bounded by the clock all the same (fd_wait.h): past that a wave stops waiting for
+// good, sets *err, and the job's outputs are overwritten with NaN.
 //
 // Per-cell arithmetic and its order are those of the step kernels: results are the same
 // bits.  Cells outside an update region have K (or B) = 0 and hold zeros, so they need no
 // test: fac * 0 - 0 * d = 0.
 #include "fd_common.h"
 #include "fd_kernels.h"
+#include "fd_wait.h"
 
 namespace swit {
 namespace rk {
@@ -50,7 +51,7 @@ namespace rk {
 typedef unsigned long long u64;
 
 
-constexpr u64 kWaitTicks = 3000000000ull;       // 30 s of the 100 MHz clock
+constexpr u64 kTicksPerMs = 100000ull;          // the 100 MHz clock of wall_clock64
 
 // lane l gets lane l+1's (up) or l-1's (dn) value, 0 past the ends; every lane active
 __device__ __forceinline__ float up1(float v) {
@@ -111,6 +112,7 @@ struct FwdArgs {
     float *end;                 // null or [ns][3][nx][nz]
     u64 *msg;                   // [G P][2 slots][2 sides][3 R][64]
     Ctl *ctl;
+    u64 limit;                  // of a wait, in ticks
 };
 
 // A value the compiler must take as changed: what is computed or loaded from it inside a
@@ -135,10 +137,13 @@ template <int R> __device__ __forceinline__ void send_col(u64 *o, unsigned tag, 
     }
 }
 // N columns' rows out of a message, polled until every word carries the tag (all loads of a
-// round in flight together).  A wave that has waited too long once waits no more.
+// round in flight together).  A wave that has waited too long once waits no more.  group_end:
+// the ticket behind the group's last.
 template <int R, int N>
-__device__ __forceinline__ void recv_cols(const u64 *in, unsigned tag, Ctl *ctl, bool &dead, float (&v)[N][R]) {
-    u64 t0 = 0, q[N][R];
+__device__ __forceinline__ void recv_cols(const u64 *in, unsigned tag, Ctl *ctl, u64 limit, unsigned group_end,
+                                          bool &dead, float (&v)[N][R]) {
+    Wait wait;
+    u64 q[N][R];
     for (;;) {
         unsigned bad = 0;
 #pragma unroll
@@ -149,9 +154,9 @@ __device__ __forceinline__ void recv_cols(const u64 *in, unsigned tag, Ctl *ctl,
                 bad |= (unsigned)(q[n][r] >> 32) ^ tag;
             }
         if (__all(bad == 0) || dead) break;
-        const u64 t = wall_clock64();
-        if (t0 == 0) t0 = t;
-        if (t - t0 > kWaitTicks) {
+        if (wait_over(wall_clock64(), limit, wait, [&] {
+                return __hip_atomic_load(&ctl->ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= group_end;
+            })) {
             dead = true;
             if ((threadIdx.x & 63) == 0) __hip_atomic_store(&ctl->err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             break;
@@ -181,17 +186,18 @@ __device__ __forceinline__ void send_edges(bool has_l, bool has_r, int wave, int
 // Fresh halo columns from the inboxes: positions 0, 1, 2 from each end (C >= 3: one wave).
 template <int R, int C>
 __device__ __forceinline__ void recv_edges(bool has_l, bool has_r, int wave, int W, const u64 *from_l,
-                                           const u64 *from_r, unsigned tag, Ctl *ctl, bool &dead, float (&f)[C][R]) {
+                                           const u64 *from_r, unsigned tag, Ctl *ctl, u64 limit, unsigned group_end,
+                                           bool &dead, float (&f)[C][R]) {
     float v[kH][R];
     if (has_l && wave == 0) {
-        recv_cols<R, kH>(from_l, tag, ctl, dead, v);
+        recv_cols<R, kH>(from_l, tag, ctl, limit, group_end, dead, v);
 #pragma unroll
         for (int h = 0; h < kH; ++h)
 #pragma unroll
             for (int r = 0; r < R; ++r) f[h][r] = v[h][r];
     }
     if (has_r && wave == W - 1) {
-        recv_cols<R, kH>(from_r, tag, ctl, dead, v);
+        recv_cols<R, kH>(from_r, tag, ctl, limit, group_end, dead, v);
 #pragma unroll
         for (int h = 0; h < kH; ++h)
 #pragma unroll
@@ -657,8 +663,10 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
                 }
             }
             // ---- exchange, in: fresh halo columns ----
-            if (edge && exch)
-                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, fresh_args<FwdArgs>()->ctl, dead, u);
+            if (edge && exch) {
+                const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
+                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, k->limit, (grp + 1) * P, dead, u);
+            }
             if (edge) __builtin_amdgcn_s_setprio(0);
             if constexpr (kLate) {
 #pragma unroll
@@ -736,6 +744,7 @@ struct BwdArgs {
     float *acc;                 // [ns][nxp][3][64 R] per-shot accumulators, zero at the start
     u64 *msg;                   // [G P][2 slots][2 sides][2 fields][3 R][64]
     Ctl *ctl;
+    u64 limit;                  // as the forward's
 };
 
 // LDS of the backward: the waves' edge columns of both wavefields (p, then u: with R >= 5 in
@@ -1223,8 +1232,9 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
             if (exch) hand_out(it - 1, i0, i1);
             if (edge && exch) {
                 const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
-                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, dead, pr);
-                recv_edges<R, C>(has_l, has_r, wave, W, box + kMsg / 2, box + kMsg + kMsg / 2, tag, k->ctl, dead, pa);
+                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, k->limit, (grp + 1) * P, dead, pr);
+                recv_edges<R, C>(has_l, has_r, wave, W, box + kMsg / 2, box + kMsg + kMsg / 2, tag, k->ctl, k->limit, (grp + 1) * P,
+                                 dead, pa);
             }
             if (edge) __builtin_amdgcn_s_setprio(0);
             put_p();
@@ -1294,6 +1304,7 @@ struct ExArgs {
     int add;                    // 0: it is zero
     u64 *msg;                   // as the forward's
     Ctl *ctl;
+    u64 limit;
 };
 
 // LDS of the exact reverse loop: the waves' edge columns of q and r, two injection stages.
@@ -1574,8 +1585,10 @@ __global__ __launch_bounds__(512) void k_ex_resident(ExArgs a) {
                 if (i0.x >= 0) f[i0.x] = gn0;
                 if (i1.x >= 0) f[i1.x] = gn1;
             }
-            if (edge && exch)
-                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, fresh_args<ExArgs>()->ctl, dead, lu);
+            if (edge && exch) {
+                const ArgPtr<ExArgs> k = fresh_args<ExArgs>();
+                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, k->limit, (grp + 1) * P, dead, lu);
+            }
             if (edge) __builtin_amdgcn_s_setprio(0);
             put_q();
             lds_barrier();

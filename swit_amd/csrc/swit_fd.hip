@@ -94,6 +94,7 @@ struct ResidentState {
     rk::u64 *msg = nullptr;      // exchange words (shared by the plan's resident launches)
     size_t f_msg = 0;
     rk::Ctl *ctl = nullptr;
+    int wait_ms = 30000;         // limit of a wait for a neighbour (SWIT_OPT_RESIDENT_WAIT)
 };
 
 struct swit_plan {
@@ -1839,6 +1840,7 @@ static int resident_forward_steps(swit_plan *pl, int it0, int it1, const float *
     a.end = end;
     a.msg = rs.msg;
     a.ctl = rs.ctl;
+    a.limit = rs.wait_ms * rk::kTicksPerMs;
     hipLaunchKernelGGL(find_fwd(rs.fc.R, rs.fc.C)->fn[hist.p ? 1 : 0], dim3(rs.fc.G * rs.fc.P), dim3(64 * rs.fc.W), rs.f_lds, st, a);
     LAUNCH_CHECK();
     return SWIT_OK;
@@ -1923,6 +1925,7 @@ static int resident_backward_steps(swit_plan *pl, const float *src, const float 
     a.acc = rs.b_acc;
     a.msg = rs.msg;
     a.ctl = rs.ctl;
+    a.limit = rs.wait_ms * rk::kTicksPerMs;
     hipLaunchKernelGGL(find_bwd(rs.bc.R, rs.bc.C)->fn, dim3(rs.bc.G * rs.bc.P), dim3(64 * rs.bc.W), rs.b_lds, st, a);
     LAUNCH_CHECK();
     return SWIT_OK;
@@ -1975,6 +1978,7 @@ static int resident_adjoint_exact(swit_plan *pl, const float *gseis, hipStream_t
     x.gk = bs.gk;
     x.msg = rs.msg;
     x.ctl = rs.ctl;
+    x.limit = rs.wait_ms * rk::kTicksPerMs;
     const size_t chunk = (size_t)pl->ns * 3 * d.nxp * d.ld;
     const int nseg = bs.ck ? bs.nck : 1;
     for (int j = nseg - 1; j >= 0; --j) {
@@ -2279,6 +2283,10 @@ extern "C" int swit_plan_set_option(swit_plan *pl, int option, int value) {
     case SWIT_OPT_RESIDENT:
         if (value != 0 && value != 1) return set_err(SWIT_EINVAL, "resident must be 0 or 1");
         pl->res.use_fwd = pl->res.use_bwd = pl->res.use_exact = value;
+        return SWIT_OK;
+    case SWIT_OPT_RESIDENT_WAIT:
+        if (value < 0) return set_err(SWIT_EINVAL, "the wait must be 0 ms or more");
+        pl->res.wait_ms = value;
         return SWIT_OK;
     case SWIT_OPT_BWD_BALANCE:
         if (value != 0 && value != 1) return set_err(SWIT_EINVAL, "backward balance must be 0 or 1");

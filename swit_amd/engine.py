@@ -118,10 +118,10 @@ class Plan:
 
     def set_option(self, option, value):
         """option: 'graph' | 'profile' | 'fwd_group' | 'fwd_colgroup' | 'bwd_colgroup' |
-        'bwd_steps' | 'bwd_tile_x' | 'bwd_balance' | 'exact_fused' | 'streams' | 'resident'
-        (batched path).  'resident' 1 (the default) keeps the wavefields in registers, one launch
+        'bwd_steps' | 'bwd_tile_x' | 'bwd_balance' | 'exact_fused' | 'streams' | 'resident' |
+        'resident_wait' (batched path).  'resident' 1 (the default) keeps the wavefields in registers, one launch
         for many steps, where the plan allows it; an option of a direction's step kernels selects
-        these for it.  'streams' 2 runs the two halves of the shots on two streams (step kernels;
+        these for it; 'resident_wait' (ms) bounds their waits.  'streams' 2 runs the two halves of the shots on two streams (step kernels;
         a resident loop takes all shots); 'bwd_balance'
         splits the one-step backward kernel's work over the XCDs by estimated cost (1, the
         default) or by item count (0).  None of them changes results."""
@@ -130,7 +130,7 @@ class Plan:
                 "bwd_colgroup": _native.SWIT_OPT_BWD_COLGROUP, "bwd_steps": _native.SWIT_OPT_BWD_STEPS,
                 "bwd_tile_x": _native.SWIT_OPT_BWD_TILE_X, "exact_fused": _native.SWIT_OPT_EXACT_FUSED,
                 "streams": _native.SWIT_OPT_STREAMS, "bwd_balance": _native.SWIT_OPT_BWD_BALANCE,
-                "resident": _native.SWIT_OPT_RESIDENT}[option]
+                "resident": _native.SWIT_OPT_RESIDENT, "resident_wait": _native.SWIT_OPT_RESIDENT_WAIT}[option]
         _native.check(self._lib.swit_plan_set_option(self._h, code, int(value)))
         if option == "bwd_steps":
             self.bwd_steps = int(value)
