@@ -1062,9 +1062,11 @@ __global__ __launch_bounds__(kThreads) void k_bwd_fused2(
 }
 
 // Cross-shot FP64 sum of the per-shot kernels and illuminations
-// (solver.f90:263-265) and g = -2 g / c (solver.f90:270).  acc: [ns][3][nx][nz].
+// (solver.f90:263-265) and g = -2 g / c (solver.f90:270).  acc: [ns][3][nx][nz].  NaN where bad is
+// set (the strips are those of a resident forward that gave up waiting).
 __global__ void k_reduce_acc(Dims d, int ns, const float *__restrict__ vp, const float *__restrict__ acc,
-                             double *__restrict__ grad, double *__restrict__ fw, double *__restrict__ bk) {
+                             const int *__restrict__ bad, double *__restrict__ grad, double *__restrict__ fw,
+                             double *__restrict__ bk) {
     size_t ni = (size_t)d.nx * d.nz;
     size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= ni) return;
@@ -1075,6 +1077,7 @@ __global__ void k_reduce_acc(Dims d, int ns, const float *__restrict__ vp, const
         f += (double)a[ni + k];
         b += (double)a[2 * ni + k];
     }
+    if (bad && *bad) g = f = b = __builtin_nan("");
     grad[k] = -2.0 * g / (double)vp[k];
     fw[k] = f;
     bk[k] = b;

@@ -367,9 +367,11 @@ __global__ void k_ex_shotsum(Dims d, int ns, const float *__restrict__ gk, doubl
 
 // dJ/dc on the interior: the shot-summed K-gradient of every padded cell that replicates
 // the interior cell (io.f90:231-300 padding), summed in FP64 column by column, times
-// dK/dc = 2 den c dt/dx.  NaN where *err is set (a resident loop that gave up waiting).
+// dK/dc = 2 den c dt/dx.  NaN where err or bad is set (a resident
+// loop that gave up waiting: this job's, or that of the forward whose history it used).
 __global__ void k_ex_fold(Dims d, const float *__restrict__ vp, const float *__restrict__ rho,
-                          const double *__restrict__ gs, const int *__restrict__ err, double *__restrict__ grad) {
+                          const double *__restrict__ gs, const int *__restrict__ err, const int *__restrict__ bad,
+                          double *__restrict__ grad) {
     const int jz = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int jx = blockIdx.y * blockDim.y + threadIdx.y + 1;
     if (jz > d.nz || jx > d.nx) return;
@@ -392,7 +394,7 @@ __global__ void k_ex_fold(Dims d, const float *__restrict__ vp, const float *__r
         for (; iz <= z1; ++iz) sum += gs[pidx(d, iz, ix)];
     }
     const size_t ki = iidx(d, jz, jx);
-    if (err && *err) sum = __builtin_nan("");
+    if ((err && *err) || (bad && *bad)) sum = __builtin_nan("");
     grad[ki] = sum * 2.0 * (double)rho[ki] * (double)vp[ki] * (double)d.dt / (double)d.dx;
 }
 

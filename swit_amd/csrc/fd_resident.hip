@@ -36,7 +36,9 @@
 // workgroups each, P at most a quarter of the chip's places, so with up to four at once (the
 // hardware queues of a process) one of them always completes.  Every
 // wait is bounded by the clock all the same (fd_wait.h): past that a wave stops waiting for
-// good, sets *err, and the job's outputs are overwritten with NaN.
+// good, sets Ctl::err, and the job's outputs are overwritten with NaN.  What an unfinished forward
+// saved for an adjoint stays marked (Ctl::bad), over other jobs and for the step kernels too,
+// until a forward that finishes takes its place: the adjoints' outputs are NaN as well.
 //
 // Per-cell arithmetic and its order are those of the step kernels: results are the same
 // bits.  Cells outside an update region have K (or B) = 0 and hold zeros, so they need no
@@ -81,9 +83,13 @@ __host__ __device__ inline int window_oe(int W, int C, int j, int P, int nxp) {
 
 constexpr int kHistPad = 64 * 8;    // floats past the divergence history: a column's lanes past the grid read them
 
+// What a forward saves for an adjoint: strips and final state, or the exact forward's history.
+enum Saved { kNothing = -1, kStrips = 0, kHistory = 1 };
+
 struct Ctl {
     unsigned ticket;
-    int err;
+    int err;                 // a wait of the job under way ran out
+    int bad[2];              // the saved strips, history are an unfinished forward's
 };
 
 struct FwdArgs {
@@ -1244,7 +1250,7 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
 }
 
 // Cross-shot FP64 sum of the resident backward's accumulators and g = -2 g / c (as
-// k_reduce_acc); NaN if a wait of the job ran out.
+// k_reduce_acc); NaN if a wait of the job, or of the forward whose strips it used, ran out.
 __global__ void k_res_reduce(Dims d, int ns, int R, int z0, const float *__restrict__ vp, const float *__restrict__ acc,
                              double *__restrict__ grad, double *__restrict__ fw, double *__restrict__ bk,
                              const Ctl *ctl) {
@@ -1259,10 +1265,10 @@ __global__ void k_res_reduce(Dims d, int ns, int R, int z0, const float *__restr
         b += (double)p[2 * n];
     }
     const size_t k = iidx(d, jz, jx);
-    const double bad = ctl->err ? __longlong_as_double(0x7ff8000000000000ll) : 0.0;
-    grad[k] = -2.0 * g / (double)vp[k] + bad;
-    fw[k] = f + bad;
-    bk[k] = b + bad;
+    if (ctl->err | ctl->bad[kStrips]) g = f = b = __builtin_nan("");
+    grad[k] = -2.0 * g / (double)vp[k];
+    fw[k] = f;
+    bk[k] = b;
 }
 
 // Adjoint sources into slot order: out[s][t][n] = in[s][map[s][n]][t] (map -1: nothing).
@@ -1678,14 +1684,18 @@ __global__ void k_res_begin(u64 *__restrict__ msg, size_t n, Ctl *ctl, int clear
     for (; i < n; i += (size_t)gridDim.x * blockDim.x) msg[i] = 0;
 }
 
+// What a forward of step kernels saves is whole.
+__global__ void k_res_saved(Ctl *ctl, int saved) { ctl->bad[saved] = 0; }
+
 // Receiver slots to traces: out[s][r][t] = in[s][t][map[s][r]], zero for a receiver past the
-// shot's own count (map -1) and at t = 0; NaN everywhere if a wait of the job ran out.
-// Tiles of 32 samples x 32 receivers through LDS; block (32, 8).
+// shot's own count (map -1) and at t = 0; NaN everywhere if a wait of the job ran out, which
+// also marks what it saved.  Tiles of 32 samples x 32 receivers through LDS; block (32, 8).
 __global__ void k_res_traces(int nt, int ngmax, const int *__restrict__ map, const float *__restrict__ in,
-                             float *__restrict__ out, const Ctl *ctl) {
+                             float *__restrict__ out, Ctl *ctl, int saved) {
     __shared__ float tile[32][33];
     const int s = blockIdx.z, r0 = blockIdx.x * 32, t0 = blockIdx.y * 32;
     const bool bad = ctl->err != 0;
+    if (saved >= 0 && blockIdx.x + blockIdx.y + blockIdx.z + threadIdx.x + threadIdx.y == 0) ctl->bad[saved] = bad;
     const int r = r0 + threadIdx.x;
     const int m = r < ngmax ? map[(size_t)s * ngmax + r] : -1;
     for (int k = threadIdx.y; k < 32; k += 8) {

@@ -688,6 +688,14 @@ static int fill(float *p, size_t n, hipStream_t st) {
     return SWIT_OK;
 }
 
+// A forward of step kernels: its strips or history take the place of an unfinished one's.
+static int resident_saved(swit_plan *pl, rk::Saved saved, hipStream_t st) {
+    if (!pl->res.ctl) return SWIT_OK;
+    hipLaunchKernelGGL(rk::k_res_saved, dim3(1), dim3(1), 0, st, pl->res.ctl, (int)saved);
+    LAUNCH_CHECK();
+    return SWIT_OK;
+}
+
 static int copyk(const float *a, float *b, size_t n, hipStream_t st) {
     int blocks = (int)std::min<size_t>((n + 255) / 256, 65536);
     if (blocks < 1) blocks = 1;
@@ -934,7 +942,7 @@ static int forward_prologue(swit_plan *pl, int save, hipStream_t st) {
         LAUNCH_CHECK();
         TRY(fill(reinterpret_cast<float *>(bs.smax), (size_t)ns * d.nt, st));   // +0.0f bits are 0
     }
-    return SWIT_OK;
+    return save ? resident_saved(pl, rk::kStrips, st) : SWIT_OK;
 }
 
 // Forward step it.  With strip saving the step's FP32 strip row goes to the plan's
@@ -1150,7 +1158,7 @@ static int adjoint_epilogue(swit_plan *pl, hipStream_t st) {
     const Dims &d = pl->d;
     const size_t ni = (size_t)d.nx * d.nz;
     hipLaunchKernelGGL(k_reduce_acc, dim3(cdiv((int)ni, 256)), dim3(256), 0, st, d, pl->ns, pl->c_int, bs.acc,
-                       bs.out, bs.out + ni, bs.out + 2 * ni);
+                       pl->res.ctl ? &pl->res.ctl->bad[rk::kStrips] : nullptr, bs.out, bs.out + ni, bs.out + 2 * ni);
     LAUNCH_CHECK();
     return SWIT_OK;
 }
@@ -1739,6 +1747,8 @@ static int resident_init(swit_plan *pl) {
     if (!rs.fwd && !rs.bwd) return SWIT_OK;
     TRY(pl->alloc(&rs.msg, std::max(rs.f_msg, std::max(rs.b_msg, rs.x_msg))));
     TRY(pl->alloc(&rs.ctl, 1));
+    HIP_TRY(hipMemset(rs.ctl, 0, sizeof(rk::Ctl)));
+    HIP_TRY(hipStreamSynchronize(nullptr));
     return SWIT_OK;
 }
 
@@ -1846,10 +1856,10 @@ static int resident_forward_steps(swit_plan *pl, int it0, int it1, const float *
     return SWIT_OK;
 }
 
-static int resident_traces(swit_plan *pl, float *seis, hipStream_t st) {
+static int resident_traces(swit_plan *pl, float *seis, rk::Saved saved, hipStream_t st) {
     const Dims &d = pl->d;
     hipLaunchKernelGGL(rk::k_res_traces, dim3(cdiv(d.ngmax, 32), cdiv(d.nt, 32), pl->ns), dim3(32, 8), 0, st, d.nt,
-                       d.ngmax, pl->res.f_map, pl->seis_t, seis, pl->res.ctl);
+                       d.ngmax, pl->res.f_map, pl->seis_t, seis, pl->res.ctl, (int)saved);
     LAUNCH_CHECK();
     return SWIT_OK;
 }
@@ -1890,7 +1900,7 @@ static int resident_forward(swit_plan *pl, const float *src, float *seis, int sa
         }
     }
     if (bs.profile) HIP_TRY(hipEventRecord(t.e1, st));
-    return resident_traces(pl, seis, st);
+    return resident_traces(pl, seis, save ? rk::kStrips : rk::kNothing, st);
 }
 
 // The reverse loop of every shot in one launch (adj: adjoint sources in slot order).
@@ -1951,7 +1961,7 @@ static int resident_forward_exact(swit_plan *pl, float *seis, hipStream_t st) {
                                        j + 1 < bs.nck ? ck + chunk : nullptr, nullptr, j == 0, st));
         }
     }
-    return resident_traces(pl, seis, st);
+    return resident_traces(pl, seis, rk::kHistory, st);
 }
 
 // Exact adjoint from the K-gradient zero: from the full history, or segment by segment (each
@@ -2869,6 +2879,7 @@ extern "C" int swit_forward_exact(swit_plan *pl, const float *src, float *seis, 
         TRY(resident_forward_exact(pl, seis, stream));
     } else {
         TRY(forward_prologue(pl, 0, stream));
+        TRY(resident_saved(pl, rk::kHistory, stream));
         TRY(exact_run(pl, 0, stream));
         hipLaunchKernelGGL(k_transpose, dim3(cdiv(d.ngmax, 32), cdiv(d.nt, 32), pl->ns), dim3(32, 8), 0, stream, d.nt,
                            d.ngmax, pl->seis_t, seis);
@@ -2908,7 +2919,8 @@ extern "C" int swit_adjoint_exact(swit_plan *pl, const float *gseis, double *gra
                        stream, d, ns, bs.gk, bs.gsum);
     LAUNCH_CHECK();
     hipLaunchKernelGGL(ex::k_ex_fold, dim3(cdiv(d.nz, 64), cdiv(d.nx, 4)), dim3(64, 4), 0, stream, d, pl->c_int,
-                       pl->rho_int, bs.gsum, resident ? &pl->res.ctl->err : nullptr, grad);
+                       pl->rho_int, bs.gsum, resident ? &pl->res.ctl->err : nullptr,
+                       pl->res.ctl ? &pl->res.ctl->bad[rk::kHistory] : nullptr, grad);
     LAUNCH_CHECK();
     return SWIT_OK;
 }
