@@ -859,6 +859,9 @@ static int batched_init(swit_plan *pl) {
     bs.use_graph = !(eg && atoi(eg) > 0);
     HIP_TRY(hipStreamCreateWithFlags(&bs.cap, hipStreamNonBlocking));
     TRY(resident_init(pl));
+    // the buffers (checkpoints too) are clear before a job on a stream that does not wait for
+    // this one writes them
+    HIP_TRY(hipStreamSynchronize(nullptr));
     bs.ready = 1;
     return SWIT_OK;
 }
@@ -1748,7 +1751,6 @@ static int resident_init(swit_plan *pl) {
     TRY(pl->alloc(&rs.msg, std::max(rs.f_msg, std::max(rs.b_msg, rs.x_msg))));
     TRY(pl->alloc(&rs.ctl, 1));
     HIP_TRY(hipMemset(rs.ctl, 0, sizeof(rk::Ctl)));
-    HIP_TRY(hipStreamSynchronize(nullptr));
     return SWIT_OK;
 }
 
