@@ -80,6 +80,15 @@ template <bool PLAIN> __device__ __forceinline__ double divide(double a, const D
 
 constexpr int kMisfitHeld = 16;     // samples of each trace per thread that stay in registers
 
+// A dead trace (no energy in obs or syn, or an obs that is not a number) contributes nothing.  A live
+// one whose synthetic is not a number is no dead trace: its misfit and adjoint source are NaN, so
+// that a forward that did not finish, or did not stay stable, is not taken for a perfect model (the
+// toolbox's rule, norm > 0, drops such traces).  This is what a trace that is not ordinary, of
+// energies so and ss, gives.
+__device__ __forceinline__ double not_ordinary(double so, double ss) {
+    return so > 0.0 && ss != ss ? __builtin_nan("") : 0.0;
+}
+
 // kind 0 waveform, 1 global correlation.  obs/syn/adj: [ntraces][nt].
 // Three passes over both traces: the first kMisfitHeld samples of each thread stay in registers,
 // longer traces read the rest again.  23569 traces of 4000 samples (1.13 GB with the adjoint
@@ -123,15 +132,16 @@ __global__ __launch_bounds__(kMisfitThreads) void k_misfit_trace(int nt, float d
     block_sums(t, sh);
     const double so = t[0], ss = t[1];
     const bool live = so > 0.0 && ss > 0.0;
+    const double other = not_ordinary(so, ss);
     if (KIND == 0) {
         double r2 = 0.0;
         each([&](int i, float of, float sf) {
             const float r = sf - of;
-            a[i] = live ? r : 0.0f;
+            a[i] = live ? r : (float)other;
             r2 += (double)r * (double)r;
         });
         r2 = block_sum(r2, sh);
-        if (threadIdx.x == 0) tmis[blockIdx.x] = live ? sqrt(r2 * (double)dt) : 0.0;
+        if (threadIdx.x == 0) tmis[blockIdx.x] = live ? sqrt(r2 * (double)dt) : other;
         return;
     }
     const double mo = t[2] / nt, ms = t[3] / nt;
@@ -150,12 +160,12 @@ __global__ __launch_bounds__(kMisfitThreads) void k_misfit_trace(int nt, float d
         constexpr bool kPlain = decltype(plain)::value;
         each([&](int i, float of, float sf) {
             const double on = divide<kPlain>((double)of, no), sn = divide<kPlain>((double)sf, ns);
-            a[i] = live ? (float)divide<kPlain>(sn * c - on, ns) : 0.0f;
+            a[i] = live ? (float)divide<kPlain>(sn * c - on, ns) : (float)other;
         });
     };
     if (no.plain || ns.plain) store(std::true_type{});
     else store(std::false_type{});
-    if (threadIdx.x == 0) tmis[blockIdx.x] = live ? -c : 0.0;
+    if (threadIdx.x == 0) tmis[blockIdx.x] = live ? -c : other;
 }
 
 // Fixed-order FP64 sum of n values into out[0]: one workgroup, each thread sums a
@@ -473,8 +483,9 @@ __attribute__((amdgpu_waves_per_eu(NMAX <= 4096 ? 4 : 1, 8))) void k_misfit_enve
     so = block_sum<T>(so, L.sh);
     ss = block_sum<T>(ss, L.sh);
     if (!(so > 0.0 && ss > 0.0)) {                    // uniform over the workgroup
-        for (int i = threadIdx.x; i < n; i += T) a[i] = 0.0f;
-        if (threadIdx.x == 0) tmis[blockIdx.x] = 0.0;
+        const double v = not_ordinary(so, ss);
+        for (int i = threadIdx.x; i < n; i += T) a[i] = (float)v;
+        if (threadIdx.x == 0) tmis[blockIdx.x] = v;
         return;
     }
     fft_lds<NMAX, T, false>(L, f);
@@ -542,8 +553,9 @@ __attribute__((amdgpu_waves_per_eu(NMAX <= 4096 ? 4 : 1, 8))) void k_misfit_trav
     dabs = block_sum<T>(dabs, L.sh);
     d2 = block_sum<T>(d2, L.sh);
     if (!(so > 0.0 && ss > 0.0 && dabs > 0.0)) {     // uniform over the workgroup
-        for (int i = threadIdx.x; i < n; i += T) a[i] = 0.0f;
-        if (threadIdx.x == 0) tmis[blockIdx.x] = 0.0;
+        const double v = not_ordinary(so, ss);
+        for (int i = threadIdx.x; i < n; i += T) a[i] = (float)v;
+        if (threadIdx.x == 0) tmis[blockIdx.x] = v;
         return;
     }
     fft_lds<NMAX, T, false>(L, f);

@@ -183,7 +183,11 @@ def forward(simu, simu_type='obs', savesnap=0):
         # one shot's gather at a time to the host and into its SU file
         ng = simu.receiver.n
         for isrc in range(srcn):
-            su.write(homepath + 'data/%s/src%d_sg.su' % (simu_type, isrc + 1), seis[isrc, :ng].cpu().numpy(),
+            gather = seis[isrc, :ng].cpu().numpy()
+            # sample 0 of a forward is 0 (csg(1,:)); NaN says that its time loop gave up
+            if np.isnan(gather[:, 0]).any():
+                raise RuntimeError('the time loop did not finish')
+            su.write(homepath + 'data/%s/src%d_sg.su' % (simu_type, isrc + 1), gather,
                      inp["dt"], inp["src_xz"][isrc, 0], inp["rec_xz"][isrc, :, 0])
         del seis
     except Exception as exc:  # the reference reports a failed solver run this way
@@ -216,6 +220,8 @@ def adjoint(simu, optim):
         grad = g.cpu().numpy().astype(np.float32)
         forw = fw.cpu().numpy().astype(np.float32)
         back = bk.cpu().numpy().astype(np.float32)
+        if np.isnan(forw).all():
+            raise RuntimeError('the time loop did not finish')
     except Exception as exc:
         print(exc)
         raise ValueError('Adjoint solver crash') from exc
