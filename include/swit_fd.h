@@ -157,7 +157,7 @@ const char *swit_last_error(void);
                                    capturing stream take the step kernels               */
 #define SWIT_OPT_RESIDENT_WAIT 2048  /* ms (default 30000) after which a workgroup of a
                                    resident loop stops waiting for a neighbour that runs
-                                   (20 times that for one that has no room to start yet);
+                                   (20 times that where one has had no room to start);
                                    its job's outputs are then NaN, those of an adjoint
                                    from the strips or history of such a forward too     */
 int swit_plan_set_option(swit_plan *plan, int option, int value);

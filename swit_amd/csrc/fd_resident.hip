@@ -30,13 +30,11 @@
 // n+2 only after it has received n+1, which is sent after n was read.
 //
 // Progress.  Workgroups take their place by a ticket counter when they start to run, and P
-// consecutive tickets form the group of one shot.  So at any time at most one group of a
-// launch is incomplete, and it waits only for workgroups that are dispatched next; complete
-// groups run to their end.  Several such launches at once hold at most P - 1 waiting
-// workgroups each, P at most a quarter of the chip's places, so with up to four at once (the
-// hardware queues of a process) one of them always completes.  Every
-// wait is bounded by the clock all the same (fd_wait.h): past that a wave stops waiting for
-// good, sets Ctl::err, and the job's outputs are overwritten with NaN.  What an unfinished forward
+// consecutive tickets form the group of one shot.  So at any time at most one group of a launch is incomplete, and it waits only for workgroups that are
+// dispatched next; complete groups run to their end.  Several such launches at once hold at
+// most P - 1 waiting workgroups each, P at most a quarter of the chip's places, so with up to
+// four at once (the hardware queues of a process) one of them always completes.  Every wait
+// is bounded by the clock all the same (fd_wait.h): past that a wave stops waiting for good, sets Ctl::err, and the job's outputs are overwritten with NaN.  What an unfinished forward
 // saved for an adjoint stays marked (Ctl::bad), over other jobs and for the step kernels too,
 // until a forward that finishes takes its place: the adjoints' outputs are NaN as well.
 //
@@ -52,8 +50,6 @@ namespace rk {
 
 typedef unsigned long long u64;
 
-
-constexpr u64 kTicksPerMs = 100000ull;          // the 100 MHz clock of wall_clock64
 
 // lane l gets lane l+1's (up) or l-1's (dn) value, 0 past the ends; every lane active
 __device__ __forceinline__ float up1(float v) {
@@ -118,7 +114,7 @@ struct FwdArgs {
     float *end;                 // null or [ns][3][nx][nz]
     u64 *msg;                   // [G P][2 slots][2 sides][3 R][64]
     Ctl *ctl;
-    u64 limit;                  // of a wait, in ticks
+    unsigned limit;             // of a wait (wait_limit)
 };
 
 // A value the compiler must take as changed: what is computed or loaded from it inside a
@@ -130,6 +126,13 @@ __device__ __forceinline__ void opaque_s(int &v) {
 __device__ __forceinline__ void opaque_v(unsigned &v) { asm volatile("" : "+v"(v)); }
 // The value is computed by here: the compiler may not move its arithmetic further down.
 __device__ __forceinline__ void pin(float &v) { asm volatile("" : "+v"(v)); }
+
+// A workgroup's place: its ticket, and the ticket behind its group's last.
+__device__ __forceinline__ void take_place(Ctl *ctl, int P, unsigned (&place)[2]) {
+    const unsigned t = atomicAdd(&ctl->ticket, 1u);
+    place[0] = t;
+    place[1] = (t / P + 1) * P;
+}
 
 // One column's rows into a message (row r at o + 64 r words).
 template <int R> __device__ __forceinline__ void send_col(u64 *o, unsigned tag, const float (&v)[R]) {
@@ -143,13 +146,13 @@ template <int R> __device__ __forceinline__ void send_col(u64 *o, unsigned tag, 
     }
 }
 // N columns' rows out of a message, polled until every word carries the tag (all loads of a
-// round in flight together).  A wave that has waited too long once waits no more.  group_end:
-// the ticket behind the group's last.
+// round in flight together).  A wave that has waited too long once waits no more.  The group is
+// looked at past the first limit only: a look at every start of a launch took 2 us of it.
 template <int R, int N>
-__device__ __forceinline__ void recv_cols(const u64 *in, unsigned tag, Ctl *ctl, u64 limit, unsigned group_end,
-                                          bool &dead, float (&v)[N][R]) {
-    Wait wait;
-    u64 q[N][R];
+__device__ __forceinline__ void recv_cols(const u64 *in, unsigned tag, Ctl *ctl, unsigned limit,
+                                          const unsigned (&place)[2], bool &dead, float (&v)[N][R]) {
+    u64 from = 0, q[N][R];
+    unsigned most = limit;
     for (;;) {
         unsigned bad = 0;
 #pragma unroll
@@ -160,9 +163,12 @@ __device__ __forceinline__ void recv_cols(const u64 *in, unsigned tag, Ctl *ctl,
                 bad |= (unsigned)(q[n][r] >> 32) ^ tag;
             }
         if (__all(bad == 0) || dead) break;
-        if (wait_over(wall_clock64(), limit, wait, [&] {
-                return __hip_atomic_load(&ctl->ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= group_end;
-            })) {
+        if (wait_over(wall_clock64(), from, most)) {
+            if (most < kRoomWaits * limit &&
+                __hip_atomic_load(&ctl->ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < place[1]) {
+                most = kRoomWaits * limit;
+                continue;
+            }
             dead = true;
             if ((threadIdx.x & 63) == 0) __hip_atomic_store(&ctl->err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             break;
@@ -192,18 +198,18 @@ __device__ __forceinline__ void send_edges(bool has_l, bool has_r, int wave, int
 // Fresh halo columns from the inboxes: positions 0, 1, 2 from each end (C >= 3: one wave).
 template <int R, int C>
 __device__ __forceinline__ void recv_edges(bool has_l, bool has_r, int wave, int W, const u64 *from_l,
-                                           const u64 *from_r, unsigned tag, Ctl *ctl, u64 limit, unsigned group_end,
-                                           bool &dead, float (&f)[C][R]) {
+                                           const u64 *from_r, unsigned tag, Ctl *ctl, unsigned limit,
+                                           const unsigned (&place)[2], bool &dead, float (&f)[C][R]) {
     float v[kH][R];
     if (has_l && wave == 0) {
-        recv_cols<R, kH>(from_l, tag, ctl, limit, group_end, dead, v);
+        recv_cols<R, kH>(from_l, tag, ctl, limit, place, dead, v);
 #pragma unroll
         for (int h = 0; h < kH; ++h)
 #pragma unroll
             for (int r = 0; r < R; ++r) f[h][r] = v[h][r];
     }
     if (has_r && wave == W - 1) {
-        recv_cols<R, kH>(from_r, tag, ctl, limit, group_end, dead, v);
+        recv_cols<R, kH>(from_r, tag, ctl, limit, place, dead, v);
 #pragma unroll
         for (int h = 0; h < kH; ++h)
 #pragma unroll
@@ -287,15 +293,15 @@ __device__ __forceinline__ void buffer_store_rows(__amdgpu_buffer_rsrc_t rs, uns
 template <int R, int C, bool HIST>
 __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs a) {
     extern __shared__ float lds[];
-    __shared__ int sh_ticket;
+    __shared__ unsigned sh_place[2];
     constexpr int PF = R * C > 20 ? 2 : 1;               // columns whose coefficients are in flight
     constexpr int kCol = 64 * R * 4;                     // bytes of a column of one array
     const int W = a.c.W, P = a.c.P;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (threadIdx.x == 0) sh_ticket = (int)atomicAdd(&a.ctl->ticket, 1u);
+    if (threadIdx.x == 0) take_place(a.ctl, P, sh_place);
     __syncthreads();
-    const int t = __builtin_amdgcn_readfirstlane(sh_ticket);
+    const int t = __builtin_amdgcn_readfirstlane(sh_place[0]);
     const int grp = __builtin_amdgcn_readfirstlane(t / P), j = __builtin_amdgcn_readfirstlane(t % P);
     float *eU = lds;                                     // [W][3][R][64]: first, last but one, last column of u
     float *eP = eU + W * 3 * R * 64;                     // [W][3][R][64]: first, second, last column of p
@@ -671,7 +677,8 @@ __global__ __launch_bounds__(R *C > 20 ? 512 : 1024) void k_fwd_resident(FwdArgs
             // ---- exchange, in: fresh halo columns ----
             if (edge && exch) {
                 const ArgPtr<FwdArgs> k = fresh_args<FwdArgs>();
-                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, k->limit, (grp + 1) * P, dead, u);
+                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, k->limit, sh_place, dead,
+                                 u);
             }
             if (edge) __builtin_amdgcn_s_setprio(0);
             if constexpr (kLate) {
@@ -750,7 +757,7 @@ struct BwdArgs {
     float *acc;                 // [ns][nxp][3][64 R] per-shot accumulators, zero at the start
     u64 *msg;                   // [G P][2 slots][2 sides][2 fields][3 R][64]
     Ctl *ctl;
-    u64 limit;                  // as the forward's
+    unsigned limit;             // as the forward's
 };
 
 // LDS of the backward: the waves' edge columns of both wavefields (p, then u: with R >= 5 in
@@ -787,15 +794,15 @@ __host__ __device__ inline int bwd_step_floats(int W, int C, int R, int ninj, in
 template <int R, int C>
 __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
     extern __shared__ float lds[];
-    __shared__ int sh_ticket;
+    __shared__ unsigned sh_place[2];
     constexpr int kCol = 64 * R * 4;                     // bytes of a column of one array
     constexpr int NI6 = (6 * C + 63) / 64;               // strip values of the window's columns per thread
     const int W = a.c.W, P = a.c.P, T = W * 64;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (threadIdx.x == 0) sh_ticket = (int)atomicAdd(&a.ctl->ticket, 1u);
+    if (threadIdx.x == 0) take_place(a.ctl, P, sh_place);
     __syncthreads();
-    const int t = __builtin_amdgcn_readfirstlane(sh_ticket);
+    const int t = __builtin_amdgcn_readfirstlane(sh_place[0]);
     const int grp = __builtin_amdgcn_readfirstlane(t / P), j = __builtin_amdgcn_readfirstlane(t % P);
     const int WC = W * C, NI = __popcll(a.imask);
     float *eP = lds;                                     // [W][2 fields][3][R][64]: first, second, last column of p
@@ -1238,8 +1245,8 @@ __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
             if (exch) hand_out(it - 1, i0, i1);
             if (edge && exch) {
                 const ArgPtr<BwdArgs> k = fresh_args<BwdArgs>();
-                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, k->limit, (grp + 1) * P, dead, pr);
-                recv_edges<R, C>(has_l, has_r, wave, W, box + kMsg / 2, box + kMsg + kMsg / 2, tag, k->ctl, k->limit, (grp + 1) * P,
+                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, k->limit, sh_place, dead, pr);
+                recv_edges<R, C>(has_l, has_r, wave, W, box + kMsg / 2, box + kMsg + kMsg / 2, tag, k->ctl, k->limit, sh_place,
                                  dead, pa);
             }
             if (edge) __builtin_amdgcn_s_setprio(0);
@@ -1310,7 +1317,7 @@ struct ExArgs {
     int add;                    // 0: it is zero
     u64 *msg;                   // as the forward's
     Ctl *ctl;
-    u64 limit;
+    unsigned limit;
 };
 
 // LDS of the exact reverse loop: the waves' edge columns of q and r, two injection stages.
@@ -1329,14 +1336,14 @@ __host__ __device__ inline int ex_set_floats(int W, int C, int R, int NI, int la
 template <int R, int C>
 __global__ __launch_bounds__(512) void k_ex_resident(ExArgs a) {
     extern __shared__ float lds[];
-    __shared__ int sh_ticket;
+    __shared__ unsigned sh_place[2];
     constexpr int kCol = 64 * R * 4;
     const int W = a.c.W, P = a.c.P, T = W * 64;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (threadIdx.x == 0) sh_ticket = (int)atomicAdd(&a.ctl->ticket, 1u);
+    if (threadIdx.x == 0) take_place(a.ctl, P, sh_place);
     __syncthreads();
-    const int t = __builtin_amdgcn_readfirstlane(sh_ticket);
+    const int t = __builtin_amdgcn_readfirstlane(sh_place[0]);
     const int grp = __builtin_amdgcn_readfirstlane(t / P), j = __builtin_amdgcn_readfirstlane(t % P);
     const int NI = __popcll(a.imask);
     float *eQ = lds;                                     // [W][3][R][64]: first, last but one, last column of qu
@@ -1593,7 +1600,8 @@ __global__ __launch_bounds__(512) void k_ex_resident(ExArgs a) {
             }
             if (edge && exch) {
                 const ArgPtr<ExArgs> k = fresh_args<ExArgs>();
-                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, k->limit, (grp + 1) * P, dead, lu);
+                recv_edges<R, C>(has_l, has_r, wave, W, box, box + kMsg, tag, k->ctl, k->limit, sh_place, dead,
+                                 lu);
             }
             if (edge) __builtin_amdgcn_s_setprio(0);
             put_q();

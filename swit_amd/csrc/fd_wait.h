@@ -1,32 +1,24 @@
-// When a wave of a resident time loop stops waiting for a neighbour's message.
+// When a wave of a resident time loop stops waiting.
 #pragma once
 
 namespace swit {
 namespace rk {
 
-// A group's windows start one by one, and one whose turn comes while other launches hold the
-// chip starts when one of these ends, after minutes if that is a survey of long records: a wave that waits for such a
-// window waits for room, not for a neighbour that is stuck.  So the limit counts from the time
-// at which the whole group is known to run; up to there a wave waits kRoomWaits limits, so
-// that every wave ends in any case.
-constexpr unsigned long long kRoomWaits = 20;
+// A neighbour's message may take one limit.  But a group's windows start one by one, and one whose
+// turn comes while other launches hold the chip starts when one of these ends, after minutes if
+// that is a survey of long records: where the group does not run as a whole at the end of the limit,
+// the wait may take kRoomWaits of it.  Every wave ends in any case.
+constexpr unsigned kRoomWaits = 20;
 
-struct Wait {
-    unsigned long long from = 0;    // start of the wait, or when its group was seen to run
-    bool runs = false;
-};
+// Limits count in units of 2^kWaitShift ticks of the 100 MHz clock (0.66 ms), so that kRoomWaits of
+// the longest (kMaxWaitMs) are a number of 32 bits.
+constexpr int kWaitShift = 16, kMaxWaitMs = 100000000;
+constexpr unsigned wait_limit(int ms) { return (unsigned)((unsigned long long)ms * 100000u >> kWaitShift); }
 
-// Whether a wait ends unfinished at the clock's `now` (never 0).  group_runs(): every window of the
-// group has started; asked only past the limit.
-template <class F>
-constexpr bool wait_over(unsigned long long now, unsigned long long limit, Wait &w, F group_runs) {
-    if (w.from == 0) w.from = now;
-    if (now - w.from < limit) return false;
-    if (w.runs) return true;
-    if (!group_runs()) return now - w.from >= kRoomWaits * limit;
-    w.runs = true;
-    w.from = now;
-    return limit == 0;
+// Whether a wait that began at clock `from` (0: begins now; the clock is never 0) has lasted the limit.
+constexpr bool wait_over(unsigned long long now, unsigned long long &from, unsigned limit) {
+    if (from == 0) from = now;
+    return (now - from) >> kWaitShift >= limit;
 }
 
 }  // namespace rk

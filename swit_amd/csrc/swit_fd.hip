@@ -1852,7 +1852,7 @@ static int resident_forward_steps(swit_plan *pl, int it0, int it1, const float *
     a.end = end;
     a.msg = rs.msg;
     a.ctl = rs.ctl;
-    a.limit = rs.wait_ms * rk::kTicksPerMs;
+    a.limit = rk::wait_limit(rs.wait_ms);
     hipLaunchKernelGGL(find_fwd(rs.fc.R, rs.fc.C)->fn[hist.p ? 1 : 0], dim3(rs.fc.G * rs.fc.P), dim3(64 * rs.fc.W), rs.f_lds, st, a);
     LAUNCH_CHECK();
     return SWIT_OK;
@@ -1937,7 +1937,7 @@ static int resident_backward_steps(swit_plan *pl, const float *src, const float 
     a.acc = rs.b_acc;
     a.msg = rs.msg;
     a.ctl = rs.ctl;
-    a.limit = rs.wait_ms * rk::kTicksPerMs;
+    a.limit = rk::wait_limit(rs.wait_ms);
     hipLaunchKernelGGL(find_bwd(rs.bc.R, rs.bc.C)->fn, dim3(rs.bc.G * rs.bc.P), dim3(64 * rs.bc.W), rs.b_lds, st, a);
     LAUNCH_CHECK();
     return SWIT_OK;
@@ -1990,7 +1990,7 @@ static int resident_adjoint_exact(swit_plan *pl, const float *gseis, hipStream_t
     x.gk = bs.gk;
     x.msg = rs.msg;
     x.ctl = rs.ctl;
-    x.limit = rs.wait_ms * rk::kTicksPerMs;
+    x.limit = rk::wait_limit(rs.wait_ms);
     const size_t chunk = (size_t)pl->ns * 3 * d.nxp * d.ld;
     const int nseg = bs.ck ? bs.nck : 1;
     for (int j = nseg - 1; j >= 0; --j) {
@@ -2297,7 +2297,8 @@ extern "C" int swit_plan_set_option(swit_plan *pl, int option, int value) {
         pl->res.use_fwd = pl->res.use_bwd = pl->res.use_exact = value;
         return SWIT_OK;
     case SWIT_OPT_RESIDENT_WAIT:
-        if (value < 0) return set_err(SWIT_EINVAL, "the wait must be 0 ms or more");
+        if (value < 0 || value > rk::kMaxWaitMs)
+            return set_err(SWIT_EINVAL, "the wait must be 0 to %d ms", rk::kMaxWaitMs);
         pl->res.wait_ms = value;
         return SWIT_OK;
     case SWIT_OPT_BWD_BALANCE:

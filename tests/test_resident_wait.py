@@ -1,6 +1,6 @@
-"""The bound on a resident loop's waits (csrc/fd_wait.h), compiled for the host: a wave gives
-a neighbour that runs the limit, counts that from the time its whole group is known to run, and ends
-in any case.  The waits are stepped with a clock of one tick."""
+"""The bounds on a resident loop's waits (csrc/fd_wait.h), compiled for the host: their length on the
+100 MHz clock, for a neighbour's message (one limit) and for one that has no room to start yet
+(kRoomWaits limits), from no wait at all to the longest one."""
 import subprocess
 
 import pytest
@@ -12,15 +12,22 @@ SOURCE = r"""
 #include <cstdlib>
 #include "fd_wait.h"
 using namespace swit::rk;
-// ticks from the start of a wait, at clock `start`, to its end; the group runs from clock `runs_at`
+// ticks, to the unit of the limit, from the first look at the clock to the end of a wait
 int main(int argc, char **argv) {
-    const unsigned long long start = atoll(argv[1]), limit = atoll(argv[2]), runs_at = atoll(argv[3]);
-    Wait w;
-    for (unsigned long long now = start;; ++now)
-        if (wait_over(now, limit, w, [&] { return now >= runs_at; })) {
-            printf("%llu\n", now - start);
-            return 0;
+    const unsigned limit = wait_limit(atoi(argv[1])) * (argv[2][0] == 'r' ? kRoomWaits : 1);
+    const unsigned long long start = atoll(argv[3]), unit = 1ull << kWaitShift;
+    unsigned long long from = 0, n = 0;
+    if (!wait_over(start, from, limit)) {
+        unsigned long long lo = 0, hi = 1ull << 40;         // in units: over at hi, not at lo
+        while (hi - lo > 1) {
+            const unsigned long long mid = lo + (hi - lo) / 2;
+            if (wait_over(start + mid * unit, from, limit)) hi = mid;
+            else lo = mid;
         }
+        n = hi;
+    }
+    if (from != start) return 1;
+    printf("%llu %u %d\n", n * unit, kRoomWaits, kMaxWaitMs);
 }
 """
 
@@ -30,23 +37,14 @@ def ticks(tmp_path_factory):
     d = tmp_path_factory.mktemp("wait")
     (d / "wait.cpp").write_text(SOURCE)
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, str(d / "wait.cpp"), "-o", str(d / "wait")], check=True)
-    return lambda *a: int(subprocess.run([str(d / "wait"), *map(str, a)], check=True, capture_output=True,
-                                         timeout=60).stdout)
+    return lambda *a: [int(v) for v in subprocess.run([str(d / "wait"), *map(str, a)], check=True,
+                                                      capture_output=True, timeout=60).stdout.split()]
 
 
-def test_a_neighbour_that_runs_gets_the_limit(ticks):
-    assert ticks(7, 1000, 0) == 2000        # a limit to ask whether the group runs, a limit from there
-
-
-@pytest.mark.parametrize("runs_at", [1500, 5000, 19000])
-def test_waiting_for_room_does_not_count(ticks, runs_at):
-    """A group that starts late, behind another launch, has the whole limit from then on."""
-    assert ticks(1, 1000, runs_at) == runs_at - 1 + 1000
-
-
-def test_a_group_that_never_starts_ends(ticks):
-    assert ticks(1, 1000, 10**9) == 20 * 1000
-
-
-def test_no_limit_ends_at_once(ticks):
-    assert ticks(1, 0, 0) == 0 and ticks(1, 0, 10**9) == 0
+@pytest.mark.parametrize("start", [1, 12345, 2**45 + 7])
+@pytest.mark.parametrize("what,limits", [("message", 1), ("room", 20)])
+@pytest.mark.parametrize("ms", [0, 1, 1000, 30000, 10**8])
+def test_length(ticks, ms, what, limits, start):
+    t, room, longest = ticks(ms, what, start)
+    assert room == 20 and longest == 10**8
+    assert ms * 100000 * limits - limits * 2**16 < t <= ms * 100000 * limits
