@@ -149,9 +149,11 @@ const char *swit_last_error(void);
                                    over the 8 XCDs: 1 (default) contiguous ranges of
                                    equal estimated bytes moved; 0 equal item counts
                                    (same results)                                      */
-#define SWIT_OPT_RESIDENT 1024  /* 1 (default): time loops that keep the wavefields in
-                                   registers, one launch for many steps, where the grid's
-                                   height allows (same results); 0: one launch per step.
+#define SWIT_OPT_RESIDENT 1024  /* 1: time loops that keep the wavefields in registers, one
+                                   launch for many steps, where the grid's height allows
+                                   (same results); 0: one launch per step.  A plan starts
+                                   with 1, but for an adjoint whose step kernels are
+                                   estimated the faster (tall grids with few shots).
                                    An option of a direction's step kernels selects these
                                    for it; the autotuner takes the faster.  Calls on a
                                    capturing stream take the step kernels               */

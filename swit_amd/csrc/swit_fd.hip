@@ -56,7 +56,8 @@ int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // Resident time loops of a plan (fd_resident.hip): the forward's window configuration, the
 // arrays laid out for it and its launch state.  use_*: SWIT_OPT_RESIDENT, and 0 for a direction
-// whose step kernels were configured by an option of theirs.
+// whose step kernels were configured by an option of theirs; use_bwd starts as the rule of
+// backward_resident_wins has it.
 struct ResidentState {
     int use_fwd = 1, use_bwd = 1, use_exact = 1;
     bool fwd = false;            // the forward's configuration exists
@@ -1430,12 +1431,14 @@ struct BwdKernel {
     int R, C;
     void (*fn)(rk::BwdArgs);
 };
-// 6 R C floats of state per thread of 256 registers
+// 6 R C floats of state per thread of 256 registers.  Eight rows a lane spilled 118 of them and
+// were slower than the step kernels from one shot (16.2 against 7.1 us at 100x400) to 49 (86 and 69;
+// 315 and 311 at 801x400).
 #define SWIT_BWD(R, C) {R, C, rk::k_bwd_resident<R, C>}
 const BwdKernel kBwdKernels[] = {
     SWIT_BWD(2, 3), SWIT_BWD(2, 6), SWIT_BWD(2, 12), SWIT_BWD(3, 3), SWIT_BWD(3, 6), SWIT_BWD(3, 8),
     SWIT_BWD(4, 3), SWIT_BWD(4, 5), SWIT_BWD(4, 6), SWIT_BWD(5, 3), SWIT_BWD(5, 4), SWIT_BWD(6, 3),
-    SWIT_BWD(7, 3), SWIT_BWD(8, 3),
+    SWIT_BWD(7, 3),
 };
 #undef SWIT_BWD
 
@@ -1483,7 +1486,8 @@ struct BwdRing {
 
 // As choose_fwd.  ring: the values of up to 15 steps fetched at once, fewer where the LDS is full
 // (a fetch waits about 2 us).
-bool choose_bwd(const swit_plan *pl, int ncu, int NI, int layers, int R, int z0, rk::Cfg *best, BwdRing *best_ring) {
+bool choose_bwd(const swit_plan *pl, int ncu, int NI, int layers, int R, int z0, rk::Cfg *best, BwdRing *best_ring,
+                double *best_us) {
     const Dims &d = pl->d;
     const int ns = pl->ns;
     double best_t = 1e30;
@@ -1515,7 +1519,24 @@ bool choose_bwd(const swit_plan *pl, int ncu, int NI, int layers, int R, int z0,
             }
         }
     }
+    *best_us = best_t;
     return best_t < 1e30;
+}
+
+// Whether the reverse loop runs resident unless an option or the autotuner says otherwise: its step
+// against the step kernels', both estimated.  More than four rows a lane cost more than choose_bwd's
+// estimate, which was fitted to fewer: two barriers more for the shared edge place, and registers that
+// spill at 7 (measured over estimated, 1 to 49 shots of widths 100 to 801: 1.22 at 5 and 6 rows, 1.42
+// at 7).  The step kernels take 7.2 us while their workgroups find room all at once (0.2 million
+// padded cells), then at least 8.5, and 12.7 us per million cells and 5.4.  So tall grids with few
+// shots gain nothing from registers: 100x330 with 50 layers, one shot, 10.1 us resident and 7.1 us by
+// the step kernels; 400x259, one shot 8.8 and 7.3, four shots 9.1 and 15.1; but 201x81, one shot, 5.1
+// and 7.5.
+bool backward_resident_wins(const Dims &d, int ns, const rk::Cfg &c, double resident_us) {
+    const double tall = c.R <= 4 ? 1.0 : c.R <= 6 ? 1.22 : 1.42;
+    const double cells = 1e-6 * d.nxp * d.nzp * ns;
+    const double step_us = cells <= 0.2 ? 7.2 : std::max(8.5, 5.4 + 12.7 * cells);
+    return tall * resident_us < step_us;
 }
 
 const BwdKernel *find_bwd(int R, int C) {
@@ -1674,7 +1695,8 @@ static int resident_init_bwd(swit_plan *pl, int ncu) {
             mask |= 1ull << ((pl->rec_cells_inj[(size_t)s * d.ngmax + r] % d.ld + 1 - z0) / R);
     const int NI = __builtin_popcountll(mask);
     BwdRing ring{};
-    if (layers > 2 || NI > 8 || !choose_bwd(pl, ncu, NI, layers, R, z0, &c, &ring)) return SWIT_OK;
+    double us = 0.0;
+    if (layers > 2 || NI > 8 || !choose_bwd(pl, ncu, NI, layers, R, z0, &c, &ring, &us)) return SWIT_OK;
     const int T = c.W * 64, WC = c.W * c.C;
     std::vector<int> itab((size_t)pl->ns * c.P * 2 * T, -1), ibase((size_t)pl->ns * c.P, 0),
         imap((size_t)pl->ns * d.ngmax, -1);
@@ -1732,6 +1754,7 @@ static int resident_init_bwd(swit_plan *pl, int ncu) {
     HIP_TRY(hipMemcpy(rs.b_imap, imap.data(), sizeof(int) * imap.size(), hipMemcpyHostToDevice));
     rs.b_msg = c.P > 1 ? (size_t)c.G * c.P * 8 * rk::kH * c.R * 64 : 0;
     rs.bwd = true;
+    rs.use_bwd = backward_resident_wins(d, pl->ns, c, us);
     return SWIT_OK;
 }
 

@@ -119,8 +119,9 @@ class Plan:
     def set_option(self, option, value):
         """option: 'graph' | 'profile' | 'fwd_group' | 'fwd_colgroup' | 'bwd_colgroup' |
         'bwd_steps' | 'bwd_tile_x' | 'bwd_balance' | 'exact_fused' | 'streams' | 'resident' |
-        'resident_wait' (batched path).  'resident' 1 (the default) keeps the wavefields in registers, one launch
-        for many steps, where the plan allows it; an option of a direction's step kernels selects
+        'resident_wait' (batched path).  'resident' 1 keeps the wavefields in registers, one launch
+        for many steps, where the plan allows it (plans start so, but for an adjoint whose step
+        kernels are estimated the faster: tall grids with few shots); an option of a direction's step kernels selects
         these for it; 'resident_wait' (ms) bounds their waits.  'streams' 2 runs the two halves of the shots on two streams (step kernels;
         a resident loop takes all shots); 'bwd_balance'
         splits the one-step backward kernel's work over the XCDs by estimated cost (1, the
