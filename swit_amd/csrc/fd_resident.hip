@@ -152,7 +152,6 @@ template <int R, int N>
 __device__ __forceinline__ void recv_cols(const u64 *in, unsigned tag, Ctl *ctl, unsigned limit,
                                           const unsigned (&place)[2], bool &dead, float (&v)[N][R]) {
     u64 from = 0, q[N][R];
-    unsigned most = limit;
     for (;;) {
         unsigned bad = 0;
 #pragma unroll
@@ -163,12 +162,10 @@ __device__ __forceinline__ void recv_cols(const u64 *in, unsigned tag, Ctl *ctl,
                 bad |= (unsigned)(q[n][r] >> 32) ^ tag;
             }
         if (__all(bad == 0) || dead) break;
-        if (wait_over(wall_clock64(), from, most)) {
-            if (most < kRoomWaits * limit &&
-                __hip_atomic_load(&ctl->ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < place[1]) {
-                most = kRoomWaits * limit;
-                continue;
-            }
+        const u64 now = wall_clock64();
+        if (wait_over(now, from, limit) &&
+            (__hip_atomic_load(&ctl->ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= place[1] ||
+             wait_over(now, from, kRoomWaits * limit))) {
             dead = true;
             if ((threadIdx.x & 63) == 0) __hip_atomic_store(&ctl->err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             break;
