@@ -1431,14 +1431,12 @@ struct BwdKernel {
     int R, C;
     void (*fn)(rk::BwdArgs);
 };
-// 6 R C floats of state per thread of 256 registers.  Eight rows a lane spilled 118 of them and
-// were slower than the step kernels from one shot (16.2 against 7.1 us at 100x400) to 49 (86 and 69;
-// 315 and 311 at 801x400).
+// 6 R C floats of state per thread of 256 registers
 #define SWIT_BWD(R, C) {R, C, rk::k_bwd_resident<R, C>}
 const BwdKernel kBwdKernels[] = {
     SWIT_BWD(2, 3), SWIT_BWD(2, 6), SWIT_BWD(2, 12), SWIT_BWD(3, 3), SWIT_BWD(3, 6), SWIT_BWD(3, 8),
     SWIT_BWD(4, 3), SWIT_BWD(4, 5), SWIT_BWD(4, 6), SWIT_BWD(5, 3), SWIT_BWD(5, 4), SWIT_BWD(6, 3),
-    SWIT_BWD(7, 3),
+    SWIT_BWD(7, 3), SWIT_BWD(8, 3),
 };
 #undef SWIT_BWD
 
@@ -1526,14 +1524,15 @@ bool choose_bwd(const swit_plan *pl, int ncu, int NI, int layers, int R, int z0,
 // Whether the reverse loop runs resident unless an option or the autotuner says otherwise: its step
 // against the step kernels', both estimated.  More than four rows a lane cost more than choose_bwd's
 // estimate, which was fitted to fewer: two barriers more for the shared edge place, and registers that
-// spill at 7 (measured over estimated, 1 to 49 shots of widths 100 to 801: 1.22 at 5 and 6 rows, 1.42
-// at 7).  The step kernels take 7.2 us while their workgroups find room all at once (0.2 million
-// padded cells), then at least 8.5, and 12.7 us per million cells and 5.4.  So tall grids with few
-// shots gain nothing from registers: 100x330 with 50 layers, one shot, 10.1 us resident and 7.1 us by
-// the step kernels; 400x259, one shot 8.8 and 7.3, four shots 9.1 and 15.1; but 201x81, one shot, 5.1
-// and 7.5.
-bool backward_resident_wins(const Dims &d, int ns, const rk::Cfg &c, double resident_us) {
-    const double tall = c.R <= 4 ? 1.0 : c.R <= 6 ? 1.22 : 1.42;
+// spill from 7 rows on (measured over estimated, 1 to 49 shots of widths 100 to 801: 1.22 at 5 and 6
+// rows, 1.42 at 7, 1.9 at 8 with one wave a SIMD and 2.75 with two).  The step kernels take 7.2 us
+// while their workgroups find room all at once (0.2 million padded cells), then at least 8.5, and
+// 12.7 us per million cells and 5.4.  So tall grids with few shots gain nothing from registers:
+// 100x400 with 50 layers, one shot, 14.7 us resident and 7.1 us by the step kernels; 400x259, one shot
+// 8.8 and 7.3, four shots 9.1 and 15.1; but 201x81, one shot, 5.1 and 7.5.
+bool backward_resident_wins(const Dims &d, int ns, int ncu, const rk::Cfg &c, double resident_us) {
+    const bool one_wave = c.W * cdiv(c.G * c.P, ncu) <= 4;
+    const double tall = c.R <= 4 ? 1.0 : c.R <= 6 ? 1.22 : c.R == 7 ? 1.42 : one_wave ? 1.9 : 2.75;
     const double cells = 1e-6 * d.nxp * d.nzp * ns;
     const double step_us = cells <= 0.2 ? 7.2 : std::max(8.5, 5.4 + 12.7 * cells);
     return tall * resident_us < step_us;
@@ -1754,7 +1753,7 @@ static int resident_init_bwd(swit_plan *pl, int ncu) {
     HIP_TRY(hipMemcpy(rs.b_imap, imap.data(), sizeof(int) * imap.size(), hipMemcpyHostToDevice));
     rs.b_msg = c.P > 1 ? (size_t)c.G * c.P * 8 * rk::kH * c.R * 64 : 0;
     rs.bwd = true;
-    rs.use_bwd = backward_resident_wins(d, pl->ns, c, us);
+    rs.use_bwd = backward_resident_wins(d, pl->ns, ncu, c, us);
     return SWIT_OK;
 }
 
