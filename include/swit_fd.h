@@ -231,8 +231,9 @@ int swit_misfit(int kind, int ntraces, int nt, float dt, const float *obs, const
 
 /* ---- plan groups: uneven grids as one job -----------------------------------------
  * A group runs several batched plans (different grids, shot counts, record lengths,
- * strip precisions) as one job.  Where every plan takes the resident time loops they run
- * one after the other, each filling the chip; otherwise each group forward / adjoint is a
+ * strip precisions) as one job.  Plans in their resident time loops run side by side where
+ * they fit the chip together (up to four) and one after the other where each fills it;
+ * otherwise, or where that is estimated clearly the faster, a group forward / adjoint is a
  * single hipGraph launch holding every plan's step kernels on its own branch, so plans with
  * short records fill the GPU while long ones finish.  No counterpart in the reference (one
  * fd2dmpi job per grid, toolbox/solver.py:24-92); results are those of
@@ -248,6 +249,11 @@ int swit_group_adjoint(swit_group *group, const float *const *src, const float *
                        double *const *grad, double *const *illum_forw, double *const *illum_back,
                        hipStream_t stream);
 int swit_group_destroy(swit_group *group);
+
+/* How the group's forward (which = 0) or adjoint (1) outside a stream capture runs: 0 as one
+ * graph of step kernels, n > 0 as n sets of plans one after the other, those of a set side
+ * by side; -1 on bad arguments. */
+int swit_group_sets(const swit_group *group, int which);
 
 /* A whole gradient of every plan in one call: each plan runs the strip-saving forward
  * (seismograms to seis), the misfit and adjoint source `kind` (SWIT_MISFIT_*) against obs, exactly as swit_misfit computes them (adjoint source to

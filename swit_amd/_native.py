@@ -45,6 +45,7 @@ EXPORTS = (
     "swit_group_adjoint",
     "swit_group_destroy",
     "swit_group_gradient",
+    "swit_group_sets",
     "swit_plan_set_option",
     "swit_plan_kernel_time",
     "swit_plan_resident",
@@ -194,6 +195,8 @@ def load(path: str | None = None):
     L.swit_plan_kernel_time.restype = ctypes.c_int
     L.swit_plan_resident.argtypes = [vp, ctypes.c_int]
     L.swit_plan_resident.restype = ctypes.c_int
+    L.swit_group_sets.argtypes = [vp, ctypes.c_int]
+    L.swit_group_sets.restype = ctypes.c_int
     if path is None:
         _lib = L
     return L

@@ -56,8 +56,8 @@ int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // Resident time loops of a plan (fd_resident.hip): the forward's window configuration, the
 // arrays laid out for it and its launch state.  use_*: SWIT_OPT_RESIDENT, and 0 for a direction
-// whose step kernels were configured by an option of theirs; use_bwd starts as the rule of
-// backward_resident_wins has it.
+// whose step kernels were configured by an option of theirs; use_bwd starts as the rule in
+// resident_init_bwd has it.
 struct ResidentState {
     int use_fwd = 1, use_bwd = 1, use_exact = 1;
     bool fwd = false;            // the forward's configuration exists
@@ -96,6 +96,8 @@ struct ResidentState {
     size_t f_msg = 0;
     rk::Ctl *ctl = nullptr;
     int wait_ms = 30000;         // limit of a wait for a neighbour (SWIT_OPT_RESIDENT_WAIT)
+    double us[2] = {0.0, 0.0};   // estimated time of a step (us), by direction
+    int ncu = 0;                 // compute units of the device
 };
 
 struct swit_plan {
@@ -499,24 +501,10 @@ static int resident_adjoint(swit_plan *pl, const float *src, const float *adjsrc
 
 // ---- public jobs -------------------------------------------------------------------
 
-extern "C" int swit_forward(swit_plan *pl, const float *src, float *seis, int save_strips,
-                            hipStream_t stream) {
-    g_err[0] = 0;
-    if (!pl || !src || !seis) return set_err(SWIT_EINVAL, "plan, src and seis are required");
-    if (!pl->model_set) return set_err(SWIT_ESTATE, "swit_plan_set_model must be called first");
+// A forward or adjoint by the given route.
+static int run_forward(swit_plan *pl, const float *src, float *seis, int save, bool resident, hipStream_t stream) {
+    if (resident) return resident_forward(pl, src, seis, save, stream);
     const Dims &d = pl->d;
-    if (save_strips < 0 || save_strips > 2) return set_err(SWIT_EINVAL, "save_strips must be 0, 1 or 2");
-    if (save_strips == 1 && (pl->flags & SWIT_PLAN_NO_STRIPS))
-        return set_err(SWIT_EINVAL, "the plan was created without strips (SWIT_PLAN_NO_STRIPS)");
-    const int save = save_strips == 1;
-    if (save_strips != 2) pl->strips_valid = false;
-    bool resident = false;
-    TRY(resident_now(pl->res.fwd, pl->res.use_fwd, stream, &resident));
-    if (resident) {
-        TRY(resident_forward(pl, src, seis, save, stream));
-        if (save_strips != 2) pl->strips_valid = save_strips == 1;
-        return SWIT_OK;
-    }
     if (pl->flags & SWIT_PATH_BATCHED)
         TRY(batched_forward(pl, src, save, stream));
     else
@@ -525,21 +513,13 @@ extern "C" int swit_forward(swit_plan *pl, const float *src, float *seis, int sa
     hipLaunchKernelGGL(k_transpose, dim3(cdiv(d.ngmax, 32), cdiv(d.nt, 32), pl->ns), dim3(32, 8), 0,
                        stream, d.nt, d.ngmax, pl->seis_t, seis);
     LAUNCH_CHECK();
-    if (save_strips != 2) pl->strips_valid = save_strips == 1;
     return SWIT_OK;
 }
 
-extern "C" int swit_adjoint(swit_plan *pl, const float *src, const float *adjsrc, double *grad,
-                            double *illum_forw, double *illum_back, hipStream_t stream) {
-    g_err[0] = 0;
-    if (!pl || !src || !adjsrc || !grad || !illum_forw || !illum_back)
-        return set_err(SWIT_EINVAL, "plan, src, adjsrc and the three outputs are required");
-    if (!pl->strips_valid)
-        return set_err(SWIT_ESTATE, "no saved strips: run swit_forward with save_strips=1 first");
-    const Dims &d = pl->d;
-    bool resident = false;
-    TRY(resident_now(pl->res.bwd, pl->res.use_bwd, stream, &resident));
+static int run_adjoint(swit_plan *pl, const float *src, const float *adjsrc, double *grad, double *illum_forw,
+                       double *illum_back, bool resident, hipStream_t stream) {
     if (resident) return resident_adjoint(pl, src, adjsrc, grad, illum_forw, illum_back, stream);
+    const Dims &d = pl->d;
     // [ns][ngmax][nt] -> [ns][nt][ngmax]
     hipLaunchKernelGGL(k_transpose, dim3(cdiv(d.nt, 32), cdiv(d.ngmax, 32), pl->ns), dim3(32, 8), 0,
                        stream, d.ngmax, d.nt, adjsrc, pl->sadj_t);
@@ -554,6 +534,36 @@ extern "C" int swit_adjoint(swit_plan *pl, const float *src, const float *adjsrc
         LAUNCH_CHECK();
     }
     return SWIT_OK;
+}
+
+extern "C" int swit_forward(swit_plan *pl, const float *src, float *seis, int save_strips,
+                            hipStream_t stream) {
+    g_err[0] = 0;
+    if (!pl || !src || !seis) return set_err(SWIT_EINVAL, "plan, src and seis are required");
+    if (!pl->model_set) return set_err(SWIT_ESTATE, "swit_plan_set_model must be called first");
+    const Dims &d = pl->d;
+    if (save_strips < 0 || save_strips > 2) return set_err(SWIT_EINVAL, "save_strips must be 0, 1 or 2");
+    if (save_strips == 1 && (pl->flags & SWIT_PLAN_NO_STRIPS))
+        return set_err(SWIT_EINVAL, "the plan was created without strips (SWIT_PLAN_NO_STRIPS)");
+    const int save = save_strips == 1;
+    if (save_strips != 2) pl->strips_valid = false;
+    bool resident = false;
+    TRY(resident_now(pl->res.fwd, pl->res.use_fwd, stream, &resident));
+    TRY(run_forward(pl, src, seis, save, resident, stream));
+    if (save_strips != 2) pl->strips_valid = save_strips == 1;
+    return SWIT_OK;
+}
+
+extern "C" int swit_adjoint(swit_plan *pl, const float *src, const float *adjsrc, double *grad,
+                            double *illum_forw, double *illum_back, hipStream_t stream) {
+    g_err[0] = 0;
+    if (!pl || !src || !adjsrc || !grad || !illum_forw || !illum_back)
+        return set_err(SWIT_EINVAL, "plan, src, adjsrc and the three outputs are required");
+    if (!pl->strips_valid)
+        return set_err(SWIT_ESTATE, "no saved strips: run swit_forward with save_strips=1 first");
+    bool resident = false;
+    TRY(resident_now(pl->res.bwd, pl->res.use_bwd, stream, &resident));
+    return run_adjoint(pl, src, adjsrc, grad, illum_forw, illum_back, resident, stream);
 }
 
 // ---- batched path (host side) --------------------------------------------------------
@@ -1308,7 +1318,7 @@ int max_windows(int per_cu, int ncu) { return per_cu * ncu / 4; }
 
 // Windows of the forward for ns shots on ncu compute units: of every (columns per wave,
 // waves) the one with the least estimated time, rounds of shots x time of a step.
-bool choose_fwd(const Dims &d, int ns, int ncu, int NS, rk::Cfg *best) {
+bool choose_fwd(const Dims &d, int ns, int ncu, int NS, rk::Cfg *best, double *us) {
     const int rows = d.nzp - (d.fs - 1) + 1;
     const int R = std::max(2, cdiv(rows, 64));
     double best_t = 1e30;
@@ -1335,6 +1345,7 @@ bool choose_fwd(const Dims &d, int ns, int ncu, int NS, rk::Cfg *best) {
             if (t < best_t) {
                 best_t = t;
                 *best = c;
+                *us = t;
             }
         }
     }
@@ -1485,7 +1496,7 @@ struct BwdRing {
 // As choose_fwd.  ring: the values of up to 15 steps fetched at once, fewer where the LDS is full
 // (a fetch waits about 2 us).
 bool choose_bwd(const swit_plan *pl, int ncu, int NI, int layers, int R, int z0, rk::Cfg *best, BwdRing *best_ring,
-                double *best_us) {
+                double *us) {
     const Dims &d = pl->d;
     const int ns = pl->ns;
     double best_t = 1e30;
@@ -1514,28 +1525,29 @@ bool choose_bwd(const swit_plan *pl, int ncu, int NI, int layers, int R, int z0,
                 best_t = t;
                 *best = c;
                 *best_ring = q;
+                *us = t;
             }
         }
     }
-    *best_us = best_t;
     return best_t < 1e30;
 }
 
-// Whether the reverse loop runs resident unless an option or the autotuner says otherwise: its step
-// against the step kernels', both estimated.  More than four rows a lane cost more than choose_bwd's
-// estimate, which was fitted to fewer: two barriers more for the shared edge place, and registers that
-// spill from 7 rows on (measured over estimated, 1 to 49 shots of widths 100 to 801: 1.22 at 5 and 6
-// rows, 1.42 at 7, 1.9 at 8 with one wave a SIMD and 2.75 with two).  The step kernels take 7.2 us
-// while their workgroups find room all at once (0.2 million padded cells), then at least 8.5, and
-// 12.7 us per million cells and 5.4.  So tall grids with few shots gain nothing from registers:
-// 100x400 with 50 layers, one shot, 14.7 us resident and 7.1 us by the step kernels; 400x259, one shot
-// 8.8 and 7.3, four shots 9.1 and 15.1; but 201x81, one shot, 5.1 and 7.5.
-bool backward_resident_wins(const Dims &d, int ns, int ncu, const rk::Cfg &c, double resident_us) {
+// Estimated time of a resident reverse step (us).  More than four rows a lane cost more than
+// choose_bwd's estimate, which was fitted to fewer: two barriers more for the shared edge place, and
+// registers that spill from 7 rows on (measured over estimated, 1 to 49 shots of widths 100 to 801:
+// 1.22 at 5 and 6 rows, 1.42 at 7, 1.9 at 8 with one wave a SIMD and 2.75 with two).
+double resident_reverse_us(const rk::Cfg &c, int ncu, double us) {
     const bool one_wave = c.W * cdiv(c.G * c.P, ncu) <= 4;
-    const double tall = c.R <= 4 ? 1.0 : c.R <= 6 ? 1.22 : c.R == 7 ? 1.42 : one_wave ? 1.9 : 2.75;
+    return us * (c.R <= 4 ? 1.0 : c.R <= 6 ? 1.22 : c.R == 7 ? 1.42 : one_wave ? 1.9 : 2.75);
+}
+
+// Estimated time of a step by the step kernels (us), forward (which = 0) and backward, fitted to the
+// same shapes: the latter 7.2 us while its workgroups find room all at once (0.2 million padded
+// cells), then at least 8.5, and 12.7 us per million cells and 5.4.
+double step_kernel_us(const Dims &d, int ns, int which) {
     const double cells = 1e-6 * d.nxp * d.nzp * ns;
-    const double step_us = cells <= 0.2 ? 7.2 : std::max(8.5, 5.4 + 12.7 * cells);
-    return tall * resident_us < step_us;
+    if (which == 0) return std::max(5.9, 5.0 + 7.3 * cells);
+    return cells <= 0.2 ? 7.2 : std::max(8.5, 5.4 + 12.7 * cells);
 }
 
 const BwdKernel *find_bwd(int R, int C) {
@@ -1694,8 +1706,8 @@ static int resident_init_bwd(swit_plan *pl, int ncu) {
             mask |= 1ull << ((pl->rec_cells_inj[(size_t)s * d.ngmax + r] % d.ld + 1 - z0) / R);
     const int NI = __builtin_popcountll(mask);
     BwdRing ring{};
-    double us = 0.0;
-    if (layers > 2 || NI > 8 || !choose_bwd(pl, ncu, NI, layers, R, z0, &c, &ring, &us)) return SWIT_OK;
+    if (layers > 2 || NI > 8 || !choose_bwd(pl, ncu, NI, layers, R, z0, &c, &ring, &rs.us[1]))
+        return SWIT_OK;
     const int T = c.W * 64, WC = c.W * c.C;
     std::vector<int> itab((size_t)pl->ns * c.P * 2 * T, -1), ibase((size_t)pl->ns * c.P, 0),
         imap((size_t)pl->ns * d.ngmax, -1);
@@ -1753,7 +1765,12 @@ static int resident_init_bwd(swit_plan *pl, int ncu) {
     HIP_TRY(hipMemcpy(rs.b_imap, imap.data(), sizeof(int) * imap.size(), hipMemcpyHostToDevice));
     rs.b_msg = c.P > 1 ? (size_t)c.G * c.P * 8 * rk::kH * c.R * 64 : 0;
     rs.bwd = true;
-    rs.use_bwd = backward_resident_wins(d, pl->ns, ncu, c, us);
+    // Unless an option or the autotuner says otherwise, the route that is estimated the faster: tall
+    // grids with few shots gain nothing from registers (100x400 with 50 layers, one shot, 14.7 us
+    // resident and 7.1 us by the step kernels; 400x259, one shot 8.8 and 7.3, four shots 9.1 and 15.1;
+    // but 201x81, one shot, 5.1 and 7.5).  The forward wins at every size.
+    rs.us[1] = resident_reverse_us(c, ncu, rs.us[1]);
+    rs.use_bwd = rs.us[1] < step_kernel_us(d, pl->ns, 1);
     return SWIT_OK;
 }
 
@@ -1765,8 +1782,9 @@ static int resident_init(swit_plan *pl) {
     int dev = 0, ncu = 0;
     HIP_TRY(hipGetDevice(&dev));
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    rs.ncu = ncu;
     TRY(resident_init_bwd(pl, ncu));
-    rs.fwd = choose_fwd(d, pl->ns, ncu, 8, &rs.fc);
+    rs.fwd = choose_fwd(d, pl->ns, ncu, 8, &rs.fc, &rs.us[0]);
     TRY(resident_init_ex(pl, ncu));
     if (rs.fwd) TRY(resident_init_fwd(pl));
     if (!rs.fwd && !rs.bwd) return SWIT_OK;
@@ -2354,7 +2372,7 @@ extern "C" int swit_plan_kernel_time(swit_plan *pl, int which, double *total_ms,
 struct swit_group {
     std::vector<swit_plan *> plans;
     hipStream_t cap = nullptr;               // capture origin
-    std::vector<hipStream_t> branch;         // one capture branch per plan
+    std::vector<hipStream_t> branch;         // a stream per plan: capture branch, or plans side by side
     hipEvent_t fork = nullptr;
     std::vector<hipEvent_t> join;
     hipGraphExec_t gf[2] = {nullptr, nullptr};   // forward without / with strip saving
@@ -2422,18 +2440,140 @@ static int group_capture(swit_group *gr, int which, int save, hipGraphExec_t *ex
     return SWIT_OK;
 }
 
-// Whether every plan of the group takes the resident loops in the given directions.  They
-// then run one after the other: each fills the chip for its whole job.  501x171x2500 with 22
-// shots, 481x121x2000 with 21 and 300x102x1500 with 21, forward, misfit and adjoint: 119 ms, as
-// one graph of the step kernels 329 ms (with an earlier reverse loop 147 ms one after the other,
-// 149 to 179 ms on concurrent streams).
-static int group_resident(swit_group *gr, bool fwd, bool bwd, hipStream_t stream, bool *yes) {
-    for (swit_plan *pl : gr->plans) {
+// How a group runs one direction: the plans in sets, one set after the other, each plan by its own
+// route, or all plans' step kernels as one graph.
+struct GroupRoute {
+    std::vector<std::vector<int>> sets;      // plans side by side
+    std::vector<char> resident;              // by plan
+    bool any = false;                        // any resident
+    double us = 0.0, graph_us = 0.0;         // estimated time either way
+    // The graph where it is clearly the faster by the estimates, which are good to a tenth: for
+    // adjoints of few shots that miss fitting together (501x171 and its companions, 3 shots, 600
+    // steps: 7.6 ms against 8.8 in turn) or lie on tall grids.
+    bool graph() const { return !any || graph_us < 0.9 * us; }
+};
+
+// The workgroups of a plan's resident loop, and what one takes of a compute unit.
+struct GroupPart {
+    int wgs, waves, per_cu;     // waves: sixteenths of a unit
+    size_t lds;
+};
+
+// Whether the loops of a set surely run at once.  The dispatcher spreads the workgroups over the
+// compute units in an order that is not ours: 250 small workgroups, two of which share a unit, leave no
+// room for 124 large ones that need half the chip (501x171 with 3 shots and its companions: no gain
+// side by side).  So: every unit takes as many workgroups as of the largest kind; or whichever plan comes
+// last finds room when the others' workgroups lie on a unit each.
+static bool group_fits(const std::vector<GroupPart> &set, int ncu) {
+    int total = 0, least = 16;
+    for (const GroupPart &p : set) {
+        total += p.wgs;
+        least = std::min(least, p.per_cu);
+    }
+    if (total <= least * ncu) return true;
+    for (const GroupPart &p : set) {
+        const int others = total - p.wgs;
+        if (others > ncu) return false;
+        int room = (ncu - others) * p.per_cu;
+        for (const GroupPart &q : set)
+            if (&q != &p)
+                room += q.wgs * std::min((16 - q.waves) / p.waves, (int)((kCuLds - q.lds) / p.lds));
+        if (room < p.wgs) return false;
+    }
+    return true;
+}
+
+// Plans whose resident loops fit the chip together run side by side, since few shots are bound by the
+// latency of a step: three lines of one shot (400x150 and two smaller), reverse loops of 600 steps: 8.1
+// ms one after the other, 3.8 side by side, 5.1 as a graph of step kernels.  Plans that do not fit
+// together gain nothing (8 shots of them 8.9, 9.7 and 15.3 ms), and each of many shots fills the chip:
+// 501x171x2500 with 22 shots, 481x121x2000 with 21 and 300x102x1500 with 21, forward, misfit and
+// adjoint: 119 ms one after the other, 329 as a graph.  Sets of up to four launches, the most that
+// surely progress together; a plan of step kernels by itself.  The graph's estimate: its longest
+// record's launches, or the cells of all, a launch's share of which does not overlap (600 steps of
+// the lines above with 1, 4 and 12 shots: 5.1, 7.9 and 22.7 ms measured, 5.2, 7.2 and 21.2 estimated).
+static int group_route(const swit_group *gr, int which, hipStream_t stream, GroupRoute *g) {
+    const size_t n = gr->plans.size();
+    std::vector<double> us(n);
+    std::vector<GroupPart> part(n);
+    std::vector<std::vector<GroupPart>> held;
+    double cells_us = 0.0, steps = 0.0;
+    g->resident.assign(n, 0);
+    for (size_t i = 0; i < n; ++i) {
+        const swit_plan *pl = gr->plans[i];
         const ResidentState &rs = pl->res;
-        TRY(resident_now((rs.fwd || !fwd) && (rs.bwd || !bwd), (rs.use_fwd || !fwd) && (rs.use_bwd || !bwd), stream, yes));
-        if (!*yes) return SWIT_OK;
+        const Dims &d = pl->d;
+        bool yes = false;
+        TRY(resident_now(which == 0 ? rs.fwd : rs.bwd, which == 0 ? rs.use_fwd : rs.use_bwd, stream, &yes));
+        g->resident[i] = yes;
+        g->any = g->any || yes;
+        us[i] = (d.nt - 1) * (yes ? rs.us[which] : step_kernel_us(d, pl->ns, which));
+        const rk::Cfg &c = which == 0 ? rs.fc : rs.bc;
+        const size_t lds = (which == 0 ? rs.f_lds : rs.b_lds) + 1024;
+        const int cu_waves = which == 0 && c.R * c.C <= 20 ? 16 : 8;
+        if (yes) part[i] = GroupPart{c.G * c.P, c.W * 16 / cu_waves, std::min(cu_waves / c.W, (int)(kCuLds / lds)), lds};
+        cells_us += (d.nt - 1) * (which == 0 ? 6.9e-6 : 12.7e-6) * d.nxp * d.nzp * pl->ns;
+        steps = std::max(steps, d.nt - 1.0);
+    }
+    g->graph_us = std::max(8.6 * steps, cells_us + (which == 0 ? 4.0 : 2.5) * steps);
+    // the longest first, each into the first set with room for it
+    std::vector<int> order(n);
+    for (size_t i = 0; i < n; ++i) order[i] = (int)i;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return us[a] > us[b]; });
+    for (int i : order) {
+        size_t k = 0;
+        for (; g->resident[i] && k < g->sets.size(); ++k) {
+            if (held[k].empty() || held[k].size() == 4) continue;
+            held[k].push_back(part[i]);
+            if (group_fits(held[k], gr->plans[i]->res.ncu)) break;
+            held[k].pop_back();
+        }
+        if (!g->resident[i] || k == g->sets.size()) {
+            k = g->sets.size();
+            g->sets.emplace_back();
+            held.emplace_back();
+            if (g->resident[i]) held[k].push_back(part[i]);
+            g->us += us[i];
+        }
+        g->sets[k].push_back(i);
     }
     return SWIT_OK;
+}
+
+// job(i, stream) of every plan, set by set.  A set of several is forked from the caller's stream and
+// joined back into it, after an error too.  The joins come last: streams share the hardware's few
+// queues, and a branch behind the caller's wait for another one would run after that.
+template <class Job> static int group_run(swit_group *gr, const GroupRoute &g, hipStream_t stream, Job job) {
+    for (const std::vector<int> &set : g.sets) {
+        if (set.size() == 1) {
+            TRY(job(set[0], stream));
+            continue;
+        }
+        HIP_TRY(hipEventRecord(gr->fork, stream));
+        int rc = SWIT_OK;
+        hipError_t e = hipSuccess;
+        size_t begun = 0;
+        for (; begun < set.size() && rc == SWIT_OK && e == hipSuccess; ++begun) {
+            const int i = set[begun];
+            e = hipStreamWaitEvent(gr->branch[i], gr->fork, 0);
+            if (e == hipSuccess) rc = job(i, gr->branch[i]);
+        }
+        for (size_t k = 0; k < begun; ++k) {
+            const int i = set[k];
+            const hipError_t er = hipEventRecord(gr->join[i], gr->branch[i]);
+            const hipError_t ew = er == hipSuccess ? hipStreamWaitEvent(stream, gr->join[i], 0) : er;
+            if (e == hipSuccess) e = ew;
+        }
+        if (rc != SWIT_OK) return rc;
+        HIP_TRY(e);
+    }
+    return SWIT_OK;
+}
+
+extern "C" int swit_group_sets(const swit_group *gr, int which) {
+    GroupRoute g;
+    if (!gr || which < 0 || which > 1 || group_route(gr, which, nullptr, &g) != SWIT_OK) return -1;
+    return g.graph() ? 0 : (int)g.sets.size();
 }
 
 extern "C" int swit_group_create(swit_plan *const *plans, int nplans, swit_group **out) {
@@ -2500,12 +2640,14 @@ extern "C" int swit_group_forward(swit_group *gr, const float *const *src, float
         if (save && (gr->plans[i]->flags & SWIT_PLAN_NO_STRIPS))
             return set_err(SWIT_EINVAL, "plan %zu was created without strips (SWIT_PLAN_NO_STRIPS)", i);
     }
-    bool resident = false;
-    TRY(group_resident(gr, true, false, stream, &resident));
-    if (resident) {
+    GroupRoute route;
+    TRY(group_route(gr, 0, stream, &route));
+    if (!route.graph()) {
         for (swit_plan *pl : gr->plans)
             if (save_strips != 2) pl->strips_valid = false;
-        for (size_t i = 0; i < n; ++i) TRY(resident_forward(gr->plans[i], src[i], seis[i], save, stream));
+        TRY(group_run(gr, route, stream, [&](int i, hipStream_t st) {
+            return run_forward(gr->plans[i], src[i], seis[i], save, route.resident[i], st);
+        }));
         for (swit_plan *pl : gr->plans)
             if (save_strips != 2) pl->strips_valid = save_strips == 1;
         return SWIT_OK;
@@ -2547,13 +2689,13 @@ extern "C" int swit_group_adjoint(swit_group *gr, const float *const *src, const
         if (!gr->plans[i]->strips_valid)
             return set_err(SWIT_ESTATE, "plan %zu: no saved strips: run a strip-saving forward first", i);
     }
-    bool resident = false;
-    TRY(group_resident(gr, false, true, stream, &resident));
-    if (resident) {
-        for (size_t i = 0; i < n; ++i)
-            TRY(resident_adjoint(gr->plans[i], src[i], adjsrc[i], grad[i], illum_forw[i], illum_back[i], stream));
-        return SWIT_OK;
-    }
+    GroupRoute route;
+    TRY(group_route(gr, 1, stream, &route));
+    if (!route.graph())
+        return group_run(gr, route, stream, [&](int i, hipStream_t st) {
+            return run_adjoint(gr->plans[i], src[i], adjsrc[i], grad[i], illum_forw[i], illum_back[i],
+                               route.resident[i], st);
+        });
     for (size_t i = 0; i < n; ++i) {
         swit_plan *pl = gr->plans[i];
         const Dims &d = pl->d;
@@ -2705,18 +2847,22 @@ extern "C" int swit_group_gradient(swit_group *gr, int kind, const float *const 
                               (const void *)illum_forw[i], (const void *)illum_back[i]})
             ptrs.push_back(q);
     }
-    bool resident = false;
-    TRY(group_resident(gr, true, true, stream, &resident));
-    if (resident) {
+    // the graph holds both directions: it is taken where it is the faster for their sum
+    GroupRoute fwd, bwd;
+    TRY(group_route(gr, 0, stream, &fwd));
+    TRY(group_route(gr, 1, stream, &bwd));
+    if ((fwd.any || bwd.any) && fwd.graph_us + bwd.graph_us >= 0.9 * (fwd.us + bwd.us)) {
         for (swit_plan *pl : gr->plans) pl->strips_valid = false;
-        for (size_t i = 0; i < n; ++i) {
+        TRY(group_run(gr, fwd, stream, [&](int i, hipStream_t st) -> int {
             swit_plan *pl = gr->plans[i];
-            TRY(resident_forward(pl, src[i], seis[i], 1, stream));
-            TRY(launch_misfit(kind, pl->ns * pl->d.ngmax, pl->d.nt, pl->d.dt, obs[i], seis[i], adj[i], work[i],
-                              misfit[i], stream));
-            TRY(resident_adjoint(pl, src[i], adj[i], grad[i], illum_forw[i], illum_back[i], stream));
-            pl->strips_valid = true;
-        }
+            TRY(run_forward(pl, src[i], seis[i], 1, fwd.resident[i], st));
+            return launch_misfit(kind, pl->ns * pl->d.ngmax, pl->d.nt, pl->d.dt, obs[i], seis[i], adj[i], work[i],
+                                 misfit[i], st);
+        }));
+        TRY(group_run(gr, bwd, stream, [&](int i, hipStream_t st) {
+            return run_adjoint(gr->plans[i], src[i], adj[i], grad[i], illum_forw[i], illum_back[i], bwd.resident[i], st);
+        }));
+        for (swit_plan *pl : gr->plans) pl->strips_valid = true;
         return SWIT_OK;
     }
     for (size_t i = 0; i < n; ++i) {

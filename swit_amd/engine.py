@@ -243,10 +243,10 @@ class Plan:
 
 class PlanGroup:
     """Several batched plans (uneven grids, shot counts, record lengths) run as one job:
-    where every plan takes the resident time loops they run one after the other, each
-    filling the chip, otherwise each forward / adjoint is a single hipGraph launch with
-    every plan's step kernels on a branch of its own.  Results equal those of each plan
-    run alone."""
+    plans in their resident time loops side by side where they fit the chip together, one
+    after the other where each fills it, or each forward / adjoint as a single hipGraph
+    launch with every plan's step kernels on a branch of its own.  Results equal those of
+    each plan run alone."""
 
     def __init__(self, plans):
         self.plans = list(plans)
@@ -258,6 +258,11 @@ class PlanGroup:
         h = ctypes.c_void_p()
         _native.check(self._lib.swit_group_create(arr, len(self.plans), ctypes.byref(h)))
         self._h = h
+
+    def sets(self, which):
+        """The sets of plans that run one after the other in the 'forward' or 'backward'
+        direction, those of a set side by side; 0: all as one graph of step kernels."""
+        return int(self._lib.swit_group_sets(self._h, {"forward": 0, "backward": 1}[which]))
 
     @staticmethod
     def _ptrs(tensors):
