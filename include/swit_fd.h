@@ -155,7 +155,8 @@ const char *swit_last_error(void);
                                    with 1, but for an adjoint whose step kernels are
                                    estimated the faster (tall grids with few shots).
                                    An option of a direction's step kernels selects these
-                                   for it; the autotuner takes the faster.  Calls on a
+                                   for it; the autotuner takes the faster, but leaves a
+                                   plan that was set to 0 with its step kernels.  Calls on a
                                    capturing stream take the step kernels               */
 #define SWIT_OPT_RESIDENT_WAIT 2048  /* ms (default 30000) after which a workgroup of a
                                    resident loop stops waiting for a neighbour that runs

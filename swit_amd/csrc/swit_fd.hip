@@ -60,6 +60,7 @@ int cdiv(int a, int b) { return (a + b - 1) / b; }
 // resident_init_bwd has it.
 struct ResidentState {
     int use_fwd = 1, use_bwd = 1, use_exact = 1;
+    bool off = false;            // SWIT_OPT_RESIDENT 0, which the autotuner leaves as it is
     bool fwd = false;            // the forward's configuration exists
     rk::Cfg fc{};
     size_t f_lds = 0;
@@ -2083,7 +2084,7 @@ static int resident_autotune(swit_plan *pl, double *us, hipStream_t st) {
     ResidentState &rs = pl->res;
     BatchedState &bs = pl->bat;
     const Dims &d = pl->d;
-    if (!rs.fwd && !rs.bwd) return SWIT_OK;
+    if (rs.off || (!rs.fwd && !rs.bwd)) return SWIT_OK;
     hipEvent_t e0, e1;
     TRY(pool_event(bs, &e0));
     TRY(pool_event(bs, &e1));
@@ -2335,6 +2336,7 @@ extern "C" int swit_plan_set_option(swit_plan *pl, int option, int value) {
     case SWIT_OPT_RESIDENT:
         if (value != 0 && value != 1) return set_err(SWIT_EINVAL, "resident must be 0 or 1");
         pl->res.use_fwd = pl->res.use_bwd = pl->res.use_exact = value;
+        pl->res.off = !value;
         return SWIT_OK;
     case SWIT_OPT_RESIDENT_WAIT:
         if (value < 0 || value > rk::kMaxWaitMs)

@@ -52,3 +52,18 @@ def test_resident_forward_with_step_kernels_backward():
     for o in out[1:]:
         for a, b in zip(o, out[0]):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.gpu
+def test_autotuner_leaves_a_plan_without_resident_loops():
+    import torch
+    w = workloads.small(seed=3, nx=150, nz=60, npml=20, nt=60, ns=3)
+    p = _plan(w)
+    p.set_model(torch.from_numpy(w.vp_init), torch.from_numpy(workloads.gardner(w.vp_init)))
+    p.set_option("resident", 0)
+    tuned = p.autotune(5)
+    assert not p.resident("forward") and not p.resident("backward") and not p.resident("exact")
+    assert tuned["fwd_us"] > 0 and tuned["bwd_us"] > 0
+    p.set_option("resident", 1)
+    p.autotune(5)                            # times both; either way the results are the same
+    p.close()
