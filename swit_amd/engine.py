@@ -583,9 +583,16 @@ def process_gathers(optim, data, dt, offsets=None, params=None, first_break_ms=N
     tp = torch.as_tensor(taper, dtype=torch.float64, device=dev) if taper is not None else None
     nbytes = ctypes.c_size_t()
     _native.check(lib.swit_process_work(ctypes.byref(p), ctypes.byref(nbytes)))
+    least = nbytes.value
     if p.filter_taps:                        # room to filter up to 65536 traces in one launch
-        nbytes.value = max(nbytes.value, 8 * (nt + 6 * p.filter_taps) * min(ng * ntr, 65536))
-    work = torch.empty(int(nbytes.value), dtype=torch.uint8, device=dev)
+        nbytes.value = max(least, 8 * (nt + 6 * p.filter_taps) * min(ng * ntr, 65536))
+    try:
+        work = torch.empty(int(nbytes.value), dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:           # as many launches as the least room takes
+        if nbytes.value == least:
+            raise
+        nbytes.value = least
+        work = torch.empty(int(nbytes.value), dtype=torch.uint8, device=dev)
     stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
     def ptr(t):
