@@ -1777,6 +1777,21 @@ static int resident_init_bwd(swit_plan *pl, int ncu) {
 
 static int resident_init_fwd(swit_plan *pl);
 
+// part(): what one of the resident loops allocates.  Where that does not fit, *fits is false, the
+// part's memory is given back and the plan goes without that loop.
+template <class Part> static int resident_part(swit_plan *pl, bool *fits, Part part) {
+    const size_t count = pl->allocs.size();
+    const int64_t bytes = pl->bytes;
+    const int rc = part();
+    *fits = rc == SWIT_OK;
+    if (rc != SWIT_ENOMEM) return rc;
+    for (size_t k = count; k < pl->allocs.size(); ++k) (void)hipFree(pl->allocs[k]);
+    pl->allocs.resize(count);
+    pl->bytes = bytes;
+    g_err[0] = 0;
+    return SWIT_OK;
+}
+
 static int resident_init(swit_plan *pl) {
     ResidentState &rs = pl->res;
     const Dims &d = pl->d;
@@ -1784,13 +1799,24 @@ static int resident_init(swit_plan *pl) {
     HIP_TRY(hipGetDevice(&dev));
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     rs.ncu = ncu;
-    TRY(resident_init_bwd(pl, ncu));
+    bool fits = false;
+    TRY(resident_part(pl, &fits, [&] { return resident_init_bwd(pl, ncu); }));
     rs.fwd = choose_fwd(d, pl->ns, ncu, 8, &rs.fc, &rs.us[0]);
-    TRY(resident_init_ex(pl, ncu));
-    if (rs.fwd) TRY(resident_init_fwd(pl));
+    TRY(resident_part(pl, &fits, [&] { return resident_init_ex(pl, ncu); }));
+    if (rs.fwd) {
+        TRY(resident_part(pl, &fits, [&] { return resident_init_fwd(pl); }));
+        if (!fits) rs.fwd = rs.ex = false;           // the exact loop takes the forward's coefficients
+    }
     if (!rs.fwd && !rs.bwd) return SWIT_OK;
-    TRY(pl->alloc(&rs.msg, std::max(rs.f_msg, std::max(rs.b_msg, rs.x_msg))));
-    TRY(pl->alloc(&rs.ctl, 1));
+    TRY(resident_part(pl, &fits, [&] {
+        TRY(pl->alloc(&rs.msg, std::max(rs.fwd ? rs.f_msg : 0, std::max(rs.bwd ? rs.b_msg : 0, rs.ex ? rs.x_msg : 0))));
+        return pl->alloc(&rs.ctl, 1);
+    }));
+    if (!fits) {
+        rs.fwd = rs.bwd = rs.ex = false;
+        rs.ctl = nullptr;
+        return SWIT_OK;
+    }
     HIP_TRY(hipMemset(rs.ctl, 0, sizeof(rk::Ctl)));
     return SWIT_OK;
 }
