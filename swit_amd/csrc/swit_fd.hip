@@ -1281,13 +1281,15 @@ struct FwdKernel {
     void (*fn[2])(rk::FwdArgs);     // without / with the divergence history
 };
 // 4 R C registers of state and K per thread: R C <= 20 at four waves per SIMD (128 registers),
-// above at two (256 registers, workgroups of at most 8 waves)
+// above at two (256 registers, workgroups of at most 8 waves).  Of the sizes in between, those that
+// choose_fwd takes on some grid (54000 of widths to 3000, heights to 480, 1 to 400 shots, 32 to 256
+// compute units).
 #define SWIT_FWD(R, C) {R, C, {rk::k_fwd_resident<R, C, false>, rk::k_fwd_resident<R, C, true>}}
 const FwdKernel kFwdKernels[] = {
     SWIT_FWD(2, 3), SWIT_FWD(2, 6), SWIT_FWD(2, 9), SWIT_FWD(2, 14), SWIT_FWD(2, 20), SWIT_FWD(2, 24),
-    SWIT_FWD(3, 3), SWIT_FWD(3, 6), SWIT_FWD(3, 9), SWIT_FWD(3, 12), SWIT_FWD(3, 14), SWIT_FWD(3, 16),
-    SWIT_FWD(4, 3), SWIT_FWD(4, 5), SWIT_FWD(4, 8), SWIT_FWD(4, 10), SWIT_FWD(4, 12),
-    SWIT_FWD(5, 3), SWIT_FWD(5, 6), SWIT_FWD(5, 8),
+    SWIT_FWD(3, 3), SWIT_FWD(3, 6), SWIT_FWD(3, 14), SWIT_FWD(3, 16),
+    SWIT_FWD(4, 3), SWIT_FWD(4, 5), SWIT_FWD(4, 8), SWIT_FWD(4, 12),
+    SWIT_FWD(5, 3), SWIT_FWD(5, 8),
     SWIT_FWD(6, 3), SWIT_FWD(6, 6), SWIT_FWD(7, 3), SWIT_FWD(7, 5), SWIT_FWD(8, 3), SWIT_FWD(8, 4),
 };
 #undef SWIT_FWD
