@@ -87,9 +87,9 @@ def load_traffic(kernel):
 def autograd_leg(w, src, obs, vp_init, rho_init, args):
     """The same gradient through torch.autograd with the exact adjoint: one step is
     seismograms(vp) (forward with the divergence history), 1/2 |d - d_obs|^2 and
-    backward (exact adjoint of all shots), timed on one stream and then with the
-    shots' halves on two streams (the value; the gradients must be identical).  The
-    whole divergence history takes
+    backward (exact adjoint of all shots).  Step kernels are timed on one stream and then
+    with the shots' halves on two (the value; the gradients must be identical); a resident
+    loop takes all shots in one launch and is timed as it is.  The whole divergence history takes
     ns * nt * (nx+2npml) * ld * 4 bytes; when the device cannot hold it the plan keeps
     checkpoints and recomputes segments instead."""
     import torch
@@ -117,12 +117,12 @@ def autograd_leg(w, src, obs, vp_init, rho_init, args):
         torch.cuda.synchronize()
         return g, time.perf_counter() - t0
 
-    # one stream, then the shots' halves on two streams (bit-identical gradients)
-    g1, el1 = timed(1)
-    g, el = timed(2)
-    same = bool(torch.equal(g, g1))
-    fd = fd_self_check(w, pe, src, obs, vp_init, rho_init, g)
     resident = pe.resident("exact")      # wavefields in registers: their bytes do not move per step
+    g1, el1 = timed(1)
+    g, el = (g1, el1) if resident else timed(2)
+    one = {} if resident else {"one_stream_value": round(w.ns * args.steps / el1, 3),
+                               "identical_to_one_stream": bool(torch.equal(g, g1))}
+    fd = fd_self_check(w, pe, src, obs, vp_init, rho_init, g)
     pe.close()
     # algorithmic bytes of one autograd gradient: the exact forward (36 N_pad + the
     # divergence history 4 N_pad + 4 ng per shot and step) and the fused exact adjoint
@@ -134,8 +134,7 @@ def autograd_leg(w, src, obs, vp_init, rho_init, args):
     per_grad = w.ns * (w.nt - 1) * ((2 if mode == "checkpoint" else 1) * fwd_b + 48 * n_pad + 4 * w.ng)
     gbs = per_grad * args.steps / el / 1e9
     return {"value": round(w.ns * args.steps / el, 3), "unit": "shot-gradients/s",
-            "ms_per_step": round(1000 * el / args.steps, 2), "streams": 2,
-            "one_stream_value": round(w.ns * args.steps / el1, 3), "identical_to_one_stream": same,
+            "ms_per_step": round(1000 * el / args.steps, 2), "streams": 1 if resident else 2, **one,
             "history": "full" if mode is True else "checkpoints", "history_gib": round(need / 2**30, 1),
             "resident": resident, "algorithmic_bytes_per_gradient": None if resident else int(per_grad),
             "achieved_gbs": None if resident else round(gbs, 1),
@@ -171,15 +170,17 @@ def fd_self_check(w, plan, src, obs, vp, rho, g):
 
 def lanes_leg(w, src, obs, vp, rho, g_ref, args, lanes=2):
     """The same gradient on engine.Lanes: the shots split into `lanes` plans, each
-    running forward, adjoint source and adjoint on a stream of its own, so that the
-    lanes' step kernels run side by side.  Timed as the main steps (warm-up, then
+    running forward, adjoint source and adjoint on a stream of its own (the lanes' step
+    kernels, or their resident loops, run side by side).  Timed as the main steps (warm-up, then
     `steps` gradients between synchronisations); the gradient is checked against the
     main step's (FP64 sums in another order)."""
     import torch
     from swit_amd.engine import Lanes
     L = Lanes(w.nx, w.nz, w.dx, w.dt, w.nt, w.npml, w.src_xz, w.rec_xz, lanes=lanes, strips=args.strips)
     L.set_model(torch.from_numpy(w.vp_true).to(vp.device), torch.from_numpy(w.rho(w.vp_true)).to(vp.device))
-    tuned = L.autotune(steps=50) if not args.no_autotune else None
+    if not args.no_autotune:
+        L.autotune(steps=50)
+    resident = [p.resident("forward") and p.resident("backward") for p in L.plans]
     L.set_model(vp, rho)
     for _ in range(args.warmup):
         L.gradient(src, obs, "Waveform", w.dt)
@@ -193,14 +194,17 @@ def lanes_leg(w, src, obs, vp, rho, g_ref, args, lanes=2):
     L.close()
     return {"lanes": lanes, "value": round(w.ns * args.steps / el, 3), "unit": "shot-gradients/s",
             "ms_per_step": round(1000 * el / args.steps, 2), "grad_rel_vs_main": rel,
-            "autotuned": [t.get("bwd_steps") for t in tuned] if tuned else None}
+            "resident": resident}
 
 
 def two_streams_leg(w, plan, step, g_ref, args):
     """The main plan with SWIT_OPT_STREAMS 2 (each half of the shots runs its time loops
     on a stream of its own): timed as the main steps; the gradient and illuminations
-    must equal the one-stream step's bit for bit."""
+    must equal the one-stream step's bit for bit.  None where both loops are resident: the
+    option then changes nothing."""
     import torch
+    if plan.resident("forward") and plan.resident("backward"):
+        return None
     plan.set_option("streams", 2)
     for _ in range(args.warmup):
         step()
@@ -519,6 +523,14 @@ def main():
                         "time_loops_gbs": round((kern["forward"]["step_bytes"] * f_n + kern["backward"]["step_bytes"]
                                                  * b_n) / ((f_ms + b_ms) * 1e-3) / 1e9, 1)}
 
+    # the launch configurations of step kernels that do not run say nothing
+    route = {"resident": {k: args.path == "batched" and plan.resident(k) for k in ("forward", "backward")}}
+    if not route["resident"]["backward"]:
+        route["bwd_steps"] = plan.bwd_steps
+    if tuned:
+        drop = {"fwd": route["resident"]["forward"], "bwd": route["resident"]["backward"]}
+        tuned = {k: v for k, v in tuned.items() if k.endswith("_us") or not drop[k[:3]]}
+
     lanes = (lanes_leg(w, src, obs, vp_init, rho_init, g[0], args)
              if args.path == "batched" and not args.no_lanes else None)
     two_streams = (two_streams_leg(w, plan, step, g, args)
@@ -561,7 +573,7 @@ def main():
         "data": "synthetic (seeded 12-layer dipping model with two faults, Ricker 5 Hz)",
         "config": {"workload": f"{w.nx}x{w.nz} grid, npml {w.npml}, nt {w.nt}, dt {w.dt}, {w.ns} shots, "
                                f"{w.ng} receivers, L2 gradient", "path": args.path, "strips": args.strips,
-                   "shots_per_step": w.ns, "autotuned": tuned, "bwd_steps": plan.bwd_steps},
+                   "shots_per_step": w.ns, "autotuned": tuned, **route},
         "roofline": roofline,
         "cpu_baseline": cpu,
         "plain_baseline": plain,

@@ -13,7 +13,7 @@
 // The work is small (801x267: 1.7 MB a field, 35 M multiply-adds a smoothing with 40 samples
 // span), so launches and serial parts decide.  One workgroup per maximum, one thread per
 // kernel's weights and a launch per pass of each field took 513 us there in 27 launches; now 8
-// launches, 75 us: fields that go through the same pass share a launch (blockIdx.z), sums and
+// launches, 9 with a land mute, 75 us: fields that go through the same pass share a launch (blockIdx.z), sums and
 // products ride on the pass that makes their inputs, and every pass leaves the maximum of its
 // output in M by an atomic on an order-preserving integer form (a maximum has no order, so the
 // bits are those of any other way).

@@ -799,8 +799,8 @@ __host__ __device__ inline int bwd_step_floats(int W, int C, int R, int ninj, in
 // stores free of branches (a wait has to assume the fewest loads in flight that any path
 // leaves, and so waited for the stores of the column before).  One shot of 201x81: 7.5 us by
 // the step kernel, 6.4, 5.2, 5.1; 801x267, 81 shots: 432 by the step kernel, 224, 186, 180
-// (R = 6: eight waves fit since the edges of p and u share their place).  Vector issue is 5.9 of
-// the 9.2 us of a round of the 49 shots.
+// (R = 6: eight waves fit since the edges of p and u share their place).  Vector issue is 5.7 of
+// the 9.2 us of a round of the 49 shots (counted: 103 instructions a padded cell).
 template <int R, int C>
 __global__ __launch_bounds__(512) void k_bwd_resident(BwdArgs a) {
     extern __shared__ float lds[];

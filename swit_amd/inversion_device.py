@@ -64,8 +64,9 @@ class DeviceProblem:
         self.kind = optim.misfit_type
         if self.kind.lower() == 'rtm':
             raise ValueError("the device loop takes a misfit, not 'RTM'")
-        # two lanes (shot halves on streams of their own): their step kernels run side by
-        # side and fill each other's idle workgroup slots
+        # two lanes (shot halves on streams of their own): where their loops are step kernels,
+        # these run side by side and fill each other's idle workgroup slots; resident loops
+        # fill the chip by themselves, and one lane is the faster (engine.Lanes has both times)
         self.lanes = Lanes(inp["nx"], inp["nz"], inp["dx"], inp["dt"], inp["nt"], inp["npml"], inp["src_xz"],
                            inp["rec_xz"], lanes=lanes, free_surface=inp["free_surface"], path="batched",
                            strips=solver.STRIPS)

@@ -39,11 +39,13 @@ WRITE_PARFILES = False
 PATH = "batched"
 # Boundary-strip storage: 'f32' (reference precision), 'f16' or 'bf16'.
 STRIPS = "f32"
-# Time the batched step kernels' launch configurations once per synthetic-data plan,
-# at its first model, and keep the fastest (the results do not depend on the choice).
+# Time the batched step kernels' launch configurations and the resident loops once per
+# synthetic-data plan, at its first model, and keep the fastest (the results do not depend on
+# the choice).
 AUTOTUNE = True
-# Batched plans with two or more shots run the two halves of the shots on two streams,
-# so that each time step's two launches overlap (bit-identical results; 1 turns it off).
+# Batched plans with two or more shots run the two halves of the shots on two streams where
+# their loops are step kernels, so that each time step's two launches overlap (bit-identical
+# results; 1 turns it off).  A resident loop takes all shots in one launch.
 STREAMS = 2
 
 _JOBS = {}         # synthetic-data plan per homepath
